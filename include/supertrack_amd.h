@@ -236,6 +236,10 @@ typedef struct {
     int32_t use_graph;            /* capture the launch sequence once, replay */
     int32_t autotune;             /* pick launch parameters by timing          */
     int32_t block_threads;        /* 0 = default / autotuned                   */
+    /* The next four name a launch shape of the block kernel (a workgroup per
+     * segment), which then scores every fast track.  All 0: the one-wave
+     * kernel (a wavefront per segment or part of one), and the block kernel,
+     * at the shapes below, for tracks that the former does not take. */
     int32_t table_slots;          /* LDS hash slots per workgroup: 1280 or 1472
                                      (one point per thread), 1536, 2048 or
                                      4096; 0 (with blocks_per_cu and
@@ -266,9 +270,10 @@ int st_batch_sync(st_batch *b);
 /* Device time of the last st_batch_run in ms: ms2[0] the fused kernel
  * (with its reset), ms2[1] the exact per-segment path. */
 int st_batch_times(st_batch *b, float *ms2);
-/* Launch parameters in use (5 entries): block_threads, table_slots,
- * blocks_per_cu, points_per_thread, hist_copies (0: the histograms count
- * straight into the device counters, too large for LDS). */
+/* Launch parameters in use (5 entries): block_threads, table_slots (per
+ * workgroup; one-wave kernel: per wave), blocks_per_cu, points_per_thread,
+ * hist_copies (0: the histograms count straight into the device counters, too
+ * large for LDS). */
 int st_batch_params(const st_batch *b, int32_t *params5);
 /* Counts of the last st_batch_run's fused kernel: stats3[0] points scored
  * (points of the in-voxel block ranges of the segments that pass the x/y
@@ -300,7 +305,7 @@ void st_batch_destroy(st_batch *b);
  * loops, harnesses that forbid hipMalloc).  The same pass as st_batch_create +
  * st_batch_run over a finished library, adding counts to each histogram's
  * device counters, but it allocates nothing: its control block (segment
- * ticket, error flag, run statistics) is a 256-byte device array of the
+ * tickets, error flag, run statistics) is a 2 KiB device array of the
  * library, one per device, held until the process ends.  Launch shape as
  * st_batch_create without autotune (opts->autotune must be 0; use_graph is
  * ignored).  Limit: the library may hold no track routed to the exact

@@ -38,9 +38,23 @@
 #include "layout.hpp"
 
 #include "batch_kernel.hpp"
+#include "wave_kernel.hpp"
 
 namespace st {
 namespace {
+
+// Points read past the end of the point arrays by the one-wave kernel's
+// prefetch (at most two rows of 64 beyond a row), never used.
+constexpr int64_t kPointPad = 256;
+
+// The one-wave kernel, compiled for six (ST_F32) and four (ST_F64) waves per
+// SIMD: what its tables leave room for, and no register is spilled (seven
+// waves with 352-slot tables: 13.7 ms against 13.1 ms on 2 nm spheres).
+const void *wave_kernel_ptr(int mode)
+{
+    return mode == ST_F64 ? (const void *)wave_kernel<ST_F64, kWaveSlots, 4>
+                          : (const void *)wave_kernel<ST_F32, kWaveSlots, 6>;
+}
 
 template <int MODE, int SLOTS, int PPT>
 const void *kernel_ptr()
@@ -97,21 +111,16 @@ int dev_put(T *dst, const T *src, size_t n)
     return ST_OK;
 }
 
-template <typename T>
-int dev_upload(T **dst, const T *src, size_t n, int64_t *bytes)
-{
-    *dst = nullptr;
-    if (n == 0) return ST_OK;
-    hipError_t e = dev_malloc((void **)dst, n * sizeof(T));
-    if (e != hipSuccess) {
-        *dst = nullptr;
-        return set_error(ST_ENOMEM, "st_library_create: hipMalloc(%zu B) failed: %s", n * sizeof(T),
-                         hipGetErrorString(e));
+// Sub-buffers of one device allocation, each at a 256-byte boundary.
+struct Carve {
+    size_t bytes = 0;
+    size_t add(size_t n)
+    {
+        const size_t at = bytes;
+        bytes += (n + 255) / 256 * 256;
+        return at;
     }
-    *bytes += (int64_t)(n * sizeof(T));
-    ST_HIP_TRY(hipMemcpy(*dst, src, n * sizeof(T), hipMemcpyHostToDevice));
-    return ST_OK;
-}
+};
 
 
 // Launch shape of the fused kernel.
@@ -119,6 +128,14 @@ struct Launch {
     int slots = 1536, blocks_per_cu = 1, ppt = 1, grid = 0;
     bool lds_hist = true;     // histograms privatised in LDS (else device atomics)
     int hist_copies = 1;      // LDS copies of the privatised histograms
+    size_t lds = 0;
+};
+
+// Launch shape of the one-wave kernel.
+struct WaveLaunch {
+    bool on = false;
+    int wg_waves = 16, blocks_per_cu = 1, grid = 0;
+    bool lds_hist = true;
     size_t lds = 0;
 };
 
@@ -139,9 +156,19 @@ struct st_library {
     float4 *p32 = nullptr;
     double *zfirst = nullptr;
     BlockF32 *blocks = nullptr;
+    // one allocation (finish): the track table, geometries, orders and the
+    // allocation-free pass's plan
+    char *tables = nullptr;
     TrackDesc *tracks_dev = nullptr;
     GeomDev *geoms_dev = nullptr;
     int32_t *order_dev = nullptr;      // fast_order on the device
+    // fast_order split by kernel: tracks of the one-wave kernel (kFlagWave)
+    // and the rest
+    std::vector<int32_t> wave_order, rest_order;
+    int32_t *wave_order_dev = nullptr, *rest_order_dev = nullptr;
+    int64_t wave_points = 0;           // points of the wave_order tracks
+    // work queues of the allocation-free pass (a batch keeps its own)
+    PlanTrack *static_plan = nullptr;
     // streamed construction: begin sizes the device arrays, appends fill them
     // in track order, finish publishes the track table
     int64_t tracks_done = 0, points_done = 0, blocks_cap = 0;
@@ -153,9 +180,13 @@ struct st_batch {
     st_batch_opts opts{};
     std::vector<st_hist *> hists;
     hipStream_t stream = nullptr;
-    Launch ln;
+    Launch ln;                 // batch_kernel: all fast tracks, or (wave.on) those wave_kernel does not take
+    WaveLaunch wave;           // wave_kernel
+    PlanTrack *wave_plan = nullptr;              // its work queues
+    unsigned int *slab = nullptr;                // its workgroups' histograms
+    unsigned long long *slab_stats = nullptr;    // and statistics
     int hist_words = 0;
-    BatchCtl *ctl = nullptr;   // per-pass control block (device)
+    BatchCtl *ctl = nullptr;   // per-pass control block (device); the plan and slabs follow it
     RecArgs rec{};                // recording buffers (cap 0: off)
     RecArgs *rec_dev = nullptr;   // their descriptor in device memory
     bool graph_ready = false;
@@ -171,8 +202,9 @@ struct st_batch {
 
 namespace {
 
+// rest: only the tracks that the one-wave kernel does not take.
 BatchArgs make_args(const st_library *L, const st_batch_opts &o, st_hist *const *hists, int n_hists,
-                    const Launch &ln, BatchCtl *ctl)
+                    const Launch &ln, BatchCtl *ctl, bool rest)
 {
     BatchArgs a{};
     a.tracks = L->tracks_dev;
@@ -184,8 +216,8 @@ BatchArgs make_args(const st_library *L, const st_batch_opts &o, st_hist *const 
     a.zfirst = L->zfirst;
     a.blocks = L->blocks;
     a.geoms = L->geoms_dev;
-    a.order = L->order_dev;
-    a.n_seg = (int64_t)L->fast_order.size() * o.n_oversamples;
+    a.order = rest ? L->rest_order_dev : L->order_dev;
+    a.n_seg = (int64_t)(rest ? L->rest_order : L->fast_order).size() * o.n_oversamples;
     a.n_os = std::max(o.n_oversamples, 1);
     a.shift_xy = o.shift_xy;
     a.shift_z = o.shift_z;
@@ -207,11 +239,73 @@ BatchArgs make_args(const st_library *L, const st_batch_opts &o, st_hist *const 
     return a;
 }
 
-// Queues one pass: the control-block reset, then the fused kernel.
-int launch_pass(int precision, const BatchArgs &args, const Launch &ln, hipStream_t stream)
+// Entries of one queue of the plan, and bytes of the whole plan (the queues,
+// then their chunk counts).
+int64_t plan_stride(const st_library *L) { return ((int64_t)L->wave_order.size() + kQueues - 1) / kQueues; }
+size_t plan_bytes(const st_library *L)
+{
+    return (size_t)(kQueues * plan_stride(L)) * sizeof(PlanTrack) + kQueues * sizeof(int64_t);
+}
+int64_t *plan_totals(const st_library *L, PlanTrack *plan)
+{
+    return reinterpret_cast<int64_t *>(plan + kQueues * plan_stride(L));
+}
+
+// The one-wave kernel's arguments; plan: its work queues.
+WaveArgs make_wave_args(const st_library *L, const st_batch_opts &o, st_hist *const *hists, int n_hists,
+                        const WaveLaunch &w, BatchCtl *ctl, PlanTrack *plan, unsigned int *slab,
+                        unsigned long long *slab_stats)
+{
+    Launch ln;
+    ln.lds_hist = w.lds_hist;
+    WaveArgs wa{};
+    wa.b = make_args(L, o, hists, n_hists, ln, ctl, false);
+    wa.plan.tracks = plan;
+    wa.plan.total = plan_totals(L, plan);
+    wa.plan.stride = plan_stride(L);
+    wa.plan.n_tracks = (int32_t)L->wave_order.size();
+    wa.plan.tickets = ctl->tickets;
+    wa.slab = slab;
+    wa.slab_stats = slab_stats;
+    return wa;
+}
+
+// Queues the kernel that fills a plan: chunks of a tenth of a wave's share of
+// the work left, but at least an even share of all of it between 2048 and
+// 12288 points (a chunk's set-up, about five rows of 64 points, then stays
+// small beside the tenth of its points that is scored).  1/8 to 1/12 and 12288
+// to 24576 points measured within 3 % of each other, 1/24 and 6144 points 9 %
+// slower.
+int launch_plan(const st_library *L, int n_os, const WaveLaunch &w, PlanTrack *plan, hipStream_t stream)
+{
+    const double waves = (double)w.grid * w.wg_waves;
+    const double even = (double)L->wave_points * n_os / waves;
+    const int min_points = (int)std::min(std::max(even, 2048.0), 12288.0);
+    wave_plan_kernel<<<1, 64 * kQueues, 0, stream>>>(L->tracks_dev, L->wave_order_dev, (int32_t)L->wave_order.size(),
+                                                     n_os, L->wave_points, n_os / (waves * 10.0), min_points,
+                                                     plan_stride(L), plan, plan_totals(L, plan));
+    ST_HIP_TRY(hipGetLastError());
+    return ST_OK;
+}
+
+// Queues one pass: the control-block reset, then (wave non-null) the one-wave
+// kernel and the sum of its workgroups' histograms, and the block kernel over
+// the tracks of args.
+int launch_pass(int precision, const BatchArgs &args, const Launch &ln, const WaveArgs *wave, const WaveLaunch &w,
+                hipStream_t stream)
 {
     batch_reset_kernel<<<1, 64, 0, stream>>>(args.ctl);
     ST_HIP_TRY(hipGetLastError());
+    if (wave && wave->plan.n_tracks > 0) {
+        WaveArgs a = *wave;
+        void *kargs[] = {&a};
+        ST_HIP_TRY(hipLaunchKernel(wave_kernel_ptr(precision), dim3(w.grid), dim3(64 * w.wg_waves), kargs, w.lds,
+                                   stream));
+        if (a.slab) {
+            slab_sum_kernel<<<(a.b.hist_lds_words + 63) / 64 + 1, 1024, 0, stream>>>(a, w.grid);
+            ST_HIP_TRY(hipGetLastError());
+        }
+    }
     if (args.n_seg == 0) return ST_OK;
     const void *k = pick_kernel(precision, ln.slots, ln.ppt);
     BatchArgs a = args;
@@ -222,9 +316,58 @@ int launch_pass(int precision, const BatchArgs &args, const Launch &ln, hipStrea
 
 int launch_fast(st_batch *b)
 {
-    BatchArgs a = make_args(b->lib, b->opts, b->hists.data(), (int)b->hists.size(), b->ln, b->ctl);
+    const st_library *L = b->lib;
+    BatchArgs a = make_args(L, b->opts, b->hists.data(), (int)b->hists.size(), b->ln, b->ctl, b->wave.on);
     a.rec = b->rec.cap > 0 ? b->rec_dev : nullptr;
-    return launch_pass(b->lib->precision, a, b->ln, b->stream);
+    if (!b->wave.on) return launch_pass(L->precision, a, b->ln, nullptr, b->wave, b->stream);
+    WaveArgs wa = make_wave_args(L, b->opts, b->hists.data(), (int)b->hists.size(), b->wave, b->ctl, b->wave_plan,
+                                 b->slab, b->slab_stats);
+    wa.b.rec = a.rec;
+    return launch_pass(L->precision, a, b->ln, &wa, b->wave, b->stream);
+}
+
+// Launch shape of the one-wave kernel: the workgroup size (4 to 16 waves share
+// one privatised histogram) that keeps most waves resident on a CU; on a tie
+// the largest (fewest histograms to sum).  Histograms that do not fit beside
+// four waves' tables are counted in the device bins.
+int configure_wave(int precision, int hist_words, WaveLaunch *out)
+{
+    const void *k = wave_kernel_ptr(precision);
+    const size_t per_wave = wave_lds(precision == ST_F64 ? 2 : 1, kWaveSlots);
+    hipFuncAttributes attr;
+    ST_HIP_TRY(hipFuncGetAttributes(&attr, k));
+    const int simd_waves = precision == ST_F64 ? 4 : 6;
+    const size_t kCuLds = 160 * 1024;
+    WaveLaunch best;
+    for (int pass = 0; pass < 2 && !best.on; ++pass) {
+        for (int wg = 4; wg <= 16; ++wg) {
+            WaveLaunch w;
+            w.lds_hist = pass == 0;
+            w.wg_waves = wg;
+            w.lds = wg * per_wave + (w.lds_hist ? (size_t)hist_words * 4 : 0);
+            // (allocated in steps: leave each workgroup a kilobyte)
+            const size_t all = w.lds + attr.sharedSizeBytes + 1024;
+            w.blocks_per_cu = std::min<int>((int)(kCuLds / all), 4 * simd_waves / wg);
+            if (w.blocks_per_cu < 1) continue;
+            w.on = true;
+            if (!best.on || w.blocks_per_cu * wg >= best.blocks_per_cu * best.wg_waves) best = w;
+        }
+    }
+    if (!best.on) return set_error(ST_EHIP, "one-wave kernel cannot be resident");
+    ST_HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)best.lds));
+    int fit = 0;
+    ST_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, k, 64 * best.wg_waves, best.lds));
+    if (fit < 1) return set_error(ST_EHIP, "one-wave kernel cannot be resident with %zu B LDS", best.lds);
+    best.blocks_per_cu = std::min(best.blocks_per_cu, fit);
+    best.grid = best.blocks_per_cu * device_cu_count();
+    *out = best;
+    return ST_OK;
+}
+
+// A launch shape named by the caller is the block kernel's.
+bool names_block_shape(const st_batch_opts &o)
+{
+    return o.table_slots || o.blocks_per_cu || o.points_per_thread || o.hist_copies;
 }
 
 // Launch shape for (table slots, workgroups per CU, points per thread, LDS
@@ -395,6 +538,22 @@ int autotune(st_batch *b)
     const int cand_bpc[] = {2, 3, 4, 5, 6, 7, 8};
     const int cand_copies[] = {1, 2, 4};
     float best = 1e30f;
+    const WaveLaunch wave = b->wave;
+    if (wave.on) {
+        for (int k = 0; k < 2; ++k) {
+            ST_HIP_TRY(hipEventRecord(ev.e[0], b->stream));
+            int rc = launch_fast(b);
+            if (rc) return rc;
+            ST_HIP_TRY(hipEventRecord(ev.e[1], b->stream));
+            ST_HIP_TRY(hipEventSynchronize(ev.e[1]));
+            float ms = 0;
+            ST_HIP_TRY(hipEventElapsedTime(&ms, ev.e[0], ev.e[1]));
+            best = std::min(best, ms);
+        }
+    }
+    const Launch rest_ln = b->ln;
+    bool block = !wave.on;
+    b->wave.on = false;   // the block kernel's candidates take every fast track
     int best_s = b->ln.slots, best_b = b->ln.blocks_per_cu, best_p = b->ln.ppt, best_c = b->ln.hist_copies;
     for (int s : cand_slots)
         for (int pp = 1; pp <= 2; ++pp)
@@ -411,6 +570,7 @@ int autotune(st_batch *b)
                 ST_HIP_TRY(hipEventElapsedTime(&ms, ev.e[0], ev.e[1]));
                 if (ms < best) {
                     best = ms;
+                    block = true;
                     best_s = s;
                     best_b = bp;
                     best_p = pp;
@@ -422,6 +582,11 @@ int autotune(st_batch *b)
                                   hipMemcpyHostToDevice, b->stream));
     ST_HIP_TRY(hipStreamSynchronize(b->stream));
     clear_error();   // candidates that did not fit set an error string
+    if (!block) {
+        b->ln = rest_ln;
+        b->wave = wave;
+        return ST_OK;
+    }
     return configure(b, best_s, best_b, best_p, best_c);
 }
 
@@ -433,7 +598,7 @@ int autotune(st_batch *b)
 // a device address: each device's address comes from hipGetSymbolAddress,
 // taken once per device with that device current, and only that address is
 // handed to kernels and copies.
-constexpr size_t kStaticScratchBytes = 256;
+constexpr size_t kStaticScratchBytes = 2048;
 static_assert(sizeof(BatchCtl) <= kStaticScratchBytes, "the control block fits the static scratch");
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 constexpr int kMaxDevices = 64;
@@ -510,13 +675,14 @@ int st_library_begin(int64_t n_tracks, int64_t n_points, const st_geometry *geom
     L->blocks_cap = n_points / kBlk + n_tracks + 1;
     int rc = ST_OK;
     int64_t bytes = 0;
-    if (!rc) rc = dev_alloc(&L->x64, n_points, &bytes);
-    if (!rc) rc = dev_alloc(&L->y64, n_points, &bytes);
-    if (!rc) rc = dev_alloc(&L->z64, n_points, &bytes);
-    if (!rc) rc = dev_alloc(&L->e64, n_points, &bytes);
+    const int64_t padded = n_points > 0 ? n_points + kPointPad : 0;
+    if (!rc) rc = dev_alloc(&L->x64, padded, &bytes);
+    if (!rc) rc = dev_alloc(&L->y64, padded, &bytes);
+    if (!rc) rc = dev_alloc(&L->z64, padded, &bytes);
+    if (!rc) rc = dev_alloc(&L->e64, padded, &bytes);
     if (!rc) rc = dev_alloc(&L->zfirst, L->blocks_cap, &bytes);
     if (!rc && precision == ST_F32) {
-        rc = dev_alloc(&L->p32, n_points, &bytes);
+        rc = dev_alloc(&L->p32, padded, &bytes);
         if (!rc) rc = dev_alloc(&L->blocks, L->blocks_cap, &bytes);
     }
     L->device_bytes = bytes;
@@ -600,6 +766,18 @@ int st_library_finish(st_library *L)
     std::stable_sort(L->fast_order.begin(), L->fast_order.end(),
                      [&](int32_t a2, int32_t b2) { return L->tracks[a2].n > L->tracks[b2].n; });
 
+    L->wave_order.clear();
+    L->rest_order.clear();
+    L->wave_points = 0;
+    for (int32_t t : L->fast_order) {
+        if (L->tracks[t].wave & kFlagWave) {
+            L->wave_order.push_back(t);
+            L->wave_points += L->tracks[t].n;
+        } else {
+            L->rest_order.push_back(t);
+        }
+    }
+
     const int n_geoms = (int)L->geoms.size();
     std::vector<GeomDev> gd(n_geoms);
     for (int i = 0; i < n_geoms; ++i) {
@@ -620,17 +798,39 @@ int st_library_finish(st_library *L)
             const double dlq = dl / g.diameter;
             gd[i].fm = 0.5 - (dlq + 1e-12);
             gd[i].mrgq = 3.0 * dlq * (1.0 + 2.0 * dlq) + 1e-14 * gd[i].r2q;
+            sphere_thresholds(gd[i].r2q, gd[i].fm, gd[i].mrgq, &gd[i].sure, &gd[i].maybe);
         }
         gd[i].N = (unsigned long long)g.n_linear;
         gd[i].N2 = gd[i].N * gd[i].N;
     }
-    int rc = ST_OK;
-    int64_t bytes = 0;
-    if (!rc) rc = dev_upload(&L->tracks_dev, L->tracks.data(), L->tracks.size(), &bytes);
-    if (!rc) rc = dev_upload(&L->geoms_dev, gd.data(), gd.size(), &bytes);
-    if (!rc) rc = dev_upload(&L->order_dev, L->fast_order.data(), L->fast_order.size(), &bytes);
-    L->device_bytes += bytes;
-    if (rc) return rc;
+    Carve c;
+    const size_t at_tracks = c.add(L->tracks.size() * sizeof(TrackDesc)), at_geoms = c.add(gd.size() * sizeof(GeomDev));
+    const size_t at_order = c.add(L->fast_order.size() * sizeof(int32_t));
+    const size_t at_wave = c.add(L->wave_order.size() * sizeof(int32_t));
+    const size_t at_rest = c.add(L->rest_order.size() * sizeof(int32_t));
+    const size_t host_bytes = c.bytes, at_plan = c.add(plan_bytes(L));
+    std::vector<char> image(host_bytes);
+    auto put = [&](size_t at, const void *src, size_t bytes) {
+        if (bytes) std::memcpy(image.data() + at, src, bytes);
+    };
+    put(at_tracks, L->tracks.data(), L->tracks.size() * sizeof(TrackDesc));
+    put(at_geoms, gd.data(), gd.size() * sizeof(GeomDev));
+    put(at_order, L->fast_order.data(), L->fast_order.size() * sizeof(int32_t));
+    put(at_wave, L->wave_order.data(), L->wave_order.size() * sizeof(int32_t));
+    put(at_rest, L->rest_order.data(), L->rest_order.size() * sizeof(int32_t));
+    if (!L->tables) {   // (kept for a retry after a failed copy)
+        int64_t bytes = 0;
+        int rc = dev_alloc(&L->tables, c.bytes, &bytes);
+        if (rc) return rc;
+        L->device_bytes += bytes;
+    }
+    ST_HIP_TRY(hipMemcpy(L->tables, image.data(), host_bytes, hipMemcpyHostToDevice));
+    L->tracks_dev = reinterpret_cast<TrackDesc *>(L->tables + at_tracks);
+    L->geoms_dev = reinterpret_cast<GeomDev *>(L->tables + at_geoms);
+    L->order_dev = reinterpret_cast<int32_t *>(L->tables + at_order);
+    L->wave_order_dev = reinterpret_cast<int32_t *>(L->tables + at_wave);
+    L->rest_order_dev = reinterpret_cast<int32_t *>(L->tables + at_rest);
+    L->static_plan = reinterpret_cast<PlanTrack *>(L->tables + at_plan);
     L->finished = true;
     return ST_OK;
 }
@@ -684,7 +884,7 @@ void st_library_destroy(st_library *L)
     if (!L) return;
     (void)hipDeviceSynchronize();
     void *ptrs[] = {L->x64, L->y64, L->z64, L->e64, L->p32,
-                    L->zfirst, L->blocks, L->tracks_dev, L->geoms_dev, L->order_dev};
+                    L->zfirst, L->blocks, L->tables};
     for (void *p : ptrs) (void)hipFree(p);
     delete L;
 }
@@ -713,9 +913,33 @@ int st_batch_create(st_library *lib, const st_batch_opts *opts, st_hist *const *
         st_batch_destroy(b);
         return code;
     };
-    hipError_t e = dev_malloc((void **)&b->ctl, sizeof(BatchCtl));
-    if (e == hipSuccess) e = hipMemset(b->ctl, 0, sizeof(BatchCtl));
+    rc = default_launch(lib->precision, b->hist_words, *opts, &b->ln);
+    if (rc) return fail(rc);
+    const bool wave = !names_block_shape(*opts) && !lib->wave_order.empty() && opts->n_oversamples > 0;
+    if (wave) {
+        rc = configure_wave(lib->precision, b->hist_words, &b->wave);
+        if (rc) return fail(rc);
+    }
+    Carve c;
+    c.add(sizeof(BatchCtl));
+    const size_t at_plan = c.add(wave ? plan_bytes(lib) : 0);
+    const size_t at_stats = c.add((size_t)b->wave.grid * kStats * sizeof(unsigned long long));
+    const size_t at_slab = c.add((size_t)b->wave.grid * (b->wave.lds_hist ? b->hist_words : 0) * sizeof(unsigned int));
+    char *work = nullptr;
+    hipError_t e = dev_malloc((void **)&work, c.bytes);
+    b->ctl = reinterpret_cast<BatchCtl *>(work);
+    if (e == hipSuccess) {
+        batch_reset_kernel<<<1, 64, 0, b->stream>>>(b->ctl);
+        e = hipGetLastError();
+    }
     if (e != hipSuccess) return fail(set_error(hip_status(e), "st_batch_create: %s", hipGetErrorString(e)));
+    if (wave) {
+        b->wave_plan = reinterpret_cast<PlanTrack *>(work + at_plan);
+        b->slab_stats = reinterpret_cast<unsigned long long *>(work + at_stats);
+        b->slab = reinterpret_cast<unsigned int *>(work + at_slab);
+        rc = launch_plan(lib, opts->n_oversamples, b->wave, b->wave_plan, b->stream);
+        if (rc) return fail(rc);
+    }
     for (const st_geometry &g : lib->geoms) {
         st_vcs *m = nullptr;
         rc = st_vcs_create(&g, opts->shift_xy, opts->shift_z, 0, 0, &m);
@@ -723,8 +947,6 @@ int st_batch_create(st_library *lib, const st_batch_opts *opts, st_hist *const *
         st_vcs_set_stream(m, b->stream);
         b->methods.push_back(m);
     }
-    rc = default_launch(lib->precision, b->hist_words, *opts, &b->ln);
-    if (rc) return fail(rc);
     if (opts->autotune && !lib->fast_order.empty() && opts->n_oversamples > 0) {
         rc = autotune(b);
         if (rc) return fail(rc);
@@ -764,8 +986,20 @@ int st_batch_run_static(st_library *lib, const st_batch_opts *opts, st_hist *con
     if (rc) return rc;
     hipStream_t stream = hip_stream ? (hipStream_t)hip_stream : default_stream();
     if (!stream) return set_error(ST_EHIP, "st_batch_run_static: no stream");
-    const BatchArgs a = make_args(lib, *opts, hists, n_hists, ln, ctl);
-    rc = launch_pass(lib->precision, a, ln, stream);
+    // the histograms of the one-wave kernel's workgroups are merged with
+    // atomics here: their slab would have to be allocated
+    WaveLaunch w;
+    const bool wave = !names_block_shape(*opts) && !lib->wave_order.empty();
+    if (wave) {
+        rc = configure_wave(lib->precision, hist_words, &w);
+        if (!rc) rc = launch_plan(lib, opts->n_oversamples, w, lib->static_plan, stream);
+        if (rc) return rc;
+    }
+    const BatchArgs a = make_args(lib, *opts, hists, n_hists, ln, ctl, wave);
+    WaveArgs wa{};
+    if (wave)
+        wa = make_wave_args(lib, *opts, hists, n_hists, w, ctl, lib->static_plan, nullptr, nullptr);
+    rc = launch_pass(lib->precision, a, ln, wave ? &wa : nullptr, w, stream);
     if (rc || !stats7) return rc;
     BatchCtl c;
     rc = read_ctl(ctl, stream, &c);
@@ -864,6 +1098,14 @@ int st_batch_balance(st_batch *b, uint64_t *balance4)
 int st_batch_params(const st_batch *b, int32_t *p)
 {
     if (!b || !p) return set_error(ST_EINVAL, "st_batch_params: null argument");
+    if (b->wave.on) {
+        p[0] = 64 * b->wave.wg_waves;
+        p[1] = kWaveSlots;
+        p[2] = b->wave.blocks_per_cu;
+        p[3] = 1;
+        p[4] = b->wave.lds_hist ? 1 : 0;
+        return ST_OK;
+    }
     p[0] = kBT;
     p[1] = b->ln.slots;
     p[2] = b->ln.blocks_per_cu;
@@ -908,8 +1150,13 @@ int st_batch_record_fetch(st_batch *b, int64_t *segments, uint64_t *keys, double
     const int64_t n_os = std::max(b->opts.n_oversamples, 1);
     std::vector<int64_t> seg(c);
     if (c) ST_HIP_TRY(hipMemcpy(seg.data(), b->rec.seg, c * sizeof(int64_t), hipMemcpyDeviceToHost));
-    for (unsigned long long i = 0; i < c; ++i)
-        seg[i] = (int64_t)b->lib->fast_order[seg[i] / n_os] * n_os + seg[i] % n_os;
+    const std::vector<int32_t> &order = b->wave.on ? b->lib->rest_order : b->lib->fast_order;
+    std::vector<char> by_wave(c);   // the one-wave kernel records segment ids and the reference's keys (bit 62)
+    for (unsigned long long i = 0; i < c; ++i) {
+        by_wave[i] = (seg[i] >> 62) & 1;
+        if (by_wave[i]) seg[i] &= ~(int64_t(1) << 62);
+        else seg[i] = (int64_t)order[seg[i] / n_os] * n_os + seg[i] % n_os;
+    }
     if (c && segments) std::memcpy(segments, seg.data(), c * sizeof(int64_t));
     if (c && keys) {
         // the reference's key from the local key and its slab's box
@@ -917,6 +1164,10 @@ int st_batch_record_fetch(st_batch *b, int64_t *segments, uint64_t *keys, double
         ST_HIP_TRY(hipMemcpy(loc.data(), b->rec.key, c * sizeof(uint64_t), hipMemcpyDeviceToHost));
         ST_HIP_TRY(hipMemcpy(bx.data(), b->rec.box, 3 * c * sizeof(uint64_t), hipMemcpyDeviceToHost));
         for (unsigned long long i = 0; i < c; ++i) {
+            if (by_wave[i]) {
+                keys[i] = loc[i];
+                continue;
+            }
             const TrackDesc &td = b->lib->tracks[seg[i] / n_os];
             const unsigned long long N = (unsigned long long)b->lib->geoms[td.geom].n_linear;
             const unsigned long long kx0 = bx[3 * i] & 0xFFFFFFFFull, ky0 = bx[3 * i] >> 32;

@@ -47,6 +47,7 @@ struct GeomDev {
     // ST_F64 thresholds in lattice units (as BlockF32's, with the FP64
     // rounding bound dl of the geometry: the data carry no FP32 rounding)
     double fm, mrgq;
+    double sure, maybe;   // squared-distance thresholds (sphere_thresholds)
     unsigned long long N, N2;
 };
 
@@ -67,6 +68,8 @@ struct HistDev {
 //   hi word plus the lo word times an odd constant); a pass that loses no
 //   entry has [3] == [4] and [5] == [6].
 constexpr int kStats = 7;
+constexpr int kQueues = 8;
+constexpr int kTicketPad = 16;
 struct BatchCtl {
     unsigned long long ticket;
     unsigned long long rec_count;
@@ -75,6 +78,8 @@ struct BatchCtl {
     int error;
     int pad;
     unsigned long long stats[kStats];
+    // the one-wave kernel's work queues, one ticket counter per 128-byte line
+    unsigned long long tickets[kQueues * kTicketPad];
 };
 constexpr unsigned long long kBalanceMul = 0x9E3779B97F4A7C15ull;
 
@@ -1038,6 +1043,7 @@ __global__ void batch_reset_kernel(BatchCtl *ctl)
         ctl->pad = 0;
     }
     if (threadIdx.x < kStats) ctl->stats[threadIdx.x] = 0;
+    if (threadIdx.x < kQueues) ctl->tickets[threadIdx.x * kTicketPad] = 0;
 }
 
 }  // namespace

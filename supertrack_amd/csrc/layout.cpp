@@ -3,8 +3,8 @@
 
 #include <algorithm>
 #include <cmath>
-#include <deque>
-#include <numeric>
+#include <utility>
+#include <vector>
 
 #include "parallel.hpp"
 
@@ -14,32 +14,71 @@ int64_t window_bound(const double *x, const double *y, const double *z, int64_t 
                      int64_t layers)
 {
     if (n == 0) return 0;
-    std::deque<int64_t> xmax, xmin, ymax, ymin;
+    // monotonic queues of the window's x and y extremes, each in a buffer of
+    // its own (an index enters each queue once)
+    struct Extreme {
+        std::vector<int64_t> at;
+        int64_t head = 0, tail = 0;
+    } q[4];
+    for (Extreme &e : q) e.at.resize(n);
     int64_t best = 0;
     int64_t j = 0;
     for (int64_t i = 0; i < n; ++i) {
-        while (j < n && z[j] - z[i] <= w) {
-            while (!xmax.empty() && x[xmax.back()] <= x[j]) xmax.pop_back();
-            xmax.push_back(j);
-            while (!xmin.empty() && x[xmin.back()] >= x[j]) xmin.pop_back();
-            xmin.push_back(j);
-            while (!ymax.empty() && y[ymax.back()] <= y[j]) ymax.pop_back();
-            ymax.push_back(j);
-            while (!ymin.empty() && y[ymin.back()] >= y[j]) ymin.pop_back();
-            ymin.push_back(j);
-            ++j;
+        for (; j < n && z[j] - z[i] <= w; ++j) {
+            while (q[0].tail > q[0].head && x[q[0].at[q[0].tail - 1]] <= x[j]) --q[0].tail;
+            while (q[1].tail > q[1].head && x[q[1].at[q[1].tail - 1]] >= x[j]) --q[1].tail;
+            while (q[2].tail > q[2].head && y[q[2].at[q[2].tail - 1]] <= y[j]) --q[2].tail;
+            while (q[3].tail > q[3].head && y[q[3].at[q[3].tail - 1]] >= y[j]) --q[3].tail;
+            for (Extreme &e : q) e.at[e.tail++] = j;
         }
         const int64_t cnt = j - i;
-        const double cx = std::floor((x[xmax.front()] - x[xmin.front()]) / D) + 2.0;
-        const double cy = std::floor((y[ymax.front()] - y[ymin.front()]) / D) + 2.0;
-        const double cells = cx * cy * (double)layers;
-        const int64_t b = cells < (double)cnt ? (int64_t)cells : cnt;
-        best = std::max(best, b);
-        if (best >= kMaxWindow + 1) return best;   // already ineligible
-        for (auto *dq : {&xmax, &xmin, &ymax, &ymin})
-            while (!dq->empty() && dq->front() <= i) dq->pop_front();
+        if (cnt > best) {   // (the bound is at most the count)
+            const double cx = std::floor((x[q[0].at[q[0].head]] - x[q[1].at[q[1].head]]) / D) + 2.0;
+            const double cy = std::floor((y[q[2].at[q[2].head]] - y[q[3].at[q[3].head]]) / D) + 2.0;
+            const double cells = cx * cy * (double)layers;
+            const int64_t b = cells < (double)cnt ? (int64_t)cells : cnt;
+            best = std::max(best, b);
+            if (best >= kMaxWindow + 1) return best;   // already ineligible
+        }
+        for (Extreme &e : q) e.head += e.tail > e.head && e.at[e.head] <= i;
     }
     return best;
+}
+
+uint32_t wave_flags(const double *x, const double *y, const double *z, int64_t n, const st_geometry &g, double xmin,
+                    double xmax, double ymin, double ymax, int64_t window)
+{
+    if (n == 0) return kFlagWave;
+    const double D = g.diameter, nl = (double)g.n_linear;
+    // bits of the segment's key box on each axis, for any shift (its extent is
+    // at most floor(range / D) + 6 spheres and at most N)
+    int bits = 0;
+    for (double range : {xmax - xmin, ymax - ymin, z[n - 1] - z[0]}) {
+        const double c = std::min(nl, std::floor(range / D) + 6.0);
+        int b = 1;
+        while (std::ldexp(1.0, b) <= c) ++b;
+        bits += b;
+        if (b > 24) return 0;   // 24-bit hash products
+    }
+    if (bits > kWaveKeyBits) return 0;
+    // A flush keeps the entries of the last scored point's layer: the spheres
+    // of one layer that the points of a z-window one diameter wide can touch.
+    // Where a track spans the voxel in x or y, a face point's carried index
+    // may add entries of the next row or layer: there the fast path's bound
+    // over three layers is used.
+    const double wide = g.length - 4.0 * D;
+    const bool spans = xmax - xmin >= wide || ymax - ymin >= wide;
+    const double w = (spans ? 2.0 : 1.0) * D * (1.0 + 1e-12) + 1e-9;
+    const bool dense = (double)n * D >= 64.0 * (z[n - 1] - z[0]);
+    int64_t kept = window;   // the wider window's bound, where that will do
+    if (!spans && (window < 0 || window > kWaveWindow || dense)) kept = window_bound(x, y, z, n, D, w, 1);
+    else if (window < 0) kept = window_bound(x, y, z, n, D, w, 3);
+    if (kept > kWaveWindow) return 0;
+    // Points of one row that share a sphere share a table entry, and LDS
+    // atomics on one address take two cycles per lane (127 for a full wave
+    // against about 14 on distinct addresses).
+    const bool fits = kept <= kHotWindow && bits + 2 <= kWaveKeyBits;
+    return dense && fits ? kFlagWave | kFlagHot : kFlagWave;
 }
 
 int64_t plan_chunk(const int64_t *offsets, int64_t n_tracks, const int32_t *geom_of_track, int64_t pbase,
@@ -54,6 +93,7 @@ int64_t plan_chunk(const int64_t *offsets, int64_t n_tracks, const int32_t *geom
         td.block0 = bbase + nblocks;
         td.geom = geom_of_track ? geom_of_track[t] : 0;
         td.flags = 0;
+        td.wave = td.pad = 0;
         nblocks += td.nblocks;
     }
     return nblocks;
@@ -81,15 +121,15 @@ void fill_chunk(const double *x, const double *y, const double *z, const double 
         TrackDesc &td = tds[t];
         const int64_t o = td.offset - pbase, n = td.n;
         const int64_t b0 = td.block0 - bbase;
-        std::vector<int64_t> idx(n);
-        std::iota(idx.begin(), idx.end(), 0);
+        // (the key beside the index: sorting indices alone reads z out of order)
+        std::vector<std::pair<double, int64_t>> idx(n);
         const double *zt = Z + base + o;
-        auto zkey = [&](int64_t i) { return std::isnan(zt[i]) ? HUGE_VAL : zt[i]; };
-        std::stable_sort(idx.begin(), idx.end(), [&](int64_t a2, int64_t b2) { return zkey(a2) < zkey(b2); });
+        for (int64_t i = 0; i < n; ++i) idx[i] = {std::isnan(zt[i]) ? HUGE_VAL : zt[i], i};
+        std::stable_sort(idx.begin(), idx.end(), [](const auto &a2, const auto &b2) { return a2.first < b2.first; });
         bool finite = true;
         double xmin = HUGE_VAL, xmax = -HUGE_VAL, ymin = HUGE_VAL, ymax = -HUGE_VAL, esum = 0.0, emax = 0.0;
         for (int64_t k = 0; k < n; ++k) {
-            const int64_t s = base + o + idx[k];
+            const int64_t s = base + o + idx[k].second;
             out.x[o + k] = X[s];
             out.y[o + k] = Y[s];
             out.z[o + k] = Z[s];
@@ -130,15 +170,18 @@ void fill_chunk(const double *x, const double *y, const double *z, const double 
             const double cy = std::min(nl, std::floor((ymax - ymin) / g.diameter) + 6.0);
             fast = fast && cx * cy <= 4294967294.0;
         }
+        int64_t W = -1;
         if (fast) {
             // entries kept by a flush come from the next point's layer (or, for
             // keys with an index equal to N, the layer below): a z-window two
             // diameters wide, touching at most three layers
             const double w = 2.0 * g.diameter * (1.0 + 1e-12) + 1e-9;
-            const int64_t W = window_bound(out.x.data() + o, out.y.data() + o, out.z.data() + o, n, g.diameter, w, 3);
+            W = window_bound(out.x.data() + o, out.y.data() + o, out.z.data() + o, n, g.diameter, w, 3);
             fast = W <= kMaxWindow;
         }
         td.flags = fast ? 0u : kFlagExact;
+        if (fast)
+            td.wave = wave_flags(out.x.data() + o, out.y.data() + o, out.z.data() + o, n, g, xmin, xmax, ymin, ymax, W);
         if (precision == ST_F32) {
             for (int b = 0; b < td.nblocks; ++b) {
                 const int64_t p0 = o + (int64_t)b * kBlk, p1 = std::min<int64_t>(p0 + kBlk, o + n);
@@ -181,6 +224,7 @@ void fill_chunk(const double *x, const double *y, const double *z, const double 
                 bk.dl = dl;
                 bk.fm = 0.5 - (dlq + 1e-12);
                 bk.mrgq = 3.0 * dlq * (1.0 + 2.0 * dlq) + 1e-14 * r2q;
+                sphere_thresholds(r2q, bk.fm, bk.mrgq, &bk.sure, &bk.maybe);
             }
         }
     });

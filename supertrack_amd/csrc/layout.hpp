@@ -16,6 +16,12 @@ constexpr int kBlk = 256;                              // points per library blo
 constexpr int64_t kMaxWindow = 768;                    // fast-path bound on spheres in a z-window two diameters wide
 constexpr int64_t kMaxFastPoints = (int64_t)1 << 22;   // fast-path bound on points per track
 constexpr uint32_t kFlagExact = 1u;                    // TrackDesc::flags: the exact per-segment path
+constexpr uint32_t kFlagWave = 1u;                     // TrackDesc::wave: fits the one-wave kernel
+constexpr uint32_t kFlagHot = 2u;                      // TrackDesc::wave: few spheres take most of a row of points
+constexpr int kHotCopies = 4;                          // table entries per sphere of a kFlagHot track
+constexpr int64_t kHotWindow = 24;                     // kFlagHot: bound on the spheres a flush keeps
+constexpr int64_t kWaveWindow = 224;                   // one-wave kernel: bound on the spheres a flush keeps
+constexpr int kWaveKeyBits = 31;                       // one-wave kernel: bits of its sphere keys
 constexpr double kTwoM44 = 1.0 / 17592186044416.0;
 // Per-point lineal energy limits of the fused kernel (its fixed-point
 // conversions are exact only under 2^51): ST_F32 y * 2^32, ST_F64 y * 2^24.
@@ -29,10 +35,12 @@ struct TrackDesc {
     int32_t nblocks;
     int32_t geom;
     uint32_t flags;
+    uint32_t wave;      // one-wave kernel: kFlagWave, kFlagHot
+    uint32_t pad;
     double xmin, xmax, ymin, ymax, zmax;
 };
 
-// ST_F32 block record (48 B, read through the scalar cache).  The fast path
+// ST_F32 block record (64 B, read through the scalar cache).  The fast path
 // works in lattice units: q = (coordinate - gso) / D, so rint(q) is the
 // sphere index and q - rint(q) the offset from the sphere centre; the voxel
 // faces are the half-way planes q = -1/2 and q = N - 1/2, so a point that is
@@ -44,10 +52,26 @@ struct TrackDesc {
 //           with a wide margin, FP64 rounding of every step, any |shift| <= H');
 //   fm      |q - rint(q)| >= fm: within dl of a half-way plane;
 //   mrgq    |sum (rint(q) - q)^2 - r^2 / D^2| <= mrgq: within the error of
-//           the squared distance.
+//           the squared distance;
+//   sure,   squared distances (lattice units) below which a point is inside
+//   maybe   its sphere and above which it is outside, whichever way a nearby
+//           half-way plane is decided (sphere_thresholds).
 struct BlockF32 {
-    double oqx, oqy, oqz, dl, fm, mrgq;
+    double oqx, oqy, oqz, dl, fm, mrgq, sure, maybe;
 };
+
+// Squared-distance thresholds of a geometry (r2q = r^2 / D^2) from fm and mrgq
+// as above.  A coordinate within dl of a half-way plane has |q - rint(q)| >= fm,
+// so its squared distance is at least fm^2: below min(r2q - mrgq, fm^2) no
+// index is in doubt and the point is inside.  Rounding such a coordinate the
+// other way changes the squared distance by at most 2 (1/2 - fm) per axis, so
+// above r2q + mrgq + 8 (1/2 - fm) the point is outside.
+inline void sphere_thresholds(double r2q, double fm, double mrgq, double *sure, double *maybe)
+{
+    const double f2 = fm > 0.0 ? fm * fm : 0.0;
+    *sure = r2q - mrgq < f2 ? r2q - mrgq : f2;
+    *maybe = r2q + mrgq + 8.0 * (0.5 - fm);
+}
 
 // One FP32 point: offsets from its block's origin (nm) and the energy (eV);
 // the same 16-byte layout as HIP's float4, which the kernel loads.
@@ -76,10 +100,21 @@ int64_t plan_chunk(const int64_t *offsets, int64_t n_tracks, const int32_t *geom
 // (finite data, at most kMaxFastPoints points, fixed-point headroom, indices
 // below 2^30 for any shift, at most 2^32 - 2 spheres in one layer of the
 // track's x/y extent, at most kMaxWindow spheres in any z-window two
-// diameters wide).  ST_F32 also gets the FP32 points and block records.
+// diameters wide), and whether the one-wave kernel takes it (kFlagWave: a
+// fast-path track whose flushes keep at most kWaveWindow spheres and whose
+// key box fits kWaveKeyBits).  ST_F32 also gets the FP32 points and block
+// records.
 void fill_chunk(const double *x, const double *y, const double *z, const double *edep, const int64_t *offsets,
                 int64_t n_tracks, const st_geometry *geoms, int precision, int64_t pbase, int64_t bbase,
                 int64_t nblocks, TrackDesc *tds, ChunkLayout &out);
+
+// The flags of a fast-path track (z-sorted points) for the one-wave kernel: 0,
+// kFlagWave, or kFlagWave | kFlagHot (at least 64 points per layer of spheres
+// on average, and so few spheres in reach that each may take kHotCopies table
+// entries, one per group of lanes).  window: window_bound of a window two
+// diameters wide and three layers, if known (else -1).
+uint32_t wave_flags(const double *x, const double *y, const double *z, int64_t n, const st_geometry &g, double xmin,
+                    double xmax, double ymin, double ymax, int64_t window = -1);
 
 // Largest number of distinct spheres that the points of any z-window of
 // width w can touch, for any shift: min(points, x-cells * y-cells * layers).
