@@ -36,6 +36,7 @@
 #include "st_internal.hpp"
 #include "st_device.hpp"
 #include "layout.hpp"
+#include "layout_gpu.hpp"
 
 #include "batch_kernel.hpp"
 #include "wave_kernel.hpp"
@@ -123,6 +124,29 @@ struct Carve {
 };
 
 
+// Bytes of the one-wave kernel's plan for n tracks (plan_stride).
+size_t plan_bytes(int64_t n)
+{
+    return (size_t)((n + kQueues - 1) / kQueues * kQueues) * sizeof(PlanTrack) + kQueues * sizeof(int64_t);
+}
+
+// A library's tables in one allocation: the track table, geometries, orders
+// (each sized for every track) and the allocation-free pass's plan.
+struct TableOffsets {
+    size_t tracks, geoms, order, wave, rest, plan, bytes;
+    TableOffsets(int64_t n_tracks, int64_t n_geoms)
+    {
+        Carve c;
+        tracks = c.add(n_tracks * sizeof(TrackDesc));
+        geoms = c.add(n_geoms * sizeof(GeomDev));
+        order = c.add(n_tracks * sizeof(int32_t));
+        wave = c.add(n_tracks * sizeof(int32_t));
+        rest = c.add(n_tracks * sizeof(int32_t));
+        plan = c.add(plan_bytes(n_tracks));
+        bytes = c.bytes;
+    }
+};
+
 // Launch shape of the fused kernel.
 struct Launch {
     int slots = 1536, blocks_per_cu = 1, ppt = 1, grid = 0;
@@ -156,9 +180,7 @@ struct st_library {
     float4 *p32 = nullptr;
     double *zfirst = nullptr;
     BlockF32 *blocks = nullptr;
-    // one allocation (finish): the track table, geometries, orders and the
-    // allocation-free pass's plan
-    char *tables = nullptr;
+    char *tables = nullptr;            // TableOffsets; the pointers below lie in it
     TrackDesc *tracks_dev = nullptr;
     GeomDev *geoms_dev = nullptr;
     int32_t *order_dev = nullptr;      // fast_order on the device
@@ -242,10 +264,7 @@ BatchArgs make_args(const st_library *L, const st_batch_opts &o, st_hist *const 
 // Entries of one queue of the plan, and bytes of the whole plan (the queues,
 // then their chunk counts).
 int64_t plan_stride(const st_library *L) { return ((int64_t)L->wave_order.size() + kQueues - 1) / kQueues; }
-size_t plan_bytes(const st_library *L)
-{
-    return (size_t)(kQueues * plan_stride(L)) * sizeof(PlanTrack) + kQueues * sizeof(int64_t);
-}
+size_t plan_bytes(const st_library *L) { return st::plan_bytes((int64_t)L->wave_order.size()); }
 int64_t *plan_totals(const st_library *L, PlanTrack *plan)
 {
     return reinterpret_cast<int64_t *>(plan + kQueues * plan_stride(L));
@@ -685,6 +704,10 @@ int st_library_begin(int64_t n_tracks, int64_t n_points, const st_geometry *geom
         rc = dev_alloc(&L->p32, padded, &bytes);
         if (!rc) rc = dev_alloc(&L->blocks, L->blocks_cap, &bytes);
     }
+    if (!rc) {
+        const TableOffsets at(n_tracks, n_geoms);
+        rc = dev_alloc(&L->tables, at.bytes, &bytes);
+    }
     L->device_bytes = bytes;
     if (rc) {
         st_library_destroy(L);
@@ -727,20 +750,25 @@ int st_library_append(st_library *L, const double *x, const double *y, const dou
     const int64_t nblocks = plan_chunk(offsets, n_tracks, geom_of_track, pbase, bbase, tds);
     if (bbase + nblocks > L->blocks_cap)
         return set_error(ST_EINVAL, "st_library_append: block table overflow");
-    ChunkLayout lay;
-    fill_chunk(x, y, z, edep, offsets, n_tracks, L->geoms.data(), precision, pbase, bbase, nblocks, tds, lay);
-    std::vector<double> &sx = lay.x, &sy = lay.y, &sz = lay.z, &se = lay.e, &zfirst = lay.zfirst;
-    std::vector<PointF32> &p32 = lay.p32;
-    std::vector<BlockF32> &blocks = lay.blocks;
-    int rc = ST_OK;
-    if (!rc) rc = dev_put(L->x64 + pbase, sx.data(), n_points);
-    if (!rc) rc = dev_put(L->y64 + pbase, sy.data(), n_points);
-    if (!rc) rc = dev_put(L->z64 + pbase, sz.data(), n_points);
-    if (!rc) rc = dev_put(L->e64 + pbase, se.data(), n_points);
-    if (!rc) rc = dev_put(L->zfirst + bbase, zfirst.data(), nblocks);
-    if (!rc && precision == ST_F32) {
-        rc = dev_put(reinterpret_cast<PointF32 *>(L->p32) + pbase, p32.data(), n_points);
-        if (!rc) rc = dev_put(L->blocks + bbase, blocks.data(), nblocks);
+    const LayoutDst dst{L->x64 + pbase, L->y64 + pbase, L->z64 + pbase, L->e64 + pbase,
+                        precision == ST_F32 ? reinterpret_cast<PointF32 *>(L->p32) + pbase : nullptr,
+                        L->zfirst + bbase, precision == ST_F32 ? L->blocks + bbase : nullptr};
+    int rc = layout_chunk_device(x + offsets[0], y + offsets[0], z + offsets[0], edep + offsets[0], n_points, n_tracks,
+                                 L->geoms.data(), n_geoms, precision, pbase, bbase, nblocks, tds, dst);
+    if (rc == ST_ENOMEM) {
+        // no room for the device's scratch beside the library: on the host
+        clear_error();
+        ChunkLayout lay;
+        fill_chunk(x, y, z, edep, offsets, n_tracks, L->geoms.data(), precision, pbase, bbase, nblocks, tds, lay);
+        rc = dev_put(dst.x, lay.x.data(), n_points);
+        if (!rc) rc = dev_put(dst.y, lay.y.data(), n_points);
+        if (!rc) rc = dev_put(dst.z, lay.z.data(), n_points);
+        if (!rc) rc = dev_put(dst.e, lay.e.data(), n_points);
+        if (!rc) rc = dev_put(dst.zfirst, lay.zfirst.data(), nblocks);
+        if (!rc && precision == ST_F32) {
+            rc = dev_put(dst.p32, lay.p32.data(), n_points);
+            if (!rc) rc = dev_put(dst.blocks, lay.blocks.data(), nblocks);
+        }
     }
     if (rc) return rc;
     L->tracks_done += n_tracks;
@@ -803,34 +831,23 @@ int st_library_finish(st_library *L)
         gd[i].N = (unsigned long long)g.n_linear;
         gd[i].N2 = gd[i].N * gd[i].N;
     }
-    Carve c;
-    const size_t at_tracks = c.add(L->tracks.size() * sizeof(TrackDesc)), at_geoms = c.add(gd.size() * sizeof(GeomDev));
-    const size_t at_order = c.add(L->fast_order.size() * sizeof(int32_t));
-    const size_t at_wave = c.add(L->wave_order.size() * sizeof(int32_t));
-    const size_t at_rest = c.add(L->rest_order.size() * sizeof(int32_t));
-    const size_t host_bytes = c.bytes, at_plan = c.add(plan_bytes(L));
-    std::vector<char> image(host_bytes);
-    auto put = [&](size_t at, const void *src, size_t bytes) {
-        if (bytes) std::memcpy(image.data() + at, src, bytes);
+    const TableOffsets at(L->n_tracks, n_geoms);
+    std::vector<char> image(at.plan);
+    auto put = [&](size_t where, const void *src, size_t bytes) {
+        if (bytes) std::memcpy(image.data() + where, src, bytes);
     };
-    put(at_tracks, L->tracks.data(), L->tracks.size() * sizeof(TrackDesc));
-    put(at_geoms, gd.data(), gd.size() * sizeof(GeomDev));
-    put(at_order, L->fast_order.data(), L->fast_order.size() * sizeof(int32_t));
-    put(at_wave, L->wave_order.data(), L->wave_order.size() * sizeof(int32_t));
-    put(at_rest, L->rest_order.data(), L->rest_order.size() * sizeof(int32_t));
-    if (!L->tables) {   // (kept for a retry after a failed copy)
-        int64_t bytes = 0;
-        int rc = dev_alloc(&L->tables, c.bytes, &bytes);
-        if (rc) return rc;
-        L->device_bytes += bytes;
-    }
-    ST_HIP_TRY(hipMemcpy(L->tables, image.data(), host_bytes, hipMemcpyHostToDevice));
-    L->tracks_dev = reinterpret_cast<TrackDesc *>(L->tables + at_tracks);
-    L->geoms_dev = reinterpret_cast<GeomDev *>(L->tables + at_geoms);
-    L->order_dev = reinterpret_cast<int32_t *>(L->tables + at_order);
-    L->wave_order_dev = reinterpret_cast<int32_t *>(L->tables + at_wave);
-    L->rest_order_dev = reinterpret_cast<int32_t *>(L->tables + at_rest);
-    L->static_plan = reinterpret_cast<PlanTrack *>(L->tables + at_plan);
+    put(at.tracks, L->tracks.data(), L->tracks.size() * sizeof(TrackDesc));
+    put(at.geoms, gd.data(), gd.size() * sizeof(GeomDev));
+    put(at.order, L->fast_order.data(), L->fast_order.size() * sizeof(int32_t));
+    put(at.wave, L->wave_order.data(), L->wave_order.size() * sizeof(int32_t));
+    put(at.rest, L->rest_order.data(), L->rest_order.size() * sizeof(int32_t));
+    ST_HIP_TRY(hipMemcpy(L->tables, image.data(), image.size(), hipMemcpyHostToDevice));
+    L->tracks_dev = reinterpret_cast<TrackDesc *>(L->tables + at.tracks);
+    L->geoms_dev = reinterpret_cast<GeomDev *>(L->tables + at.geoms);
+    L->order_dev = reinterpret_cast<int32_t *>(L->tables + at.order);
+    L->wave_order_dev = reinterpret_cast<int32_t *>(L->tables + at.wave);
+    L->rest_order_dev = reinterpret_cast<int32_t *>(L->tables + at.rest);
+    L->static_plan = reinterpret_cast<PlanTrack *>(L->tables + at.plan);
     L->finished = true;
     return ST_OK;
 }

@@ -66,6 +66,9 @@ struct BlockF32 {
 // index is in doubt and the point is inside.  Rounding such a coordinate the
 // other way changes the squared distance by at most 2 (1/2 - fm) per axis, so
 // above r2q + mrgq + 8 (1/2 - fm) the point is outside.
+#ifdef __HIPCC__
+__host__ __device__
+#endif
 inline void sphere_thresholds(double r2q, double fm, double mrgq, double *sure, double *maybe)
 {
     const double f2 = fm > 0.0 ? fm * fm : 0.0;
