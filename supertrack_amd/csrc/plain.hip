@@ -82,6 +82,7 @@ constexpr int kScoreBlock = 256;
 constexpr int kScoreRows = 4;
 constexpr int kScoreTile = kScoreBlock * kScoreRows;
 constexpr int kWaves = kScoreBlock / 64;
+constexpr int kPlainTiles = 256;
 
 // Geometry of the membership test, in the reference's units.
 struct ScoreGeom {
@@ -152,10 +153,16 @@ __global__ __launch_bounds__(kScoreBlock) void score_kernel(ScoreArgs a)
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
-    if (tid == 0)
-        s_tile = (int)(atomicAdd(a.ticket, 1ull) - a.ticket_base);
-    __syncthreads();
-    const int tile = s_tile;
+    // Tiles wait for lower tiles only.  Up to kPlainTiles workgroups are all
+    // resident at once, so theirs need no tickets (a device atomic and a
+    // barrier before the first load: 8.0 -> 7.6 us on a 150e3-point track,
+    // 4.8 us either way on 5e3 points).
+    int tile = blockIdx.x;
+    if (a.num_tiles > kPlainTiles) {
+        if (tid == 0) s_tile = (int)(atomicAdd(a.ticket, 1ull) - a.ticket_base);
+        __syncthreads();
+        tile = s_tile;
+    }
     const int64_t base = (int64_t)tile * kScoreTile;
     const double sx = a.shifts[3 * a.os + 0];
     const double sy = a.shifts[3 * a.os + 1];
@@ -170,9 +177,9 @@ __global__ __launch_bounds__(kScoreBlock) void score_kernel(ScoreArgs a)
         key[r] = 0;
         yv[r] = 0.0;
         const int64_t i = base + (int64_t)r * kScoreBlock + tid;
-        if (i < a.n && score_point(a.x[i], a.y[i], a.z[i], sx, sy, sz, a.g, key[r])) {
+        if (i < a.n) {
             yv[r] = a.lin[i];   // ScoreTrackInSphere's value (:322), computed once per track
-            flag[r] = true;
+            flag[r] = score_point(a.x[i], a.y[i], a.z[i], sx, sy, sz, a.g, key[r]);
         }
     }
 
@@ -556,6 +563,337 @@ __global__ __launch_bounds__(kSortThreads) void hist_lds_kernel(HistArgs a)
     const int m = *a.count;
     if (m <= 0 || m > kLdsCap) return;
     lds_sort_reduce_bin(a, m, smem);
+}
+
+// ---------------------------------------------------------------------------
+// Histogram of up to kScanPairs pairs: one launch, no sort
+// ---------------------------------------------------------------------------
+// The keys are split over the workgroups by a hash, so that every sphere's
+// pairs meet in one workgroup.  Each workgroup reads all keys (they are in L2)
+// and lists its own pairs in LDS in pair order; a small table gives each
+// sphere's first pair and its number of pairs, and the thread of the first
+// pair adds the others from the list, left to right.
+//
+// What bounds it is latency (keys, energies and bin edges are dependent trips
+// to memory, and the launch itself takes 2 us), so the work is split until a
+// list is short rather than gathered on one CU, and keys are held in registers
+// so that all are on their way at once.  A 5e3-point track's oversample
+// (about 900 pairs): 10.3 us in one workgroup (hist_lds_kernel), 5.9 us here
+// in 64; a 150e3-point track's (25e3 pairs, 2 nm spheres): 68 us in the radix
+// sort's 8 launches, 21.5 us here.  With few spheres of very many pairs the
+// radix sort's reduction read a sphere's run pair by pair from memory (60 ms
+// for 20 oversamples of 2e5 points in 100 nm spheres).
+//
+// A workgroup whose list would exceed kScanList splits its share over 16
+// hash values more, one after the other; a share that still does not fit holds
+// a few spheres with very many pairs each (a 100 nm sphere can take tens of
+// thousands), which are summed one by one in key order.
+constexpr int64_t kScanPairs = (int64_t)1 << 18;
+constexpr int kScanThreads = 1024;
+constexpr int kScanWaves = kScanThreads / 64;
+constexpr int kScanList = 1024;
+constexpr int kScanTable = 2048;
+constexpr int kScanAhead = 8;    // rows of 64 pairs per wave read before the count is known
+constexpr int kScanRows = 28;    // rows of 64 keys per wave held in registers
+constexpr int kScanSmall = kScanWaves * 64 * kScanAhead;   // pairs capacity read ahead
+
+struct ScanArgs {
+    HistArgs h;
+    int part_bits;   // log2 of the workgroups
+    int capacity;    // of the pairs: how far keys and energies may be read
+};
+
+// Partitions for a pairs capacity: about one per 128 possible pairs (a track
+// puts about a fifth of its points in spheres), 4 to 256.
+inline int scan_part_bits(int64_t capacity)
+{
+    int b = 2;
+    while (b < 8 && (capacity >> b) > 128) ++b;
+    return b;
+}
+
+// Bin of v as bin_fast's, its two edges loaded together.
+__device__ __forceinline__ void scan_bin(const HistArgs &h, double v)
+{
+    if (!(v >= h.guess.e0 && v < h.guess.en)) return;
+    float t;
+    if (h.guess.type == ST_HIST_LIN) t = (float)((v - h.guess.origin) * h.guess.inv_width);
+    else t = (__log2f((float)v) - h.guess.log2_origin) * h.guess.log2_inv_width;
+    int b = (t > 0.0f) ? (int)fminf(t, (float)(h.guess.nbins - 1)) : 0;
+    const double lo = h.edges[b], hi = h.edges[b + 1];
+    if (!(v >= lo && v < hi)) b = bin_fast(h.edges, h.guess, v);
+    if (b >= 0) atomicAdd(&h.bins[b], 1ull);
+}
+
+// AHEAD: a capacity of at most kScanSmall, read before the count is known
+// (garbage past the count is never selected): one trip to memory instead of
+// three.
+template <bool AHEAD>
+__global__ __launch_bounds__(kScanThreads) void hist_scan_kernel(ScanArgs a)
+{
+    __shared__ uint64_t s_key[kScanList];
+    __shared__ double s_y[kScanList];
+    __shared__ unsigned long long s_tkey[kScanTable];   // spheres of the list (~0: none)
+    __shared__ uint32_t s_first[kScanTable], s_num[kScanTable];
+    __shared__ uint32_t s_cnt[2][kScanWaves];
+    __shared__ uint64_t s_min[kScanWaves];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint64_t lt_mask = (1ull << lane) - 1ull;
+    const uint64_t *keys = a.h.keys;
+    const double *y = a.h.y;
+    const int bits = a.part_bits;
+    const uint32_t part = blockIdx.x;
+    auto hash = [](uint64_t k) { return k * 0x9E3779B97F4A7C15ull; };
+    auto mine = [&](uint64_t k) { return (uint32_t)(hash(k) >> (64 - bits)) == part; };
+    constexpr int kRows = AHEAD ? kScanAhead : kScanRows;
+    const int span = ((a.capacity + kScanWaves - 1) / kScanWaves + 63) & ~63;   // per wave, if read ahead
+    uint64_t q[kRows];
+    double yr[AHEAD ? kRows : 1];
+    if constexpr (AHEAD) {
+#pragma unroll
+        for (int u = 0; u < kRows; ++u) {
+            const int i = wave * span + u * 64 + lane;
+            q[u] = 0;
+            yr[u] = 0.0;
+            if (u * 64 < span && i < a.capacity) {
+                q[u] = keys[i];
+                yr[u] = y[i];
+            }
+        }
+    }
+    const int m = *a.h.count;
+    for (int s = tid; s < kScanTable; s += kScanThreads) {
+        s_tkey[s] = ~0ull;
+        s_first[s] = ~0u;
+        s_num[s] = 0;
+    }
+    if (m <= 0) return;
+    // wave w reads keys [w_lo, w_hi): the lists of the waves, in order, are in
+    // pair order
+    const int per_wave = AHEAD ? span : ((m + kScanWaves - 1) / kScanWaves + 63) & ~63;
+    const int w_lo = min(wave * per_wave, m), w_hi = min(w_lo + per_wave, m);
+
+    // the waves' counts -> this wave's offset; all of them in total
+    int half = 0;
+    auto offsets = [&](uint32_t count, uint32_t &total) {
+        // (alternating halves: the next call's counts cannot overtake a slower
+        // wave's reads)
+        if (lane == 0) s_cnt[half][wave] = count;
+        __syncthreads();
+        uint32_t off = 0;
+        total = 0;
+#pragma unroll
+        for (int w = 0; w < kScanWaves; ++w) {
+            const uint32_t c = s_cnt[half][w];
+            off += w < wave ? c : 0u;
+            total += c;
+        }
+        half ^= 1;
+        return off;
+    };
+    auto put = [&](uint64_t mask, bool sel, uint32_t &off, uint64_t k, double v) {
+        if (sel) {
+            const uint32_t pos = off + (uint32_t)__popcll(mask & lt_mask);
+            s_key[pos] = k;
+            s_y[pos] = v;
+        }
+        off += (uint32_t)__popcll(mask);
+    };
+    // Sums and bins the n listed pairs (the table is empty before and after).
+    // A key of ~0 takes no table slot: it is told from the others by its list.
+    auto reduce_list = [&](int n) {
+        __syncthreads();
+        uint64_t k = 0;
+        uint32_t slot = 0;
+        if (tid < n) {
+            k = s_key[tid];
+            slot = (uint32_t)(hash(k) >> 20) & (kScanTable - 1);
+            if (k != ~0ull) {
+                while (true) {
+                    const unsigned long long prev = atomicCAS(&s_tkey[slot], ~0ull, (unsigned long long)k);
+                    if (prev == ~0ull || prev == k) break;
+                    slot = (slot + 1) & (kScanTable - 1);
+                }
+                atomicMin(&s_first[slot], (uint32_t)tid);
+                atomicAdd(&s_num[slot], 1u);
+            }
+        }
+        __syncthreads();
+        bool first = false;
+        uint32_t more = 0;   // pairs of the sphere still to come
+        if (tid < n) {
+            if (k != ~0ull) {
+                first = s_first[slot] == (uint32_t)tid;
+                more = s_num[slot] - 1u;
+            } else {
+                first = true;
+                more = ~0u;
+                for (int j = 0; j < tid; ++j) first = first && s_key[j] != k;
+            }
+        }
+        if (first) {
+            double acc = s_y[tid];
+            for (int j = tid + 1; more != 0u && j < n; j += 4) {
+                uint64_t kj[4];
+                double yj[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int jj = min(j + u, n - 1);
+                    kj[u] = s_key[jj];
+                    yj[u] = s_y[jj];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    if (j + u < n && kj[u] == k) {
+                        acc = acc + yj[u];
+                        --more;
+                    }
+                }
+            }
+            scan_bin(a.h, acc);
+        }
+    };
+    auto clear_table = [&]() {
+        __syncthreads();
+        for (int s = tid; s < kScanTable; s += kScanThreads) {
+            s_tkey[s] = ~0ull;
+            s_first[s] = ~0u;
+            s_num[s] = 0;
+        }
+    };
+    // lists the pairs that match(hash) selects; returns how many there are
+    // (listed only if they fit)
+    auto list_matching = [&](auto match) -> int {
+        uint32_t count = 0, total = 0;
+        auto rows = [&](auto each) {
+#pragma unroll 1
+            for (int base = w_lo; base < w_hi; base += 64 * 8) {
+                uint64_t q[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int i = base + u * 64 + lane;
+                    q[u] = i < w_hi ? keys[i] : 0;
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int i = base + u * 64 + lane;
+                    const bool sel = i < w_hi && match(hash(q[u]));
+                    each(__ballot(sel), sel, q[u], i);
+                }
+            }
+        };
+        rows([&](uint64_t mask, bool, uint64_t, int) { count += (uint32_t)__popcll(mask); });
+        uint32_t off = offsets(count, total);
+        if (total <= (uint32_t)kScanList)
+            rows([&](uint64_t mask, bool sel, uint64_t k, int i) { put(mask, sel, off, k, sel ? y[i] : 0.0); });
+        return (int)total;
+    };
+
+    uint32_t total = 0, count = 0;
+    if (AHEAD || per_wave <= 64 * kRows) {
+        uint32_t sel = 0;   // this lane's selected rows
+        if constexpr (!AHEAD) {
+#pragma unroll
+            for (int u = 0; u < kRows; ++u) {
+                const int i = w_lo + u * 64 + lane;
+                q[u] = 0;
+                if (u * 64 < per_wave && i < w_hi) q[u] = keys[i];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kRows; ++u) {
+            if (u * 64 >= per_wave) continue;
+            const bool s = w_lo + u * 64 + lane < w_hi && mine(q[u]);
+            sel |= s ? 1u << u : 0u;
+            count += (uint32_t)__popcll(__ballot(s));
+        }
+        uint32_t off = offsets(count, total);
+        if (total <= (uint32_t)kScanList) {
+#pragma unroll
+            for (int u = 0; u < kRows; ++u) {
+                if (u * 64 >= per_wave) continue;
+                const bool s = (sel >> u) & 1u;
+                const uint64_t mask = __ballot(s);
+                if (mask == 0ull) continue;
+                double v = 0.0;
+                if constexpr (AHEAD) v = yr[u];
+                else if (s) v = y[w_lo + u * 64 + lane];
+                put(mask, s, off, q[u], v);
+            }
+        }
+    } else {
+        total = (uint32_t)list_matching([&](uint64_t h) { return (uint32_t)(h >> (64 - bits)) == part; });
+    }
+    if (total <= (uint32_t)kScanList) {
+        reduce_list((int)total);
+        return;
+    }
+    for (uint32_t sub = 0; sub < 16; ++sub) {
+        const uint32_t want = part * 16 + sub;
+        auto match = [&](uint64_t h) { return (uint32_t)(h >> (60 - bits)) == want; };
+        __syncthreads();   // the list is free again
+        const int n = list_matching(match);
+        if (n <= kScanList) {
+            reduce_list(n);
+            clear_table();
+            continue;
+        }
+        // few spheres, many pairs: in ascending key order, one scan each, which
+        // sums the current key's pairs in order and finds the next key
+        uint64_t cur = 0;
+        bool have = false;   // false: only look for the first key
+        while (true) {
+            uint64_t next = ~0ull;
+            bool more = false;
+            double acc = -0.0;   // -0.0 + y is y, whatever y is
+            for (int base = 0; base < m; base += kScanThreads) {
+                const int i = base + tid;
+                uint64_t k = 0;
+                bool hit = false;
+                if (i < m) {
+                    k = keys[i];
+                    const bool sel = match(hash(k));
+                    hit = sel && have && k == cur;
+                    if (sel && (!have || k > cur) && (!more || k < next)) {
+                        next = k;
+                        more = true;
+                    }
+                }
+                if (!have) continue;
+                const uint64_t mask = __ballot(hit);
+                uint32_t all;
+                uint32_t off = offsets((uint32_t)__popcll(mask), all);
+                put(mask, hit, off, k, hit ? y[i] : 0.0);
+                __syncthreads();
+                if (tid == 0)
+                    for (uint32_t j = 0; j < all; ++j) acc = acc + s_y[j];
+                __syncthreads();
+            }
+            // the smallest next key of all threads
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1) {
+                const uint64_t o = __shfl_xor(next, d, 64);
+                const bool om = __shfl_xor((int)more, d, 64) != 0;
+                if (om && (!more || o < next)) next = o;
+                more = more || om;
+            }
+            __syncthreads();
+            if (lane == 0) {
+                s_min[wave] = next;
+                s_cnt[0][wave] = more ? 1u : 0u;
+            }
+            __syncthreads();
+            if (have && tid == 0) scan_bin(a.h, acc);
+            have = false;
+            for (int w = 0; w < kScanWaves; ++w) {
+                if (!s_cnt[0][w]) continue;
+                if (!have || s_min[w] < cur) cur = s_min[w];
+                have = true;
+            }
+            __syncthreads();
+            if (!have) break;
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -986,6 +1324,13 @@ int hist_add_pairs(st_hist *h, const st_pairs *pairs, hipStream_t stream)
     ha.guess = h->guess;
     ha.bins = (unsigned long long *)h->bins_dev;
     h->bins_zero = false;
+    if (pairs->capacity <= kScanPairs) {
+        const ScanArgs sa{ha, scan_part_bits(pairs->capacity), (int)pairs->capacity};
+        if (pairs->capacity <= kScanSmall) hist_scan_kernel<true><<<1 << sa.part_bits, kScanThreads, 0, stream>>>(sa);
+        else hist_scan_kernel<false><<<1 << sa.part_bits, kScanThreads, 0, stream>>>(sa);
+        ST_HIP_TRY(hipGetLastError());
+        return ST_OK;
+    }
     // small inputs (decided on the device) take the one-workgroup LDS sort
     hist_lds_kernel<<<1, kSortThreads, kLdsBytes, stream>>>(ha);
     ST_HIP_TRY(hipGetLastError());
@@ -1430,7 +1775,7 @@ int st_vcs_process_oversample(st_vcs *m, const st_track *track, st_pairs *out)
     a.num_tiles = tiles;
     score_kernel<<<tiles, kScoreBlock, 0, m->stream>>>(a);
     ST_HIP_TRY(hipGetLastError());
-    m->ticket_base += (uint64_t)tiles;
+    if (tiles > kPlainTiles) m->ticket_base += (uint64_t)tiles;
     m->oversample++;
     return ST_OK;
 }
