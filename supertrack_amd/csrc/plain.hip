@@ -1456,6 +1456,12 @@ int queue_flush(st_vcs *m)
     return rc;
 }
 
+void queue_consume(st_vcs *m, st_hist *h)
+{
+    m->queue_consumers.back().push_back(h);
+    if (std::find(h->producers.begin(), h->producers.end(), m) == h->producers.end()) h->producers.push_back(m);
+}
+
 // Flushes every method whose queued oversamples h consumes.
 int queue_flush_producers(st_hist *h)
 {
@@ -1927,9 +1933,7 @@ int st_hist_add(st_hist *h, const st_pairs *pairs)
     if (pairs->volume) {
         st_vcs *m = queue_producer(pairs->volume);
         if (m && m->queue_active && m->queue_count > 0 && m->queue_pairs.volume == pairs->volume) {
-            m->queue_consumers.back().push_back(h);
-            if (std::find(h->producers.begin(), h->producers.end(), m) == h->producers.end())
-                h->producers.push_back(m);
+            queue_consume(m, h);
             return ST_OK;
         }
     }

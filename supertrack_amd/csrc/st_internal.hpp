@@ -119,4 +119,6 @@ struct st_vcs {
 namespace st {
 // Runs the pending queued oversamples of m (no-op if none).
 int queue_flush(st_vcs *m);
+// Makes h a consumer of m's last queued oversample.
+void queue_consume(st_vcs *m, st_hist *h);
 }  // namespace st
