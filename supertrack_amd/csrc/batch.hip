@@ -207,6 +207,7 @@ struct st_batch {
     PlanTrack *wave_plan = nullptr;              // its work queues
     unsigned int *slab = nullptr;                // its workgroups' histograms
     unsigned long long *slab_stats = nullptr;    // and statistics
+    CtlReport *report = nullptr;                 // the last pass's outcome (pinned host memory, or null)
     int hist_words = 0;
     BatchCtl *ctl = nullptr;   // per-pass control block (device); the plan and slabs follow it
     RecArgs rec{};                // recording buffers (cap 0: off)
@@ -308,8 +309,8 @@ int launch_plan(const st_library *L, int n_os, const WaveLaunch &w, PlanTrack *p
 }
 
 // Queues one pass: the control-block reset, then (wave non-null) the one-wave
-// kernel and the sum of its workgroups' histograms, and the block kernel over
-// the tracks of args.
+// kernel, the block kernel over the tracks of args, and (wave) the sum of the
+// one-wave kernel's workgroup histograms, which ends the pass.
 int launch_pass(int precision, const BatchArgs &args, const Launch &ln, const WaveArgs *wave, const WaveLaunch &w,
                 hipStream_t stream)
 {
@@ -320,16 +321,17 @@ int launch_pass(int precision, const BatchArgs &args, const Launch &ln, const Wa
         void *kargs[] = {&a};
         ST_HIP_TRY(hipLaunchKernel(wave_kernel_ptr(precision), dim3(w.grid), dim3(64 * w.wg_waves), kargs, w.lds,
                                    stream));
-        if (a.slab) {
-            slab_sum_kernel<<<(a.b.hist_lds_words + 63) / 64 + 1, 1024, 0, stream>>>(a, w.grid);
-            ST_HIP_TRY(hipGetLastError());
-        }
     }
-    if (args.n_seg == 0) return ST_OK;
-    const void *k = pick_kernel(precision, ln.slots, ln.ppt);
-    BatchArgs a = args;
-    void *kargs[] = {&a};
-    ST_HIP_TRY(hipLaunchKernel(k, dim3(ln.grid), dim3(kBT), kargs, ln.lds, stream));
+    if (args.n_seg > 0) {
+        const void *k = pick_kernel(precision, ln.slots, ln.ppt);
+        BatchArgs a = args;
+        void *kargs[] = {&a};
+        ST_HIP_TRY(hipLaunchKernel(k, dim3(ln.grid), dim3(kBT), kargs, ln.lds, stream));
+    }
+    if (wave && wave->plan.n_tracks > 0 && wave->slab) {
+        slab_sum_kernel<<<(wave->b.hist_lds_words + 63) / 64 + 1, 1024, 0, stream>>>(*wave, w.grid);
+        ST_HIP_TRY(hipGetLastError());
+    }
     return ST_OK;
 }
 
@@ -342,6 +344,7 @@ int launch_fast(st_batch *b)
     WaveArgs wa = make_wave_args(L, b->opts, b->hists.data(), (int)b->hists.size(), b->wave, b->ctl, b->wave_plan,
                                  b->slab, b->slab_stats);
     wa.b.rec = a.rec;
+    wa.report = b->report;
     return launch_pass(L->precision, a, b->ln, &wa, b->wave, b->stream);
 }
 
@@ -654,15 +657,29 @@ int static_scratch(BatchCtl **out)
 }
 
 // Waits for the work queued on `stream` and copies the control block back.
-int read_ctl(const BatchCtl *ctl, hipStream_t stream, BatchCtl *out)
+int read_ctl(const BatchCtl *ctl, hipStream_t stream, CtlReport *out)
 {
-    ST_HIP_TRY(hipMemcpyAsync(out, ctl, sizeof *out, hipMemcpyDeviceToHost, stream));
+    constexpr size_t kBytes = offsetof(BatchCtl, tickets);   // the host needs no queue state
+    BatchCtl c;
+    ST_HIP_TRY(hipMemcpyAsync(&c, ctl, kBytes, hipMemcpyDeviceToHost, stream));
     ST_HIP_TRY(hipStreamSynchronize(stream));
+    out->rec_count = c.rec_count;
+    out->error = c.error;
+    std::copy(c.stats, c.stats + kStats, out->stats);
+    return ST_OK;
+}
+
+// The same for a batch: a pass of the one-wave kernel has already reported.
+int read_report(const st_batch *b, CtlReport *out)
+{
+    if (!b->wave.on || !b->report) return read_ctl(b->ctl, b->stream, out);
+    ST_HIP_TRY(hipStreamSynchronize(b->stream));
+    *out = *b->report;
     return ST_OK;
 }
 
 // The kernel's error flag and the conservation totals of a finished pass.
-int check_ctl(const BatchCtl &c)
+int check_ctl(const CtlReport &c)
 {
     if (c.error)
         return set_error(ST_ESTATE,
@@ -964,6 +981,8 @@ int st_batch_create(st_library *lib, const st_batch_opts *opts, st_hist *const *
         b->wave_plan = reinterpret_cast<PlanTrack *>(work + at_plan);
         b->slab_stats = reinterpret_cast<unsigned long long *>(work + at_stats);
         b->slab = reinterpret_cast<unsigned int *>(work + at_slab);
+        b->report = (CtlReport *)report_slot_take(sizeof(CtlReport));   // (null: the control block is copied)
+        if (b->report) *b->report = CtlReport{};
         rc = launch_plan(lib, opts->n_oversamples, b->wave, b->wave_plan, b->stream);
         if (rc) return fail(rc);
     }
@@ -1029,7 +1048,7 @@ int st_batch_run_static(st_library *lib, const st_batch_opts *opts, st_hist *con
         wa = make_wave_args(lib, *opts, hists, n_hists, w, ctl, lib->static_plan, nullptr, nullptr);
     rc = launch_pass(lib->precision, a, ln, wave ? &wa : nullptr, w, stream);
     if (rc || !stats7) return rc;
-    BatchCtl c;
+    CtlReport c;
     rc = read_ctl(ctl, stream, &c);
     if (rc) return rc;
     for (int i = 0; i < kStats; ++i) stats7[i] = (int64_t)c.stats[i];
@@ -1078,6 +1097,7 @@ int st_batch_run(st_batch *b)
         if (rc) return rc;
     }
     ST_HIP_TRY(hipEventRecord(b->ev[1], b->stream));
+    if (b->lib->exact.empty()) return ST_OK;
     int rc = run_exact(b);
     if (rc) return rc;
     ST_HIP_TRY(hipEventRecord(b->ev[2], b->stream));
@@ -1088,17 +1108,19 @@ int st_batch_times(st_batch *b, float *ms2)
 {
     if (!b || !ms2) return set_error(ST_EINVAL, "st_batch_times: null argument");
     if (!b->ev[0]) return set_error(ST_ESTATE, "st_batch_times before st_batch_run");
-    ST_HIP_TRY(hipEventSynchronize(b->ev[2]));
+    const bool exact = !b->lib->exact.empty();
+    ST_HIP_TRY(hipEventSynchronize(b->ev[exact ? 2 : 1]));
     ST_HIP_TRY(hipEventElapsedTime(&ms2[0], b->ev[0], b->ev[1]));
-    ST_HIP_TRY(hipEventElapsedTime(&ms2[1], b->ev[1], b->ev[2]));
+    ms2[1] = 0.0f;
+    if (exact) ST_HIP_TRY(hipEventElapsedTime(&ms2[1], b->ev[1], b->ev[2]));
     return ST_OK;
 }
 
 int st_batch_sync(st_batch *b)
 {
     if (!b) return set_error(ST_EINVAL, "st_batch_sync: null batch");
-    BatchCtl c;
-    int rc = read_ctl(b->ctl, b->stream, &c);
+    CtlReport c;
+    int rc = read_report(b, &c);
     if (rc) return rc;
     return check_ctl(c);
 }
@@ -1106,8 +1128,8 @@ int st_batch_sync(st_batch *b)
 int st_batch_stats(st_batch *b, int64_t *stats3)
 {
     if (!b || !stats3) return set_error(ST_EINVAL, "st_batch_stats: null argument");
-    BatchCtl c;
-    int rc = read_ctl(b->ctl, b->stream, &c);
+    CtlReport c;
+    int rc = read_report(b, &c);
     if (rc) return rc;
     for (int i = 0; i < 3; ++i) stats3[i] = (int64_t)c.stats[i];
     return ST_OK;
@@ -1116,8 +1138,8 @@ int st_batch_stats(st_batch *b, int64_t *stats3)
 int st_batch_balance(st_batch *b, uint64_t *balance4)
 {
     if (!b || !balance4) return set_error(ST_EINVAL, "st_batch_balance: null argument");
-    BatchCtl c;
-    int rc = read_ctl(b->ctl, b->stream, &c);
+    CtlReport c;
+    int rc = read_report(b, &c);
     if (rc) return rc;
     for (int i = 0; i < 4; ++i) balance4[i] = c.stats[3 + i];
     return ST_OK;
@@ -1166,8 +1188,8 @@ int st_batch_record(st_batch *b, int64_t capacity)
 int st_batch_record_fetch(st_batch *b, int64_t *segments, uint64_t *keys, double *sums, int64_t *count)
 {
     if (!b || !count) return set_error(ST_EINVAL, "st_batch_record_fetch: null argument");
-    BatchCtl ctl;
-    int rc = read_ctl(b->ctl, b->stream, &ctl);
+    CtlReport ctl;
+    int rc = read_report(b, &ctl);
     if (rc) return rc;
     const unsigned long long c = ctl.rec_count;
     *count = (int64_t)c;
@@ -1218,6 +1240,7 @@ void st_batch_destroy(st_batch *b)
     for (st_vcs *m : b->methods) st_vcs_destroy(m);
     for (hipEvent_t e : b->ev)
         if (e) (void)hipEventDestroy(e);
+    report_slot_give(b->report, sizeof(CtlReport));
     st_track_free(&b->scratch);
     st_pairs_free(&b->pairs);
     void *ptrs[] = {b->ctl, b->rec.seg, b->rec.key, b->rec.box, b->rec.sum, b->rec_dev};

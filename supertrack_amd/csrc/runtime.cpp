@@ -62,6 +62,52 @@ hipError_t pinned_malloc(void **p, size_t bytes, unsigned int flags)
 }
 
 namespace {
+// Slots of pinned, mapped host memory that the device reports into, kept for
+// the next caller: making one costs about 25 us.  At most kKeptSlots of a
+// size wait unused; st_shutdown gives them back.
+constexpr size_t kSlotBytes[] = {4096, 65536};
+constexpr size_t kKeptSlots = 8;
+std::mutex g_slot_mu;
+std::vector<void *> g_slots[2];
+
+int slot_class(size_t bytes) { return bytes <= kSlotBytes[0] ? 0 : 1; }
+}  // namespace
+
+void *report_slot_take(size_t bytes)
+{
+    if (bytes > kSlotBytes[1]) return nullptr;
+    const int c = slot_class(bytes);
+    {
+        std::lock_guard<std::mutex> lock(g_slot_mu);
+        if (!g_slots[c].empty()) {
+            void *p = g_slots[c].back();
+            g_slots[c].pop_back();
+            return p;
+        }
+    }
+    void *p = nullptr;
+    if (hipHostMalloc(&p, kSlotBytes[c], hipHostMallocMapped | hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return p;
+}
+
+void report_slot_give(void *p, size_t bytes)
+{
+    if (!p) return;
+    const int c = slot_class(bytes);
+    {
+        std::lock_guard<std::mutex> lock(g_slot_mu);
+        if (g_slots[c].size() < kKeptSlots) {
+            g_slots[c].push_back(p);
+            return;
+        }
+    }
+    (void)hipHostFree(p);
+}
+
+namespace {
 // per-device default streams, created on first use, destroyed by st_shutdown
 std::mutex g_stream_mu;
 std::vector<hipStream_t> g_streams;
@@ -223,6 +269,13 @@ int st_debug_fail_allocation(int64_t countdown)
 
 int st_shutdown(void)
 {
+    {
+        std::lock_guard<std::mutex> slots(g_slot_mu);
+        for (std::vector<void *> &kept : g_slots) {
+            for (void *p : kept) (void)hipHostFree(p);
+            kept.clear();
+        }
+    }
     std::lock_guard<std::mutex> lock(g_stream_mu);
     int cur = 0;
     const bool have_cur = hipGetDevice(&cur) == hipSuccess;

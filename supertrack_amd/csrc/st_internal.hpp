@@ -11,6 +11,10 @@
 namespace st {
 
 int device_cu_count();
+// Pinned, device-mapped host memory for up to 64 KiB that the device reports
+// into (null: none to be had); given back once no queued work writes to it.
+void *report_slot_take(size_t bytes);
+void report_slot_give(void *p, size_t bytes);
 void make_geometry(double half_length_ini, double diameter_ini, st_geometry *g);
 void make_edges(int type, float lo, float hi, int nbins, double *edges);
 

@@ -48,9 +48,17 @@ struct WavePlan {
     unsigned long long *tickets;   // [kQueues * kTicketPad], cleared per pass
 };
 
+// What the host reads of a pass's control block.
+struct CtlReport {
+    unsigned long long rec_count;
+    unsigned long long stats[kStats];
+    int error, pad;
+};
+
 struct WaveArgs {
     BatchArgs b;
     WavePlan plan;
+    CtlReport *report;              // where slab_sum_kernel reports the pass (host memory; null: nowhere)
     unsigned int *slab;             // [workgroup][hist_lds_words]; null: merge with atomics
     unsigned long long *slab_stats; // [workgroup][kStats]
 };
@@ -978,7 +986,7 @@ void wave_kernel(WaveArgs wa)
 
 // Adds the workgroups' histograms and statistics to the device counters: 64
 // bins per workgroup, its 16 waves over the slab's rows (the last workgroup:
-// the statistics).  Launched with (hist_lds_words + 63) / 64 + 1 workgroups.
+// the statistics, and the report to the host).  Launched with (hist_lds_words + 63) / 64 + 1 workgroups.
 __global__ __launch_bounds__(1024) void slab_sum_kernel(WaveArgs wa, int rows)
 {
     __shared__ unsigned long long s_sum[16][64];
@@ -997,11 +1005,20 @@ __global__ __launch_bounds__(1024) void slab_sum_kernel(WaveArgs wa, int rows)
     __syncthreads();
     if (wave != 0) return;
     for (int k = 1; k < 16; ++k) sum += s_sum[k][lane];
-    if (sum == 0) return;
     if (stats) {
-        atomicAdd(&wa.b.ctl->stats[lane], sum);
+        // the last kernel of the pass: the control block is complete
+        if (lane < kStats) {
+            sum += wa.b.ctl->stats[lane];
+            wa.b.ctl->stats[lane] = sum;
+        }
+        if (wa.report) {
+            if (lane < kStats) wa.report->stats[lane] = sum;
+            if (lane == kStats) wa.report->rec_count = wa.b.ctl->rec_count;
+            if (lane == kStats + 1) wa.report->error = wa.b.ctl->error;
+        }
         return;
     }
+    if (sum == 0) return;
     for (int h = 0; h < wa.b.n_hists; ++h) {
         const int b = w - wa.b.hist[h].lds_offset;
         if (b >= 0 && b < wa.b.hist[h].guess.nbins) atomicAdd(&wa.b.hist[h].bins[b], sum);
