@@ -37,6 +37,7 @@
 #include "st_device.hpp"
 #include "layout.hpp"
 #include "layout_gpu.hpp"
+#include "transfer.hpp"
 
 #include "batch_kernel.hpp"
 #include "wave_kernel.hpp"
@@ -868,7 +869,8 @@ int st_library_finish(st_library *L)
     put(at.order, L->fast_order.data(), L->fast_order.size() * sizeof(int32_t));
     put(at.wave, L->wave_order.data(), L->wave_order.size() * sizeof(int32_t));
     put(at.rest, L->rest_order.data(), L->rest_order.size() * sizeof(int32_t));
-    ST_HIP_TRY(hipMemcpy(L->tables, image.data(), image.size(), hipMemcpyHostToDevice));
+    const UploadPart part{L->tables, image.data(), image.size()};
+    ST_HIP_TRY(upload(&part, 1));
     L->tracks_dev = reinterpret_cast<TrackDesc *>(L->tables + at.tracks);
     L->geoms_dev = reinterpret_cast<GeomDev *>(L->tables + at.geoms);
     L->order_dev = reinterpret_cast<int32_t *>(L->tables + at.order);
@@ -929,7 +931,7 @@ void st_library_destroy(st_library *L)
     (void)hipDeviceSynchronize();
     void *ptrs[] = {L->x64, L->y64, L->z64, L->e64, L->p32,
                     L->zfirst, L->blocks, L->tables};
-    for (void *p : ptrs) (void)hipFree(p);
+    for (void *p : ptrs) (void)dev_free(p);
     delete L;
 }
 
@@ -1167,11 +1169,11 @@ int st_batch_params(const st_batch *b, int32_t *p)
 int st_batch_record(st_batch *b, int64_t capacity)
 {
     if (!b || capacity < 0) return set_error(ST_EINVAL, "st_batch_record: bad arguments");
-    (void)hipFree(b->rec.seg);
-    (void)hipFree(b->rec.key);
-    (void)hipFree(b->rec.box);
-    (void)hipFree(b->rec.sum);
-    (void)hipFree(b->rec_dev);
+    (void)dev_free(b->rec.seg);
+    (void)dev_free(b->rec.key);
+    (void)dev_free(b->rec.box);
+    (void)dev_free(b->rec.sum);
+    (void)dev_free(b->rec_dev);
     b->rec = RecArgs{};
     b->rec_dev = nullptr;
     if (capacity == 0) return ST_OK;
@@ -1244,7 +1246,7 @@ void st_batch_destroy(st_batch *b)
     st_track_free(&b->scratch);
     st_pairs_free(&b->pairs);
     void *ptrs[] = {b->ctl, b->rec.seg, b->rec.key, b->rec.box, b->rec.sum, b->rec_dev};
-    for (void *p : ptrs) (void)hipFree(p);
+    for (void *p : ptrs) (void)dev_free(p);
     delete b;
 }
 

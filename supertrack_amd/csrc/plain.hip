@@ -16,6 +16,7 @@
 
 #include "st_common.hpp"
 #include "st_internal.hpp"
+#include "transfer.hpp"
 #include "st_device.hpp"
 
 namespace st {
@@ -1199,9 +1200,22 @@ __global__ void zero_u64_kernel(unsigned long long *p, int64_t n)
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = 0;
 }
 
+// New pairs (st_pairs_alloc): zeros and their count in one launch, where two
+// clears and a copy took three.
+__global__ void empty_pairs_kernel(unsigned long long *key, unsigned long long *y, int64_t n, int32_t *count,
+                                   int32_t value)
+{
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i0 == 0) *count = value;
+    for (int64_t i = i0; i < n; i += stride) {
+        key[i] = 0;
+        y[i] = 0;
+    }
+}
+
 // Counts to host memory (pinned, mapped), cleared behind: one launch and one
-// wait where a copy, a wait, a clear and a wait took four (fetch of a small batch's 1000
-// bins: 38 us -> 14 us).
+// wait where a copy, a wait, a clear and a wait took four (1000 bins: 38 us -> 14 us).
 __global__ void fetch_counts_kernel(unsigned long long *bins, unsigned long long *out, int n, int reset)
 {
     const int stride = (int)(gridDim.x * blockDim.x);
@@ -1235,7 +1249,7 @@ int grow(T **p, int64_t *cap, int64_t need)
 {
     if (need <= *cap && *p) return ST_OK;
     if (*p) {
-        (void)hipFree(*p);
+        (void)dev_free(*p);
         *p = nullptr;
         *cap = 0;
     }
@@ -1292,18 +1306,21 @@ int ensure_sort_buffers(st_hist *h, int64_t cap)
 {
     // each allocated on its own, so that a failure between them leaves no
     // half-made state behind for the next call
+    bool cleared = false;
     if (!h->digit_counts) {
         ST_ALLOC_TRY(dev_malloc((void **)&h->digit_counts, (size_t)kMaxPasses * kGDigits * sizeof(unsigned int)));
         ST_HIP_TRY(hipMemset(h->digit_counts, 0, (size_t)kMaxPasses * kGDigits * sizeof(unsigned int)));
+        cleared = true;
     }
     if (!h->os_ticket) {
         ST_ALLOC_TRY(dev_malloc((void **)&h->os_ticket, sizeof(unsigned long long)));
         ST_HIP_TRY(hipMemset(h->os_ticket, 0, sizeof(unsigned long long)));
         h->os_ticket_base = 0;
+        cleared = true;
     }
     if (cap > h->sort_capacity) {
-        (void)hipFree(h->keys_a); (void)hipFree(h->keys_b); (void)hipFree(h->vals_a); (void)hipFree(h->vals_b);
-        (void)hipFree(h->os_status);
+        (void)dev_free(h->keys_a); (void)dev_free(h->keys_b); (void)dev_free(h->vals_a); (void)dev_free(h->vals_b);
+        (void)dev_free(h->os_status);
         h->keys_a = h->keys_b = nullptr;
         h->vals_a = h->vals_b = nullptr;
         h->os_status = nullptr;
@@ -1316,7 +1333,9 @@ int ensure_sort_buffers(st_hist *h, int64_t cap)
         ST_ALLOC_TRY(dev_malloc((void **)&h->os_status, (size_t)tiles * kGDigits * sizeof(unsigned long long)));
         ST_HIP_TRY(hipMemset(h->os_status, 0, (size_t)tiles * kGDigits * sizeof(unsigned long long)));
         h->sort_capacity = cap;
+        cleared = true;
     }
+    if (cleared) ST_HIP_TRY(hipStreamSynchronize(nullptr));   // h's stream does not wait for the clears
     return ST_OK;
 }
 
@@ -1419,8 +1438,16 @@ int queue_flush(st_vcs *m)
     const int cnt = m->queue_count;
     const int64_t n = m->n;
     int rc = ensure_sort_attributes();
-    if (!rc) rc = grow(&m->queue_key, &m->queue_key_capacity, std::max<int64_t>((int64_t)cnt * n, 1));
-    if (!rc) rc = grow(&m->queue_y, &m->queue_y_capacity, std::max<int64_t>((int64_t)cnt * n, 1));
+    // (rows grow by doubling up to 2^20 pairs: a loop over tracks of growing
+    // size would otherwise free and allocate them again track by track)
+    int64_t rows = (int64_t)cnt * n;
+    if (rows <= (1 << 20)) {
+        int64_t r = 4096;
+        while (r < rows) r *= 2;
+        rows = r;
+    }
+    if (!rc) rc = grow(&m->queue_key, &m->queue_key_capacity, rows);
+    if (!rc) rc = grow(&m->queue_y, &m->queue_y_capacity, rows);
     std::vector<st_hist *> consumers;
     if (!rc) {
         QueuedArgs a{};
@@ -1557,11 +1584,8 @@ int st_track_upload(st_track *t, const double *x, const double *y, const double 
     const size_t bytes = (size_t)n * sizeof(double);
     if (bytes) {
         ST_HIP_TRY(hipDeviceSynchronize());
-        ST_HIP_TRY(hipMemcpy(t->x, x, bytes, hipMemcpyHostToDevice));
-        ST_HIP_TRY(hipMemcpy(t->y, y, bytes, hipMemcpyHostToDevice));
-        ST_HIP_TRY(hipMemcpy(t->z, z, bytes, hipMemcpyHostToDevice));
-        ST_HIP_TRY(hipMemcpy(t->edep, edep, bytes, hipMemcpyHostToDevice));
-        ST_HIP_TRY(hipDeviceSynchronize());
+        const UploadPart parts[4] = {{t->x, x, bytes}, {t->y, y, bytes}, {t->z, z, bytes}, {t->edep, edep, bytes}};
+        ST_HIP_TRY(upload(parts, 4));
     }
     t->n = n;
     return ST_OK;
@@ -1570,10 +1594,10 @@ int st_track_upload(st_track *t, const double *x, const double *y, const double 
 void st_track_free(st_track *t)
 {
     if (!t) return;
-    (void)hipFree(t->x);
-    (void)hipFree(t->y);
-    (void)hipFree(t->z);
-    (void)hipFree(t->edep);
+    (void)dev_free(t->x);
+    (void)dev_free(t->y);
+    (void)dev_free(t->z);
+    (void)dev_free(t->edep);
     t->x = t->y = t->z = t->edep = nullptr;
     t->n = t->capacity = 0;
 }
@@ -1592,23 +1616,21 @@ int st_pairs_alloc(st_pairs *p, int64_t capacity)
     hipError_t e1 = dev_malloc((void **)&p->volume, n * sizeof(uint64_t));
     hipError_t e2 = dev_malloc((void **)&p->edep, n * sizeof(double));
     hipError_t e3 = dev_malloc((void **)&p->count_dev, sizeof(int32_t));
-    hipError_t e4 = pinned_malloc((void **)&p->num_elements, sizeof(int32_t),
-                                  hipHostMallocMapped | hipHostMallocCoherent);
-    if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess || e4 != hipSuccess) {
-        if (e4 != hipSuccess) p->num_elements = nullptr;
+    p->num_elements = (int32_t *)report_slot_take(sizeof(int32_t), true);
+    if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess || !p->num_elements) {
         st_pairs_free(p);
         return set_error(ST_ENOMEM, "st_pairs_alloc: device or pinned host allocation failed");
     }
-    // kernels store through the same address (unified addressing)
-    void *mapped = nullptr;
-    if (hipHostGetDevicePointer(&mapped, p->num_elements, 0) != hipSuccess || mapped != p->num_elements) {
-        st_pairs_free(p);
-        return set_error(ST_EHIP, "st_pairs_alloc: pinned count is not mapped at its host address");
-    }
-    ST_HIP_TRY(hipMemset(p->volume, 0, n * sizeof(uint64_t)));
-    ST_HIP_TRY(hipMemset(p->edep, 0, n * sizeof(double)));
     const int32_t c = (int32_t)capacity;
-    ST_HIP_TRY(hipMemcpy(p->count_dev, &c, sizeof c, hipMemcpyHostToDevice));
+    hipStream_t stream = default_stream();
+    empty_pairs_kernel<<<grid_for((int64_t)n, 256, 4096), 256, 0, stream>>>(
+        (unsigned long long *)p->volume, (unsigned long long *)p->edep, (int64_t)n, p->count_dev, c);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(stream);
+    if (e != hipSuccess) {
+        st_pairs_free(p);
+        return set_error(ST_EHIP, "st_pairs_alloc: %s", hipGetErrorString(e));
+    }
     *p->num_elements = c;
     p->capacity = capacity;
     p->key_bound = 0;
@@ -1623,10 +1645,10 @@ void st_pairs_free(st_pairs *p)
         if (m) (void)queue_flush(m);
     }
     if (p->volume || p->edep || p->count_dev || p->num_elements) (void)hipDeviceSynchronize();
-    (void)hipFree(p->volume);
-    (void)hipFree(p->edep);
-    (void)hipFree(p->count_dev);
-    if (p->num_elements) (void)hipHostFree(p->num_elements);
+    (void)dev_free(p->volume);
+    (void)dev_free(p->edep);
+    (void)dev_free(p->count_dev);
+    report_slot_give(p->num_elements, sizeof(int32_t));   // (the device is idle)
     p->volume = nullptr;
     p->edep = nullptr;
     p->count_dev = nullptr;
@@ -1664,6 +1686,7 @@ int st_vcs_create(const st_geometry *g, int32_t shift_xy, int32_t shift_z,
     m->stream = default_stream();
     hipError_t e = dev_malloc((void **)&m->ticket, sizeof(unsigned long long));
     if (e == hipSuccess) e = hipMemset(m->ticket, 0, sizeof(unsigned long long));
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);   // m's stream does not wait for the clear
     if (e != hipSuccess) {
         st_vcs_destroy(m);
         return set_error(hip_status(e), "st_vcs_create: %s", hipGetErrorString(e));
@@ -1839,13 +1862,13 @@ void st_vcs_destroy(st_vcs *m)
     if (!m) return;
     (void)queue_flush(m);
     if (m->stream) (void)hipStreamSynchronize(m->stream);
-    (void)hipFree(m->queue_key);
-    (void)hipFree(m->queue_y);
+    (void)dev_free(m->queue_key);
+    (void)dev_free(m->queue_y);
     if (m->queue_event) (void)hipEventDestroy(m->queue_event);
-    (void)hipFree(m->lineal);
-    (void)hipFree(m->shifts);
-    (void)hipFree(m->status);
-    (void)hipFree(m->ticket);
+    (void)dev_free(m->lineal);
+    (void)dev_free(m->shifts);
+    (void)dev_free(m->status);
+    (void)dev_free(m->ticket);
     delete m;
 }
 
@@ -1891,10 +1914,10 @@ int st_hist_create(int32_t type, float lo, float hi, int32_t nbins, st_hist **ou
     h->stream = default_stream();
     hipError_t e = dev_malloc((void **)&h->edges_dev, ((size_t)nbins + 1) * sizeof(double));
     if (e == hipSuccess) e = dev_malloc((void **)&h->bins_dev, (size_t)nbins * sizeof(uint64_t));
-    if (e == hipSuccess)
+    if (e == hipSuccess) e = hipMemset(h->bins_dev, 0, (size_t)nbins * sizeof(uint64_t));
+    if (e == hipSuccess)   // (ends after the clear, which h's stream does not wait for)
         e = hipMemcpy(h->edges_dev, h->edges_host.data(), ((size_t)nbins + 1) * sizeof(double),
                       hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemset(h->bins_dev, 0, (size_t)nbins * sizeof(uint64_t));
     if (e != hipSuccess) {
         st_hist_destroy(h);
         return set_error(hip_status(e), "st_hist_create: %s", hipGetErrorString(e));
@@ -2024,15 +2047,15 @@ void st_hist_destroy(st_hist *h)
     if (!h) return;
     (void)queue_flush_producers(h);
     if (h->stream) (void)hipStreamSynchronize(h->stream);
-    (void)hipFree(h->edges_dev);
-    (void)hipFree(h->bins_dev);
-    (void)hipFree(h->keys_a);
-    (void)hipFree(h->keys_b);
-    (void)hipFree(h->vals_a);
-    (void)hipFree(h->vals_b);
-    (void)hipFree(h->os_status);
-    (void)hipFree(h->digit_counts);
-    (void)hipFree(h->os_ticket);
+    (void)dev_free(h->edges_dev);
+    (void)dev_free(h->bins_dev);
+    (void)dev_free(h->keys_a);
+    (void)dev_free(h->keys_b);
+    (void)dev_free(h->vals_a);
+    (void)dev_free(h->vals_b);
+    (void)dev_free(h->os_status);
+    (void)dev_free(h->digit_counts);
+    (void)dev_free(h->os_ticket);
     delete h;
 }
 

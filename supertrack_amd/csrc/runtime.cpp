@@ -1,14 +1,19 @@
 // runtime.cpp -- status strings, device memory helpers, geometry and bin
 // edges of libsupertrack_amd (host code).
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstring>
+#include <map>
 #include <mutex>
+#include <new>
+#include <unordered_map>
 #include <vector>
 
 #include "st_common.hpp"
 #include "st_internal.hpp"
+#include "transfer.hpp"
 
 namespace st {
 
@@ -43,22 +48,131 @@ bool injected_failure()
 }
 }  // namespace
 
-hipError_t dev_malloc(void **p, size_t bytes)
+namespace {
+// Device blocks given back and kept for the next taker of their size.  A track
+// or a small library makes and frees a handful of them; hipMalloc and hipFree
+// take 2-5 us each at 80 kB, but 150-220 us at 2-8 MB.  Blocks of up to
+// kPoolBlock are kept, kPoolBytes of them at most; a taker waits until the
+// device is done with what used the block before it was given back, as hipFree
+// would have.  An allocation that fails gives them all back and tries again.
+constexpr size_t kPoolBlock = (size_t)8 << 20, kPoolBytes = (size_t)16 << 20;
+struct Kept {
+    void *p;
+    uint64_t given;   // g_pool_clock when it was given back
+};
+std::mutex g_pool_mu;
+// (the maps are never destroyed: objects may be freed at exit)
+auto &g_pool = *new std::map<std::pair<int, size_t>, std::vector<Kept>>;          // (device, size)
+auto &g_pool_live = *new std::unordered_map<void *, std::pair<int, size_t>>;      // blocks handed out
+auto &g_pool_synced = *new std::map<int, uint64_t>;   // device: blocks given back before this are free of work
+size_t g_pool_bytes = 0;
+uint64_t g_pool_clock = 0;
+
+// Four sizes to an octave.
+size_t pool_size(size_t bytes)
 {
-    if (injected_failure()) {
-        *p = nullptr;
-        return hipErrorOutOfMemory;
-    }
-    return hipMalloc(p, bytes);
+    size_t step = 256;
+    while (bytes > step * 4) step *= 2;
+    return (bytes + step - 1) / step * step;
 }
 
-hipError_t pinned_malloc(void **p, size_t bytes, unsigned int flags)
+// All kept blocks back to the device (g_pool_mu held).
+void pool_trim()
 {
-    if (injected_failure()) {
-        *p = nullptr;
-        return hipErrorOutOfMemory;
+    for (auto &size : g_pool)
+        for (const Kept &k : size.second) (void)hipFree(k.p);
+    g_pool.clear();
+    g_pool_bytes = 0;
+}
+}  // namespace
+
+hipError_t dev_malloc(void **p, size_t bytes)
+{
+    *p = nullptr;
+    if (injected_failure()) return hipErrorOutOfMemory;
+    int dev = 0;
+    if (bytes == 0 || bytes > kPoolBlock || hipGetDevice(&dev) != hipSuccess) {
+        hipError_t e = hipMalloc(p, bytes);
+        if (e == hipErrorOutOfMemory) {
+            std::lock_guard<std::mutex> lock(g_pool_mu);
+            if (g_pool_bytes > 0) {
+                (void)hipGetLastError();
+                pool_trim();
+                e = hipMalloc(p, bytes);
+            }
+        }
+        return e;
     }
-    return hipHostMalloc(p, bytes, flags);
+    const size_t size = pool_size(bytes);
+    Kept got{nullptr, 0};
+    uint64_t now = 0;
+    bool clean = false;
+    {
+        std::lock_guard<std::mutex> lock(g_pool_mu);
+        auto it = g_pool.find({dev, size});
+        if (it != g_pool.end() && !it->second.empty()) {
+            got = it->second.back();
+            it->second.pop_back();
+            g_pool_bytes -= size;
+            now = ++g_pool_clock;
+            auto synced = g_pool_synced.find(dev);
+            clean = synced != g_pool_synced.end() && got.given < synced->second;
+        }
+    }
+    if (got.p && !clean) {
+        if (hipDeviceSynchronize() == hipSuccess) {
+            std::lock_guard<std::mutex> lock(g_pool_mu);
+            try {
+                uint64_t &synced = g_pool_synced[dev];
+                synced = std::max(synced, now);
+            } catch (const std::bad_alloc &) {   // (waited for again the next time)
+            }
+        } else {
+            // (under a capture, or after an error): a block of its own
+            (void)hipGetLastError();
+            (void)hipFree(got.p);
+            got.p = nullptr;
+        }
+    }
+    if (!got.p) {
+        hipError_t e = hipMalloc(&got.p, size);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            std::lock_guard<std::mutex> lock(g_pool_mu);
+            pool_trim();
+            e = hipMalloc(&got.p, size);
+        }
+        if (e != hipSuccess) return e;
+    }
+    try {
+        std::lock_guard<std::mutex> lock(g_pool_mu);
+        g_pool_live[got.p] = {dev, size};
+    } catch (const std::bad_alloc &) {   // no host memory to note it in: freed straight away later
+    }
+    *p = got.p;
+    return hipSuccess;
+}
+
+hipError_t dev_free(void *p)
+{
+    if (!p) return hipSuccess;
+    {
+        std::lock_guard<std::mutex> lock(g_pool_mu);
+        auto it = g_pool_live.find(p);
+        if (it != g_pool_live.end()) {
+            const std::pair<int, size_t> where = it->second;
+            g_pool_live.erase(it);
+            try {
+                if (g_pool_bytes + where.second <= kPoolBytes) {
+                    g_pool[where].push_back({p, ++g_pool_clock});
+                    g_pool_bytes += where.second;
+                    return hipSuccess;
+                }
+            } catch (const std::bad_alloc &) {
+            }
+        }
+    }
+    return hipFree(p);
 }
 
 namespace {
@@ -68,14 +182,17 @@ namespace {
 constexpr size_t kSlotBytes[] = {4096, 65536};
 constexpr size_t kKeptSlots = 8;
 std::mutex g_slot_mu;
-std::vector<void *> g_slots[2];
+struct SlotLists {
+    std::vector<void *> of[2];
+};
+auto &g_slots = (new SlotLists)->of;   // (never destroyed, as above)
 
 int slot_class(size_t bytes) { return bytes <= kSlotBytes[0] ? 0 : 1; }
 }  // namespace
 
-void *report_slot_take(size_t bytes)
+void *report_slot_take(size_t bytes, bool counted)
 {
-    if (bytes > kSlotBytes[1]) return nullptr;
+    if (bytes > kSlotBytes[1] || (counted && injected_failure())) return nullptr;
     const int c = slot_class(bytes);
     {
         std::lock_guard<std::mutex> lock(g_slot_mu);
@@ -86,8 +203,14 @@ void *report_slot_take(size_t bytes)
         }
     }
     void *p = nullptr;
-    if (hipHostMalloc(&p, kSlotBytes[c], hipHostMallocMapped | hipHostMallocPortable) != hipSuccess) {
+    void *mapped = nullptr;   // kernels store through the same address (unified addressing)
+    if (hipHostMalloc(&p, kSlotBytes[c], hipHostMallocMapped | hipHostMallocPortable | hipHostMallocCoherent) !=
+        hipSuccess) {
         (void)hipGetLastError();
+        return nullptr;
+    }
+    if (hipHostGetDevicePointer(&mapped, p, 0) != hipSuccess || mapped != p) {
+        (void)hipHostFree(p);
         return nullptr;
     }
     return p;
@@ -99,9 +222,12 @@ void report_slot_give(void *p, size_t bytes)
     const int c = slot_class(bytes);
     {
         std::lock_guard<std::mutex> lock(g_slot_mu);
-        if (g_slots[c].size() < kKeptSlots) {
-            g_slots[c].push_back(p);
-            return;
+        try {
+            if (g_slots[c].size() < kKeptSlots) {
+                g_slots[c].push_back(p);
+                return;
+            }
+        } catch (const std::bad_alloc &) {
         }
     }
     (void)hipHostFree(p);
@@ -212,7 +338,7 @@ int st_malloc(void **ptr, size_t bytes)
 
 int st_free(void *ptr)
 {
-    if (ptr) ST_HIP_TRY(hipFree(ptr));
+    if (ptr) ST_HIP_TRY(dev_free(ptr));
     return ST_OK;
 }
 
@@ -223,8 +349,8 @@ int st_memcpy_htod(void *dst, const void *src, size_t bytes)
 {
     if (!bytes) return ST_OK;
     ST_HIP_TRY(hipDeviceSynchronize());
-    ST_HIP_TRY(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice));
-    ST_HIP_TRY(hipDeviceSynchronize());
+    const UploadPart part{dst, src, bytes};
+    ST_HIP_TRY(upload(&part, 1));
     return ST_OK;
 }
 
@@ -232,7 +358,7 @@ int st_memcpy_dtoh(void *dst, const void *src, size_t bytes)
 {
     if (!bytes) return ST_OK;
     ST_HIP_TRY(hipDeviceSynchronize());
-    ST_HIP_TRY(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
+    ST_HIP_TRY(download(dst, src, bytes));
     return ST_OK;
 }
 
@@ -269,6 +395,11 @@ int st_debug_fail_allocation(int64_t countdown)
 
 int st_shutdown(void)
 {
+    staging_shutdown();
+    {
+        std::lock_guard<std::mutex> pool(g_pool_mu);
+        pool_trim();
+    }
     {
         std::lock_guard<std::mutex> slots(g_slot_mu);
         for (std::vector<void *> &kept : g_slots) {

@@ -30,11 +30,13 @@ void clear_error();
 // first use and kept for the life of the process.
 hipStream_t default_stream();
 
-// Every device and pinned-host allocation of the library goes through these,
-// so that st_debug_fail_allocation can make the n-th one fail (with
-// hipErrorOutOfMemory, as a full device would).
+// Every device allocation of the library goes through these, so that
+// st_debug_fail_allocation can make the n-th one fail (with
+// hipErrorOutOfMemory, as a full device would).  dev_free takes any device
+// pointer; small blocks are kept for the next dev_malloc, which waits for the
+// work that was queued before they were given back.
 hipError_t dev_malloc(void **p, size_t bytes);
-hipError_t pinned_malloc(void **p, size_t bytes, unsigned int flags);
+hipError_t dev_free(void *p);
 
 // Status for a failed HIP call: ST_ENOMEM for an allocation failure.
 inline int hip_status(hipError_t e)

@@ -13,7 +13,8 @@ namespace st {
 int device_cu_count();
 // Pinned, device-mapped host memory for up to 64 KiB that the device reports
 // into (null: none to be had); given back once no queued work writes to it.
-void *report_slot_take(size_t bytes);
+// counted: one of the allocations that st_debug_fail_allocation counts.
+void *report_slot_take(size_t bytes, bool counted = false);
 void report_slot_give(void *p, size_t bytes);
 void make_geometry(double half_length_ini, double diameter_ini, st_geometry *g);
 void make_edges(int type, float lo, float hi, int nbins, double *edges);
