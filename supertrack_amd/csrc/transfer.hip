@@ -33,9 +33,8 @@ constexpr size_t kLargeFrom = (size_t)2 << 20, kPerWorker = (size_t)8 << 20;
 constexpr size_t kSlot[2] = {(size_t)512 << 10, (size_t)8 << 20};   // bytes of a buffer (small, large)
 constexpr size_t kKeep[2] = {16, kMaxWorkers};                      // pairs of buffers kept (16 + 32 MiB)
 
-// A pair of buffers, filled and copied in turn.  The copies run on the null
-// stream, as hipMemcpy's do (a stream of their own costs 40 MB of device memory
-// for its queue).
+// A pair of buffers, filled and copied in turn on the null stream, as
+// hipMemcpy copies.
 struct Stage {
     int dev = 0, kind = 0;
     char *slot[2] = {nullptr, nullptr};
