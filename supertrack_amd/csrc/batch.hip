@@ -788,6 +788,12 @@ int st_library_append(st_library *L, const double *x, const double *y, const dou
         clear_error();
         ChunkLayout lay;
         fill_chunk(x, y, z, edep, offsets, n_tracks, L->geoms.data(), precision, pbase, bbase, nblocks, tds, lay);
+        if (precision == ST_F64)
+            for (int64_t t = 0; t < n_tracks; ++t) {
+                if (tds[t].flags & kFlagExact) continue;
+                double *e = lay.e.data() + (tds[t].offset - pbase);
+                for (int32_t p = 0; p < tds[t].n; ++p) e[p] = lineal_energy(e[p], L->geoms[tds[t].geom]);
+            }
         rc = dev_put(dst.x, lay.x.data(), n_points);
         if (!rc) rc = dev_put(dst.y, lay.y.data(), n_points);
         if (!rc) rc = dev_put(dst.z, lay.z.data(), n_points);

@@ -86,7 +86,8 @@ constexpr unsigned long long kBalanceMul = 0x9E3779B97F4A7C15ull;
 struct BatchArgs {
     // library
     const TrackDesc *tracks;
-    const double *x64, *y64, *z64, *e64;
+    const double *x64, *y64, *z64;
+    const double *e64;          // ST_F64, fast tracks: lineal energy; others: energy
     const float4 *p32;          // ST_F32: (dx, dy, dz, edep) per point
     const double *zfirst;
     const BlockF32 *blocks;
@@ -888,7 +889,7 @@ void batch_kernel(BatchArgs a)
                                                          a.z64[td.offset + ri], key);
                         }
                         if constexpr (MODE == ST_F64) {
-                            if (in) Acc<ST_F64>::split(cur[j].w / g.denom, v0, v1);
+                            if (in) Acc<ST_F64>::split(cur[j].w, v0, v1);
                         } else {
                             v0 = rint_to_i64((double)cur[j].w * g.yscale);
                         }

@@ -76,6 +76,16 @@ inline void sphere_thresholds(double r2q, double fm, double mrgq, double *sure, 
     *maybe = r2q + mrgq + 8.0 * (0.5 - fm);
 }
 
+// A deposit's lineal energy.  ST_F64 libraries hold it in place of the energy
+// for their fast-path tracks.
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+inline double lineal_energy(double edep, const st_geometry &g)
+{
+    return edep / ((2. / 3.) * g.diameter);
+}
+
 // One FP32 point: offsets from its block's origin (nm) and the energy (eV);
 // the same 16-byte layout as HIP's float4, which the kernel loads.
 struct PointF32 {

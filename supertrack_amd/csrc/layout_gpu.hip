@@ -508,6 +508,20 @@ __global__ __launch_bounds__(kThreads) void flags_kernel(TrackDesc *tds, const T
     tds[t].wave = fast && (passed & kTestWave) ? kFlagWave | ((passed & kTestHot) ? kFlagHot : 0u) : 0u;
 }
 
+// ST_F64: the fast-path tracks' energies become lineal energies (scored once
+// per oversample, where a division is a dozen instructions: 256 tracks x 100,
+// 10 nm spheres, 1.40 -> 1.34 ms).
+__global__ __launch_bounds__(kThreads) void lineal_kernel(const TrackDesc *tds, const int32_t *block_track, double *e,
+                                                          int64_t pbase, int64_t bbase, Geoms geoms)
+{
+    const int64_t b = blockIdx.x;
+    const TrackDesc &td = tds[block_track[b]];
+    const int64_t r = (b - (td.block0 - bbase)) * kBlk + threadIdx.x;
+    if ((td.flags & kFlagExact) || r >= td.n) return;
+    double &v = e[td.offset - pbase + r];
+    v = lineal_energy(v, geoms.g[td.geom]);
+}
+
 }  // namespace
 
 int layout_chunk_device(const double *x, const double *y, const double *z, const double *edep, int64_t n_points,
@@ -612,6 +626,8 @@ int layout_chunk_device(const double *x, const double *y, const double *z, const
     if (nblocks > 0)
         window_kernel<<<(unsigned)nblocks, kThreads, 0, stream>>>(tds_dev, bt, dst, pbase, bbase, gs, tests);
     flags_kernel<<<(unsigned)((n_tracks + kThreads - 1) / kThreads), kThreads, 0, stream>>>(tds_dev, tests, n_tracks);
+    if (precision == ST_F64 && nblocks > 0)
+        lineal_kernel<<<(unsigned)nblocks, kThreads, 0, stream>>>(tds_dev, bt, dst.e, pbase, bbase, gs);
     ST_HIP_TRY(hipGetLastError());
     ST_HIP_TRY(hipMemcpyAsync(tds, tds_dev, n_tracks * sizeof(TrackDesc), hipMemcpyDeviceToHost, stream));
     ST_HIP_TRY(hipStreamSynchronize(stream));

@@ -199,6 +199,7 @@ __device__ __forceinline__ unsigned mad24(unsigned a, unsigned b, unsigned c)
     return r;
 }
 
+// Slots are named by the byte offset of their key (four times their number).
 // Home slot: the low 24 bits of lx * a + ly * b + lz * c (a, b, c the R3
 // sequence's fractions in 2^24ths) scaled to the table size.
 // copy: kCopyHash times the entry's copy number (0 unless the track is hot).
@@ -207,7 +208,14 @@ template <int SLOTS>
 __device__ __forceinline__ unsigned lattice_slot(unsigned lx, unsigned ly, unsigned lz, unsigned copy)
 {
     const unsigned h = mad24(lx, 13743434u, mad24(ly, 11258244u, mad24(lz, 9222436u, copy)));
-    return (unsigned)(((unsigned long long)(h & 0xFFFFFFu) * (unsigned)(SLOTS << 8)) >> 32);
+    return (unsigned)(((unsigned long long)(h & 0xFFFFFFu) * (unsigned)(SLOTS << 10)) >> 32) & ~3u;
+}
+
+// The slot after (the last one wraps: the smaller of the two as unsigned numbers).
+template <int SLOTS>
+__device__ __forceinline__ unsigned lattice_next(unsigned slot)
+{
+    return min(slot + 4u, slot + 4u - 4u * (unsigned)SLOTS);
 }
 
 // First i in [0, n) with pred(i), else n, by one wave (n uniform, the answer
@@ -362,6 +370,10 @@ void wave_kernel(WaveArgs wa)
     unsigned long long *const tacc0 = reinterpret_cast<unsigned long long *>(mine);
     unsigned long long *const tacc1 = tacc0 + SLOTS;   // kWords == 2
     unsigned int *const tkey = reinterpret_cast<unsigned int *>(mine + SLOTS * 8 * kWords);
+    // a slot's key and sums
+    auto key_of = [&](unsigned slot) -> unsigned & { return *(unsigned *)((char *)tkey + slot); };
+    auto acc0_of = [&](unsigned slot) -> unsigned long long & { return *(unsigned long long *)((char *)tacc0 + 2u * slot); };
+    auto acc1_of = [&](unsigned slot) -> unsigned long long & { return *(unsigned long long *)((char *)tacc1 + 2u * slot); };
     unsigned short *const tlist = reinterpret_cast<unsigned short *>(mine + SLOTS * (8 * kWords + 4));
     unsigned int *const lhist = reinterpret_cast<unsigned int *>(smem + n_waves * wave_lds(kWords, SLOTS));
     WaveRare &rare = s_rare[wave];
@@ -606,7 +618,7 @@ void wave_kernel(WaveArgs wa)
                                            (k >> bits_x) & ((1u << (bits_xy - bits_x)) - 1u), k >> bits_xy,
                                            (k & ((1u << bits_c) - 1u)) * kCopyHash);
             };
-            const double invD = detach(g.invD), yscale = detach(MODE == ST_F64 ? g.denom : g.yscale);
+            const double invD = detach(g.invD), yscale = detach(g.yscale);   // (ST_F32)
             double bqx = rare.ox, bqy = rare.oy, bqz = rare.oz, sure = detach(g.sure), maybe = detach(g.maybe);
             const BlockF32 *blk = detach(a.blocks + td.block0);
             bool edge = false;   // the block's rows need the box and count tests
@@ -625,12 +637,8 @@ void wave_kernel(WaveArgs wa)
             // Scores the row at `row`, then flushes if the table is a quarter
             // full or the part ends; returns true at its end.  (Parts start at
             // a block's first row.)
-            auto step = [&](const PointT &p) __attribute__((always_inline)) -> bool {
-                // lattice units relative to the box corner (batch_kernel);
-                // decisions are kept as lane masks in scalar registers
-                const double qx = fma((double)p.x, invD, bqx);
-                const double qy = fma((double)p.y, invD, bqy);
-                const double qz = fma((double)p.z, invD, bqz);
+            auto step = [&](double qx, double qy, double qz, double w) __attribute__((always_inline)) -> bool {
+                // (decisions are kept as lane masks in scalar registers)
                 const double tx = qx + kRoundMagic, ty = qy + kRoundMagic, tz = qz + kRoundMagic;
                 const double ux = (tx - kRoundMagic) - qx, uy = (ty - kRoundMagic) - qy, uz = (tz - kRoundMagic) - qz;
                 const double distq = fma(ux, ux, fma(uy, uy, uz * uz));
@@ -664,17 +672,9 @@ void wave_kernel(WaveArgs wa)
                         if (in_xy && lz + 1u <= nz + 1u) {
                             // (batch_kernel's exact_local for bit-field keys: an
                             // index N is carried into the next one)
-                            double x, y, z;
-                            if constexpr (MODE == ST_F64) {
-                                x = p.x;
-                                y = p.y;
-                                z = p.z;
-                            } else {
-                                const uint64_t i8 = (uint64_t)(unsigned)(row + lane) * 8u;
-                                x = load_global<double>(rare.x, i8);
-                                y = load_global<double>(rare.y, i8);
-                                z = load_global<double>(rare.z, i8);
-                            }
+                            const uint64_t i8 = (uint64_t)(unsigned)(row + lane) * 8u;
+                            const double x = load_global<double>(rare.x, i8), y = load_global<double>(rare.y, i8),
+                                         z = load_global<double>(rare.z, i8);
                             unsigned gx, gy, gz;
                             if (exact_member(x, y, z, e, gx, gy, gz)) {
                                 if (gx >= e.N) {
@@ -706,25 +706,25 @@ void wave_kernel(WaveArgs wa)
                     unsigned long long v0, v1 = 0;
                     if constexpr (MODE == ST_F64) {
                         long long s0, s1;
-                        Acc<ST_F64>::split(p.w / yscale, s0, s1);   // (yscale: the denominator)
+                        Acc<ST_F64>::split(w, s0, s1);
                         v0 = (unsigned long long)s0;
                         v1 = (unsigned long long)s1;
                     } else {
-                        // rint(w * yscale) (the low word of the magic constant is zero)
-                        const double tw = (double)p.w * yscale + kRoundMagic;
+                        // rint of w (the low word of the magic constant is zero)
+                        const double tw = w + kRoundMagic;
                         v0 = ((unsigned long long)((unsigned)__double2hiint(tw) - 0x43380000u) << 32) |
                              (unsigned)__double2loint(tw);
                     }
-                    const unsigned key = (lz << bits_xy) | ((ly << bits_x) | ((lx << bits_c) | copy));
+                    const unsigned key = (lz << bits_xy) + ((ly << bits_x) + ((lx << bits_c) + copy));
                     h = lattice_slot<SLOTS>(lx, ly, lz, copy_hash);
-                    prev = atomicCAS(&tkey[h], kEmpty32, key);
+                    prev = atomicCAS(&key_of(h), kEmpty32, key);
 #pragma unroll 1
                     while (prev != kEmpty32 && prev != key) {
-                        h = next_slot<SLOTS>(h);
-                        prev = atomicCAS(&tkey[h], kEmpty32, key);
+                        h = lattice_next<SLOTS>(h);
+                        prev = atomicCAS(&key_of(h), kEmpty32, key);
                     }
-                    atomicAdd(&tacc0[h], v0);
-                    if (kWords == 2) atomicAdd(&tacc1[h], v1);
+                    atomicAdd(&acc0_of(h), v0);
+                    if (kWords == 2) atomicAdd(&acc1_of(h), v1);
                     bal_in += Acc<MODE>::balance(v0, v1);
                 }
                 asm("" : "+v"(prev));   // compared once, here
@@ -764,25 +764,25 @@ void wave_kernel(WaveArgs wa)
                         bool fresh = false;
                         unsigned h = 0;
                         if (lane < cnt - r) {
-                            const int sl = tlist[r + lane];
-                            const unsigned k = tkey[sl];
+                            const unsigned sl = tlist[r + lane];
+                            const unsigned k = key_of(sl);
                             if (k < bound && (k & (kHotCopies - 1u)) != 0u) {
                                 const unsigned k0 = k & ~(kHotCopies - 1u);
                                 h = home(k0);
-                                unsigned prev = atomicCAS(&tkey[h], kEmpty32, k0);
+                                unsigned prev = atomicCAS(&key_of(h), kEmpty32, k0);
 #pragma unroll 1
                                 while (prev != kEmpty32 && prev != k0) {
-                                    h = next_slot<SLOTS>(h);
-                                    prev = atomicCAS(&tkey[h], kEmpty32, k0);
+                                    h = lattice_next<SLOTS>(h);
+                                    prev = atomicCAS(&key_of(h), kEmpty32, k0);
                                 }
                                 fresh = prev == kEmpty32;
-                                atomicAdd(&tacc0[h], tacc0[sl]);
-                                tacc0[sl] = 0;
+                                atomicAdd(&acc0_of(h), acc0_of(sl));
+                                acc0_of(sl) = 0;
                                 if (kWords == 2) {
-                                    atomicAdd(&tacc1[h], tacc1[sl]);
-                                    tacc1[sl] = 0;
+                                    atomicAdd(&acc1_of(h), acc1_of(sl));
+                                    acc1_of(sl) = 0;
                                 }
-                                tkey[sl] = kMerged32;
+                                key_of(sl) = kMerged32;
                             }
                         }
                         const unsigned long long m = __ballot(fresh);
@@ -799,7 +799,7 @@ void wave_kernel(WaveArgs wa)
 #pragma unroll 1
                 for (int r = 0; r < n; r += 128) {
                     unsigned k[2];
-                    int sl[2];
+                    unsigned sl[2];
                     unsigned long long m_done[2], m_keep[2], v0[2] = {}, v1[2] = {};
                     double v[2];
 #pragma unroll
@@ -811,7 +811,7 @@ void wave_kernel(WaveArgs wa)
                     }
 #pragma unroll
                     for (int u = 0; u < 2; ++u)
-                        if (lane_of(m_keep[u])) k[u] = tkey[sl[u]];
+                        if (lane_of(m_keep[u])) k[u] = key_of(sl[u]);
 #pragma unroll
                     for (int u = 0; u < 2; ++u) {
                         m_done[u] = __ballot(k[u] < bound) & m_keep[u];
@@ -820,7 +820,7 @@ void wave_kernel(WaveArgs wa)
                             m_done[u] &= ~m_merged;
                             m_keep[u] &= ~m_merged;
                             n_retired += (unsigned)__popcll(m_merged);
-                            if (lane_of(m_merged)) tkey[sl[u]] = kEmpty32;
+                            if (lane_of(m_merged)) key_of(sl[u]) = kEmpty32;
                         }
                         m_keep[u] &= ~m_done[u];
                         n_retired += (unsigned)__popcll(m_done[u]);
@@ -828,12 +828,12 @@ void wave_kernel(WaveArgs wa)
                         if (lane_of(m_keep[u])) tlist[cnt + lanes_below(m_keep[u])] = (unsigned short)sl[u];
                         cnt += __popcll(m_keep[u]);
                         if (lane_of(m_done[u])) {
-                            v0[u] = tacc0[sl[u]];
-                            tkey[sl[u]] = kEmpty32;
-                            tacc0[sl[u]] = 0;
+                            v0[u] = acc0_of(sl[u]);
+                            key_of(sl[u]) = kEmpty32;
+                            acc0_of(sl[u]) = 0;
                             if (kWords == 2) {
-                                v1[u] = tacc1[sl[u]];
-                                tacc1[sl[u]] = 0;
+                                v1[u] = acc1_of(sl[u]);
+                                acc1_of(sl[u]) = 0;
                             }
                         }
                     }
@@ -876,21 +876,21 @@ void wave_kernel(WaveArgs wa)
                     // table, then enter it again
                     if (lane < cnt) {
                         const unsigned sl = tlist[lane];
-                        const unsigned k = tkey[sl];
+                        const unsigned k = key_of(sl);
                         unsigned to = home(k);
                         if (to != sl) {
-                            const unsigned long long v0 = tacc0[sl];
-                            tacc0[sl] = 0;
+                            const unsigned long long v0 = acc0_of(sl);
+                            acc0_of(sl) = 0;
                             unsigned long long v1 = 0;
                             if (kWords == 2) {
-                                v1 = tacc1[sl];
-                                tacc1[sl] = 0;
+                                v1 = acc1_of(sl);
+                                acc1_of(sl) = 0;
                             }
-                            tkey[sl] = kEmpty32;
+                            key_of(sl) = kEmpty32;
 #pragma unroll 1
-                            while (atomicCAS(&tkey[to], kEmpty32, k) != kEmpty32) to = next_slot<SLOTS>(to);
-                            tacc0[to] = v0;
-                            if (kWords == 2) tacc1[to] = v1;
+                            while (atomicCAS(&key_of(to), kEmpty32, k) != kEmpty32) to = lattice_next<SLOTS>(to);
+                            acc0_of(to) = v0;
+                            if (kWords == 2) acc1_of(to) = v1;
                             tlist[lane] = (unsigned short)to;
                         }
                     }
@@ -908,23 +908,23 @@ void wave_kernel(WaveArgs wa)
                         bool mv = false;
                         if (lane < cnt - r) {
                             const unsigned sl = tlist[r + lane];
-                            const unsigned k = tkey[sl];
+                            const unsigned k = key_of(sl);
                             unsigned to = home(k);
 #pragma unroll 1
                             while (to != sl) {
-                                if (atomicCAS(&tkey[to], kEmpty32, k) == kEmpty32) {
-                                    tacc0[to] = tacc0[sl];
-                                    tacc0[sl] = 0;
+                                if (atomicCAS(&key_of(to), kEmpty32, k) == kEmpty32) {
+                                    acc0_of(to) = acc0_of(sl);
+                                    acc0_of(sl) = 0;
                                     if (kWords == 2) {
-                                        tacc1[to] = tacc1[sl];
-                                        tacc1[sl] = 0;
+                                        acc1_of(to) = acc1_of(sl);
+                                        acc1_of(sl) = 0;
                                     }
-                                    tkey[sl] = kEmpty32;
+                                    key_of(sl) = kEmpty32;
                                     tlist[r + lane] = (unsigned short)to;
                                     mv = true;
                                     break;
                                 }
-                                to = next_slot<SLOTS>(to);
+                                to = lattice_next<SLOTS>(to);
                             }
                         }
                         moved |= __ballot(mv) != 0ull;
@@ -934,20 +934,23 @@ void wave_kernel(WaveArgs wa)
                 return false;
             };
             // the next row's points are loaded before the current ones are
-            // scored (moved out of the load's registers first, so that the
-            // wait is for the load issued a row ago)
+            // scored, but after these are in lattice units relative to the box
+            // corner (batch_kernel): the load's registers are free by then (2 nm
+            // spheres, 256 tracks x 1000: 11.76 -> 11.59 ms against moving them)
             PointT ahead;
             fetch(ahead);
             row -= 64;
             bool last = false;
 #pragma unroll 1
             while (!last) {
-                PointT p = ahead;
-                asm volatile("" : "+v"(p.x), "+v"(p.y), "+v"(p.z), "+v"(p.w));
-                fetch(ahead);
                 row += 64;
                 if ((row & (kBlk - 1)) == 0) new_block();
-                last = step(p);
+                double qx = fma((double)ahead.x, invD, bqx), qy = fma((double)ahead.y, invD, bqy),
+                       qz = fma((double)ahead.z, invD, bqz), w = (double)ahead.w;
+                if constexpr (MODE == ST_F32) w *= yscale;
+                asm volatile("" : "+v"(qx), "+v"(qy), "+v"(qz), "+v"(w));
+                fetch(ahead);
+                last = step(qx, qy, qz, w);
             }
             if (lane == 0) {
                 atomicAdd(&s_stats[2], (unsigned long long)n_in);
