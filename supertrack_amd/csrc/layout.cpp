@@ -196,12 +196,13 @@ void fill_chunk(const double *x, const double *y, const double *z, const double 
                 for (int a3 = 0; a3 < 3; ++a3) {
                     org[a3] = (std::isfinite(lo3[a3]) && std::isfinite(hi3[a3])) ? 0.5 * (lo3[a3] + hi3[a3]) : 0.0;
                 }
-                double err = 0.0;
+                double err = 0.0, extent = 0.0;
                 for (int64_t p = p0; p < p1; ++p) {
                     for (int a3 = 0; a3 < 3; ++a3) {
                         const double d = arr[a3][p] - org[a3];
                         const float f = (float)d;
                         (a3 == 0 ? out.p32[p].x : a3 == 1 ? out.p32[p].y : out.p32[p].z) = f;
+                        extent = std::max(extent, (double)std::fabs(f));
                         const double e1 = std::fabs((double)f - d) + std::fabs(d) * 2.3e-16;
                         if (std::isfinite(e1)) err = std::max(err, e1);
                         else err = HUGE_VAL;
@@ -225,6 +226,7 @@ void fill_chunk(const double *x, const double *y, const double *z, const double 
                 bk.fm = 0.5 - (dlq + 1e-12);
                 bk.mrgq = 3.0 * dlq * (1.0 + 2.0 * dlq) + 1e-14 * r2q;
                 sphere_thresholds(r2q, bk.fm, bk.mrgq, &bk.sure, &bk.maybe);
+                single_terms(bk, extent * invD, g);
             }
         }
     });

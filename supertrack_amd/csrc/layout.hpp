@@ -5,6 +5,7 @@
 // batch.hip to build the device library and by the CPU tests on its own.
 #pragma once
 
+#include <cmath>
 #include <cstdint>
 #include <vector>
 
@@ -40,7 +41,7 @@ struct TrackDesc {
     double xmin, xmax, ymin, ymax, zmax;
 };
 
-// ST_F32 block record (64 B, read through the scalar cache).  The fast path
+// ST_F32 block record (128 B, read through the scalar cache).  The fast path
 // works in lattice units: q = (coordinate - gso) / D, so rint(q) is the
 // sphere index and q - rint(q) the offset from the sphere centre; the voxel
 // faces are the half-way planes q = -1/2 and q = N - 1/2, so a point that is
@@ -55,9 +56,16 @@ struct TrackDesc {
 //           the squared distance;
 //   sure,   squared distances (lattice units) below which a point is inside
 //   maybe   its sphere and above which it is outside, whichever way a nearby
-//           half-way plane is decided (sphere_thresholds).
+//           half-way plane is decided (sphere_thresholds);
+//   k*, f*  oq* as its nearest integer and the rest, and
+//   *32     the thresholds for a point brought to lattice units in FP32
+//           (single_terms).
 struct BlockF32 {
     double oqx, oqy, oqz, dl, fm, mrgq, sure, maybe;
+    int32_t kx, ky, kz;
+    float fx, fy, fz;
+    float fm32, sure32, maybe32;
+    float pad[7];
 };
 
 // Squared-distance thresholds of a geometry (r2q = r^2 / D^2) from fm and mrgq
@@ -74,6 +82,44 @@ inline void sphere_thresholds(double r2q, double fm, double mrgq, double *sure, 
     const double f2 = fm > 0.0 ? fm * fm : 0.0;
     *sure = r2q - mrgq < f2 ? r2q - mrgq : f2;
     *maybe = r2q + mrgq + 8.0 * (0.5 - fm);
+}
+
+// The FP32 terms of a block record whose other terms are set.  extent: the
+// largest |FP32 offset| / D of the block.  A coordinate is then
+// fma(offset, 1 / D, f + f') lattice units from sphere k + k' (f', k': the same
+// of the segment's shift), off by at most dl / D, the rounding of 1 / D and of
+// the fma (2^-24 of extent, and of extent + 1) and of f, f' and their sum
+// (2^-24); the squared distance, at most 3/4, rounds three times.  Where the
+// bounds mean nothing every point is in doubt.
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+inline void single_terms(BlockF32 &bk, double extent, const st_geometry &g)
+{
+    const double ulp = 5.9604644775390625e-08;   // 2^-24
+    const double k[3] = {rint(bk.oqx), rint(bk.oqy), rint(bk.oqz)};
+    bk.kx = bk.ky = bk.kz = 0;
+    bk.fx = bk.fy = bk.fz = 0.0f;
+    bk.fm32 = bk.sure32 = -1.0f;
+    bk.maybe32 = HUGE_VALF;
+    for (float &v : bk.pad) v = 0.0f;
+    if (!(extent < 65536.0 && fabs(k[0]) < 1073741824.0 && fabs(k[1]) < 1073741824.0 && fabs(k[2]) < 1073741824.0))
+        return;
+    bk.kx = (int32_t)k[0];
+    bk.ky = (int32_t)k[1];
+    bk.kz = (int32_t)k[2];
+    bk.fx = (float)(bk.oqx - k[0]);
+    bk.fy = (float)(bk.oqy - k[1]);
+    bk.fz = (float)(bk.oqz - k[2]);
+    const double e = bk.dl / g.diameter + ulp * (2.0 * extent + 2.0) * (1.0 + 1e-6);
+    if (!(e < 0.25)) return;
+    const double fm = 0.5 - (e + 8.0 * ulp);   // (8 ulp: the rounding of the squares compared with fm^2)
+    double sure, maybe;
+    sphere_thresholds((g.radius * g.radius) / (g.diameter * g.diameter), fm, 3.0 * e * (1.0 + 2.0 * e) + 4.0 * ulp,
+                      &sure, &maybe);
+    bk.fm32 = (float)(fm - ulp);
+    bk.sure32 = (float)(sure - ulp);
+    bk.maybe32 = (float)(maybe + 2.0 * ulp);
 }
 
 // A deposit's lineal energy.  ST_F64 libraries hold it in place of the energy

@@ -291,7 +291,7 @@ __global__ __launch_bounds__(kThreads) void block_kernel(BlockArgs a)
     if (!a.dst.p32) return;
     // the block's FP32 record (fill_chunk's operations)
     const st_geometry g = a.geoms.g[td.geom];
-    double org[3], err = 0.0;
+    double org[3], err = 0.0, extent = 0.0;
     float f[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -299,10 +299,14 @@ __global__ __launch_bounds__(kThreads) void block_kernel(BlockArgs a)
         const double d = v[k] - org[k];
         f[k] = (float)d;
         const double e1 = fabs((double)f[k] - d) + fabs(d) * 2.3e-16;
-        if (act) err = isfinite(e1) ? fmax(err, e1) : HUGE_VAL;
+        if (act) {
+            err = isfinite(e1) ? fmax(err, e1) : HUGE_VAL;
+            extent = fmax(extent, (double)fabsf(f[k]));
+        }
     }
     if (act) a.dst.p32[p] = PointF32{f[0], f[1], f[2], (float)e};
     err = block_reduce(err, s, upper);
+    extent = block_reduce(extent, s, upper);
     if (tid != 0) return;
     const double invD = 1.0 / g.diameter;
     BlockF32 bk;
@@ -318,6 +322,7 @@ __global__ __launch_bounds__(kThreads) void block_kernel(BlockArgs a)
     bk.fm = 0.5 - (dlq + 1e-12);
     bk.mrgq = 3.0 * dlq * (1.0 + 2.0 * dlq) + 1e-14 * r2q;
     sphere_thresholds(r2q, bk.fm, bk.mrgq, &bk.sure, &bk.maybe);
+    single_terms(bk, extent * invD, g);
     a.dst.blocks[b] = bk;
 }
 

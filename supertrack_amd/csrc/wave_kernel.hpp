@@ -184,6 +184,8 @@ struct WaveRare {
     int64_t geom;              // the track's geometry
     int64_t seg;               // track * oversamples + oversample (recording)
     double ox, oy, oz;         // lattice-unit offsets that make the rounded coordinates local indices
+    float fx, fy, fz;          // ST_F32: the rest of ox.. beside its nearest integer,
+    int kx, ky, kz;            // and the integer
 };
 
 __device__ __forceinline__ bool lane_of(unsigned long long mask)
@@ -203,11 +205,16 @@ __device__ __forceinline__ unsigned mad24(unsigned a, unsigned b, unsigned c)
 // Home slot: the low 24 bits of lx * a + ly * b + lz * c (a, b, c the R3
 // sequence's fractions in 2^24ths) scaled to the table size.
 // copy: kCopyHash times the entry's copy number (0 unless the track is hot).
+constexpr unsigned kLatticeX = 13743434u, kLatticeY = 11258244u, kLatticeZ = 9222436u;
 constexpr unsigned kCopyHash = 7555035u;
+// Rounds an FP32 number below 2^22 to an integer when added: the low bits of
+// the sum are the integer, above them this number's.
+constexpr float kMagic32 = 12582912.0f;   // 1.5 * 2^23
+constexpr int kMagic32Bits = 0x4B400000;
 template <int SLOTS>
 __device__ __forceinline__ unsigned lattice_slot(unsigned lx, unsigned ly, unsigned lz, unsigned copy)
 {
-    const unsigned h = mad24(lx, 13743434u, mad24(ly, 11258244u, mad24(lz, 9222436u, copy)));
+    const unsigned h = mad24(lx, kLatticeX, mad24(ly, kLatticeY, mad24(lz, kLatticeZ, copy)));
     return (unsigned)(((unsigned long long)(h & 0xFFFFFFu) * (unsigned)(SLOTS << 10)) >> 32) & ~3u;
 }
 
@@ -259,6 +266,13 @@ __device__ __forceinline__ double detach(double v)
     return r;
 }
 
+__device__ __forceinline__ float detach(float v)
+{
+    float r;
+    asm("s_mov_b32 %0, %1" : "=s"(r) : "s"(v));
+    return r;
+}
+
 template <typename T>
 __device__ __forceinline__ const T *detach(const T *p)
 {
@@ -278,6 +292,7 @@ __device__ __forceinline__ T load_global(const void *base, uint64_t offset)
     return *(const __attribute__((address_space(1))) T *)((Bytes)base + offset);
 }
 typedef float Float4 __attribute__((ext_vector_type(4)));
+typedef double Double2 __attribute__((ext_vector_type(2), aligned(8)));
 
 // Acc<ST_F32>::value of a sum below 2^52 units: its bits under the exponent
 // whose unit is 2^-32, less that exponent's value.
@@ -301,22 +316,36 @@ __device__ __forceinline__ ArgsPtr args_here()
 __device__ __forceinline__ void bin_two(ArgsPtr args, int h, const double (&v)[2], const unsigned long long (&mask)[2],
                                         unsigned int *lhist)
 {
-    typedef const __attribute__((address_space(1))) double *GlobalPtr;
     const auto &hd = args->b.hist[h];
-    const int type = hd.guess.type;
-    const float top = (float)(hd.guess.nbins - 1);
-    const GlobalPtr edges = (GlobalPtr)hd.edges;
+    // what the common case needs of the histogram, in one wait (as the code
+    // came to need them they were five scalar waits and two rounds of edge
+    // loads: 2 nm spheres, 256 tracks x 1000, 11.21 -> 10.76 ms, with a branch
+    // in place of both conversions of the sums)
+    int type = hd.guess.type, nbins = hd.guess.nbins;
+    float log2_origin = hd.guess.log2_origin, log2_inv_width = hd.guess.log2_inv_width;
+    const double *edges = hd.edges;
+    int in_lds = args->b.hist_lds_words, lds_offset = hd.lds_offset;
+    asm volatile("" : "+s"(type), "+s"(nbins), "+s"(log2_origin), "+s"(log2_inv_width), "+s"(edges), "+s"(in_lds),
+                 "+s"(lds_offset));
+    // closed-form guesses, clamped into [0, nbins - 1]: always a valid load
+    float f[2];
+    if (type == ST_HIST_LIN) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) f[u] = (float)((v[u] - hd.guess.origin) * hd.guess.inv_width);
+    } else {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) f[u] = (__log2f((float)v[u]) - log2_origin) * log2_inv_width;
+    }
+    asm volatile("" : "+v"(f[0]), "+v"(f[1]));   // (one branch for both)
+    const float top = (float)(nbins - 1);
     int b[2];
     double lo[2], hi[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-        // closed-form guess, clamped into [0, nbins - 1]: always a valid load
-        float f;
-        if (type == ST_HIST_LIN) f = (float)((v[u] - hd.guess.origin) * hd.guess.inv_width);
-        else f = (__log2f((float)v[u]) - hd.guess.log2_origin) * hd.guess.log2_inv_width;
-        b[u] = (int)__builtin_amdgcn_fmed3f(f, 0.0f, top);
-        lo[u] = edges[(unsigned)b[u]];
-        hi[u] = edges[(unsigned)b[u] + 1u];
+        b[u] = (int)__builtin_amdgcn_fmed3f(f[u], 0.0f, top);
+        const Double2 pair = load_global<Double2>(edges, (unsigned)b[u] * 8u);
+        lo[u] = pair.x;
+        hi[u] = pair.y;
     }
     unsigned long long miss[2];
 #pragma unroll
@@ -342,7 +371,7 @@ __device__ __forceinline__ void bin_two(ArgsPtr args, int h, const double (&v)[2
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
         if (lane_of(mask[u]) && b[u] >= 0) {
-            if (args->b.hist_lds_words) atomicAdd(&lhist[hd.lds_offset + b[u]], 1u);
+            if (in_lds) atomicAdd(&lhist[lds_offset + b[u]], 1u);
             else atomicAdd(&hd.bins[b[u]], 1ull);
         }
     }
@@ -584,6 +613,15 @@ void wave_kernel(WaveArgs wa)
                     rare.ox = (MODE == ST_F64 ? sqx - g.qc : sqx) - (double)kx0;
                     rare.oy = (MODE == ST_F64 ? sqy - g.qc : sqy) - (double)ky0;
                     rare.oz = (MODE == ST_F64 ? (sqz + g.H * g.invD) - g.qc : sqz) - (double)k_first;
+                    if constexpr (MODE == ST_F32) {
+                        const double kx = rint(rare.ox), ky = rint(rare.oy), kz = rint(rare.oz);
+                        rare.kx = (int)kx;
+                        rare.ky = (int)ky;
+                        rare.kz = (int)kz;
+                        rare.fx = (float)(rare.ox - kx);
+                        rare.fy = (float)(rare.oy - ky);
+                        rare.fz = (float)(rare.oz - kz);
+                    }
                 }
                 wave_lds_fence();
             }
@@ -613,13 +651,29 @@ void wave_kernel(WaveArgs wa)
             const int flush_at = uniform_i32(bits_c ? kHotFlushAt : kFlushAt);
             static_assert(kHotCopies == 4, "two key bits");
             const unsigned copy = lane & ((1u << bits_c) - 1u), copy_hash = copy * kCopyHash;
+            // ST_F32: the rounded coordinates carry kMagic32's bits and count
+            // from the block's sphere; these make them local indices, and the
+            // key and the hash of what they carry are folded into the terms of
+            // the copy (all modulo 2^32, the hash modulo 2^24)
+            int cx = 0, cy = 0, cz = 0;
+            unsigned key0 = copy, hash0 = copy_hash;
             auto home = [&](unsigned k) {
                 return lattice_slot<SLOTS>((k >> bits_c) & ((1u << (bits_x - bits_c)) - 1u),
                                            (k >> bits_x) & ((1u << (bits_xy - bits_x)) - 1u), k >> bits_xy,
                                            (k & ((1u << bits_c) - 1u)) * kCopyHash);
             };
             const double invD = detach(g.invD), yscale = detach(g.yscale);   // (ST_F32)
-            double bqx = rare.ox, bqy = rare.oy, bqz = rare.oz, sure = detach(g.sure), maybe = detach(g.maybe);
+            using Real = typename std::conditional<MODE == ST_F64, double, float>::type;
+            constexpr Real kMagic = MODE == ST_F64 ? (Real)kRoundMagic : (Real)kMagic32;
+            Real bqx, bqy, bqz, sure, maybe;
+            const Real inv = MODE == ST_F64 ? (Real)invD : (Real)__int_as_float(uniform_i32(__float_as_int((float)invD)));
+            if constexpr (MODE == ST_F64) {
+                bqx = rare.ox;
+                bqy = rare.oy;
+                bqz = rare.oz;
+                sure = detach(g.sure);
+                maybe = detach(g.maybe);
+            }
             const BlockF32 *blk = detach(a.blocks + td.block0);
             bool edge = false;   // the block's rows need the box and count tests
             auto new_block = [&]() __attribute__((always_inline)) {
@@ -627,40 +681,82 @@ void wave_kernel(WaveArgs wa)
                 // block-uniform terms of the row's block (scalar loads)
                 if constexpr (MODE == ST_F32) {
                     const BlockF32 bk = load_uniform(blk + row / kBlk);
-                    bqx = bk.oqx + rare.ox;
-                    bqy = bk.oqy + rare.oy;
-                    bqz = bk.oqz + rare.oz;
-                    sure = detach(bk.sure);
-                    maybe = detach(bk.maybe);
+                    bqx = bk.fx + rare.fx;
+                    bqy = bk.fy + rare.fy;
+                    bqz = bk.fz + rare.fz;
+                    sure = detach(bk.sure32);
+                    maybe = detach(bk.maybe32);
+                    cx = bk.kx + uniform_i32(rare.kx) - kMagic32Bits;
+                    cy = bk.ky + uniform_i32(rare.ky) - kMagic32Bits;
+                    cz = bk.kz + uniform_i32(rare.kz) - kMagic32Bits;
+                    key0 = copy + (((unsigned)cx << bits_c) + ((unsigned)cy << bits_x) + ((unsigned)cz << bits_xy));
+                    hash0 = copy_hash + ((unsigned)cx * kLatticeX + (unsigned)cy * kLatticeY + (unsigned)cz * kLatticeZ);
                 }
             };
             // Scores the row at `row`, then flushes if the table is a quarter
             // full or the part ends; returns true at its end.  (Parts start at
             // a block's first row.)
-            auto step = [&](double qx, double qy, double qz, double w) __attribute__((always_inline)) -> bool {
-                // (decisions are kept as lane masks in scalar registers)
-                const double tx = qx + kRoundMagic, ty = qy + kRoundMagic, tz = qz + kRoundMagic;
-                const double ux = (tx - kRoundMagic) - qx, uy = (ty - kRoundMagic) - qy, uz = (tz - kRoundMagic) - qz;
-                const double distq = fma(ux, ux, fma(uy, uy, uz * uz));
-                unsigned lx = (unsigned)__double2loint(tx), ly = (unsigned)__double2loint(ty),
-                         lz = (unsigned)__double2loint(tz);
-                const int layer = (int)lz;
+            auto step = [&](Real qx, Real qy, Real qz, double w) __attribute__((always_inline)) -> bool {
+                // ST_F32: FP32 arithmetic, relative to a sphere near the block's
+                // origin so that its error stays below the block's own; rows
+                // with a point in doubt (0.9 % at 2 nm) go on to FP64.  19 FP64
+                // instructions of a row became FP32 ones, additions and
+                // products at nearly twice the rate: 256 tracks x 1000, 2 nm
+                // spheres, 11.59 -> 11.21 ms; x 100, 10 nm, 1.064 -> 1.040.
+                // (Decisions are kept as lane masks in scalar registers.)
+                const Real tx = qx + kMagic, ty = qy + kMagic, tz = qz + kMagic;
+                const Real ux = (tx - kMagic) - qx, uy = (ty - kMagic) - qy, uz = (tz - kMagic) - qz;
+                unsigned lx, ly, lz;   // local indices less cx, cy, cz
+                Real distq;
+                if constexpr (MODE == ST_F64) {
+                    distq = fma(ux, ux, fma(uy, uy, uz * uz));
+                    lx = (unsigned)__double2loint(tx);
+                    ly = (unsigned)__double2loint(ty);
+                    lz = (unsigned)__double2loint(tz);
+                } else {
+                    distq = fmaf(ux, ux, fmaf(uy, uy, uz * uz));
+                    lx = __float_as_uint(tx);
+                    ly = __float_as_uint(ty);
+                    lz = __float_as_uint(tz);
+                }
+                const int layer0 = (int)lz;
                 unsigned long long m_in = __ballot(distq < sure);
                 unsigned long long m_near = __ballot(distq <= maybe) & ~m_in;
                 if (edge) {
                     const int left = r_end - row;
                     const unsigned long long m_valid = left >= 64 ? ~0ull : (1ull << left) - 1ull;
-                    m_in &= m_valid & __ballot(lx < nx) & __ballot(ly < ny) & __ballot(lz < nz);
+                    m_in &= m_valid & __ballot(lx + (unsigned)cx < nx) & __ballot(ly + (unsigned)cy < ny) &
+                            __ballot(lz + (unsigned)cz < nz);
                     m_near &= m_valid;
                 }
                 if (m_near != 0ull) {
                     bool in = false;
                     if (lane_of(m_near)) {
+                        bool near = true;
+                        if constexpr (MODE == ST_F32) {
+                            // within the error bound of FP32 arithmetic: again
+                            // in FP64, from the FP32 offsets
+                            const Float4 p = load_global<Float4>(p0, (uint64_t)(unsigned)(row + lane) * 16u);
+                            const BlockF32 bk = load_uniform(blk + row / kBlk);
+                            const double qx = fma((double)p.x, invD, bk.oqx + rare.ox);
+                            const double qy = fma((double)p.y, invD, bk.oqy + rare.oy);
+                            const double qz = fma((double)p.z, invD, bk.oqz + rare.oz);
+                            const double tx = qx + kRoundMagic, ty = qy + kRoundMagic, tz = qz + kRoundMagic;
+                            const double ux = (tx - kRoundMagic) - qx, uy = (ty - kRoundMagic) - qy,
+                                         uz = (tz - kRoundMagic) - qz;
+                            const double distq = fma(ux, ux, fma(uy, uy, uz * uz));
+                            lx = (unsigned)__double2loint(tx);
+                            ly = (unsigned)__double2loint(ty);
+                            lz = (unsigned)__double2loint(tz);
+                            in = distq < bk.sure && lx < nx && ly < ny && lz < nz;
+                            near = distq <= bk.maybe && !(distq < bk.sure);
+                        }
+                        const int layer = (int)lz;
                         // any decision within the error bound is redone exactly
                         // from FP64, unless clearly outside (an index beyond the
                         // box by more than one)
                         const ExactParams &e = ex;
-                        const bool in_xy = lx + 1u <= nx + 1u && ly + 1u <= ny + 1u;
+                        const bool in_xy = near && lx + 1u <= nx + 1u && ly + 1u <= ny + 1u;
                         if constexpr (MODE == ST_F32) {
                             // (statistic: counted against the whole segment's
                             // box, by the part that holds the layer)
@@ -697,6 +793,9 @@ void wave_kernel(WaveArgs wa)
                                 in = lx < nx && ly < ny && lz < nz;
                             }
                         }
+                        lx -= (unsigned)cx;
+                        ly -= (unsigned)cy;
+                        lz -= (unsigned)cz;
                     }
                     m_in |= __ballot(in);
                 }
@@ -715,8 +814,8 @@ void wave_kernel(WaveArgs wa)
                         v0 = ((unsigned long long)((unsigned)__double2hiint(tw) - 0x43380000u) << 32) |
                              (unsigned)__double2loint(tw);
                     }
-                    const unsigned key = (lz << bits_xy) + ((ly << bits_x) + ((lx << bits_c) + copy));
-                    h = lattice_slot<SLOTS>(lx, ly, lz, copy_hash);
+                    const unsigned key = (lz << bits_xy) + ((ly << bits_x) + ((lx << bits_c) + key0));
+                    h = lattice_slot<SLOTS>(lx, ly, lz, hash0);
                     prev = atomicCAS(&key_of(h), kEmpty32, key);
 #pragma unroll 1
                     while (prev != kEmpty32 && prev != key) {
@@ -740,9 +839,9 @@ void wave_kernel(WaveArgs wa)
                 if (!last) {
                     // Every later point lies in a layer >= that of this row's
                     // last point; a key's layer is never below its point's.
-                    int lb = __builtin_amdgcn_readlane(layer, 63);
-                    double fm;
-                    if constexpr (MODE == ST_F32) fm = load_uniform(&blk[row / kBlk].fm);
+                    int lb = __builtin_amdgcn_readlane(layer0, 63) + cz;
+                    Real fm;
+                    if constexpr (MODE == ST_F32) fm = *(const __attribute__((address_space(4))) float *)(const void *)&blk[row / kBlk].fm32;
                     else fm = load_uniform(&args_here()->b.geoms[rare.geom].fm);
                     if (__ballot(fabs(uz) >= fm) >> 63) {
                         // rare: the exact layer, as the reference rounds it
@@ -843,8 +942,9 @@ void wave_kernel(WaveArgs wa)
                         if constexpr (MODE == ST_F32) v[u] = small_value(v0[u]);
                         else v[u] = Acc<MODE>::value(v0[u], v1[u]);
                     }
-                    if (MODE == ST_F32 && __ballot(((v0[0] | v0[1]) >> 52) != 0ull) != 0ull) {
+                    if (MODE == ST_F32 && __ballot(((unsigned)(v0[0] >> 32) | (unsigned)(v0[1] >> 32)) >= 1u << 20) != 0ull) {
                         // a sum of 2^20 or more, or a negative one
+                        asm volatile("");   // (a branch: not both forms and a select)
 #pragma unroll
                         for (int u = 0; u < 2; ++u) v[u] = Acc<MODE>::value(v0[u], v1[u]);
                     }
@@ -945,8 +1045,17 @@ void wave_kernel(WaveArgs wa)
             while (!last) {
                 row += 64;
                 if ((row & (kBlk - 1)) == 0) new_block();
-                double qx = fma((double)ahead.x, invD, bqx), qy = fma((double)ahead.y, invD, bqy),
-                       qz = fma((double)ahead.z, invD, bqz), w = (double)ahead.w;
+                Real qx, qy, qz;
+                double w = (double)ahead.w;
+                if constexpr (MODE == ST_F64) {
+                    qx = fma(ahead.x, inv, bqx);
+                    qy = fma(ahead.y, inv, bqy);
+                    qz = fma(ahead.z, inv, bqz);
+                } else {
+                    qx = fmaf(ahead.x, inv, bqx);
+                    qy = fmaf(ahead.y, inv, bqy);
+                    qz = fmaf(ahead.z, inv, bqz);
+                }
                 if constexpr (MODE == ST_F32) w *= yscale;
                 asm volatile("" : "+v"(qx), "+v"(qy), "+v"(qz), "+v"(w));
                 fetch(ahead);
