@@ -64,8 +64,8 @@ struct BlockF32 {
     double oqx, oqy, oqz, dl, fm, mrgq, sure, maybe;
     int32_t kx, ky, kz;
     float fx, fy, fz;
-    float fm32, sure32, maybe32;
-    float pad[7];
+    float sure32, maybe32;
+    float pad[8];
 };
 
 // Squared-distance thresholds of a geometry (r2q = r^2 / D^2) from fm and mrgq
@@ -100,7 +100,7 @@ inline void single_terms(BlockF32 &bk, double extent, const st_geometry &g)
     const double k[3] = {rint(bk.oqx), rint(bk.oqy), rint(bk.oqz)};
     bk.kx = bk.ky = bk.kz = 0;
     bk.fx = bk.fy = bk.fz = 0.0f;
-    bk.fm32 = bk.sure32 = -1.0f;
+    bk.sure32 = -1.0f;
     bk.maybe32 = HUGE_VALF;
     for (float &v : bk.pad) v = 0.0f;
     if (!(extent < 65536.0 && fabs(k[0]) < 1073741824.0 && fabs(k[1]) < 1073741824.0 && fabs(k[2]) < 1073741824.0))
@@ -117,7 +117,6 @@ inline void single_terms(BlockF32 &bk, double extent, const st_geometry &g)
     double sure, maybe;
     sphere_thresholds((g.radius * g.radius) / (g.diameter * g.diameter), fm, 3.0 * e * (1.0 + 2.0 * e) + 4.0 * ulp,
                       &sure, &maybe);
-    bk.fm32 = (float)(fm - ulp);
     bk.sure32 = (float)(sure - ulp);
     bk.maybe32 = (float)(maybe + 2.0 * ulp);
 }

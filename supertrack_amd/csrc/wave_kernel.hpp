@@ -181,7 +181,6 @@ constexpr int wave_lds(int words, int slots)
 struct WaveRare {
     ExactParams e;
     const double *x, *y, *z;   // the track's FP64 points
-    int64_t geom;              // the track's geometry
     int64_t seg;               // track * oversamples + oversample (recording)
     double ox, oy, oz;         // lattice-unit offsets that make the rounded coordinates local indices
     float fx, fy, fz;          // ST_F32: the rest of ox.. beside its nearest integer,
@@ -266,10 +265,19 @@ __device__ __forceinline__ double detach(double v)
     return r;
 }
 
-__device__ __forceinline__ float detach(float v)
+// The same value in every lane's vector registers (scalar ones are spilled
+// around the point loop and read back for each row).
+__device__ __forceinline__ float to_lanes(float v)
 {
     float r;
-    asm("s_mov_b32 %0, %1" : "=s"(r) : "s"(v));
+    asm("v_mov_b32 %0, %1" : "=v"(r) : "s"(v));
+    return r;
+}
+
+__device__ __forceinline__ double to_lanes(double v)
+{
+    double r;
+    asm("v_mov_b64 %0, %1" : "=v"(r) : "s"(v));
     return r;
 }
 
@@ -607,7 +615,6 @@ void wave_kernel(WaveArgs wa)
                     rare.x = a.x64 + td.offset;
                     rare.y = a.y64 + td.offset;
                     rare.z = a.z64 + td.offset;
-                    rare.geom = td.geom;
                     rare.seg = (int64_t)t * a.n_os + os;
                     const double sqx = sh.x * g.invD, sqy = sh.y * g.invD, sqz = sh.z * g.invD;
                     rare.ox = (MODE == ST_F64 ? sqx - g.qc : sqx) - (double)kx0;
@@ -671,8 +678,8 @@ void wave_kernel(WaveArgs wa)
                 bqx = rare.ox;
                 bqy = rare.oy;
                 bqz = rare.oz;
-                sure = detach(g.sure);
-                maybe = detach(g.maybe);
+                sure = to_lanes(g.sure);
+                maybe = to_lanes(g.maybe);
             }
             const BlockF32 *blk = detach(a.blocks + td.block0);
             bool edge = false;   // the block's rows need the box and count tests
@@ -684,8 +691,8 @@ void wave_kernel(WaveArgs wa)
                     bqx = bk.fx + rare.fx;
                     bqy = bk.fy + rare.fy;
                     bqz = bk.fz + rare.fz;
-                    sure = detach(bk.sure32);
-                    maybe = detach(bk.maybe32);
+                    sure = to_lanes(bk.sure32);
+                    maybe = to_lanes(bk.maybe32);
                     cx = bk.kx + uniform_i32(rare.kx) - kMagic32Bits;
                     cy = bk.ky + uniform_i32(rare.ky) - kMagic32Bits;
                     cz = bk.kz + uniform_i32(rare.kz) - kMagic32Bits;
@@ -839,11 +846,9 @@ void wave_kernel(WaveArgs wa)
                 if (!last) {
                     // Every later point lies in a layer >= that of this row's
                     // last point; a key's layer is never below its point's.
+                    // (its rounding is certain below fm, and sure <= fm^2)
                     int lb = __builtin_amdgcn_readlane(layer0, 63) + cz;
-                    Real fm;
-                    if constexpr (MODE == ST_F32) fm = *(const __attribute__((address_space(4))) float *)(const void *)&blk[row / kBlk].fm32;
-                    else fm = load_uniform(&args_here()->b.geoms[rare.geom].fm);
-                    if (__ballot(fabs(uz) >= fm) >> 63) {
+                    if (__ballot(!(uz * uz < sure)) >> 63) {
                         // rare: the exact layer, as the reference rounds it
                         const ExactParams &e = ex;
                         lb = uniform_i32((int)nearest_index(((load_global<double>(rare.z, (uint64_t)(unsigned)(row + 63) * 8u) + e.H) + e.sz) - e.gso, e.D, e.invD) -
@@ -891,7 +896,9 @@ void wave_kernel(WaveArgs wa)
                         wave_lds_fence();
                     }
                 }
-                if (cnt > kList && lane == 0) atomicOr(&args->b.ctl->error, 2);   // cannot happen (the bound above)
+                if (cnt > kList) {   // cannot happen (the bound above)
+                    if (lane == 0) atomicOr(&args->b.ctl->error, 2);
+                }
                 const int n = min(cnt, kList);
                 cnt = 0;
                 // two rows of 64 entries at a time: their LDS and edge loads overlap
