@@ -220,7 +220,8 @@ struct st_batch {
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
     // exact path
     std::vector<st_vcs *> methods;    // one per geometry
-    st_track scratch{};
+    double *exact_z = nullptr;                   // the exact track under way: its shifted z
+    int64_t exact_capacity = 0;
     st_pairs pairs{};
 };
 
@@ -330,7 +331,7 @@ int launch_pass(int precision, const BatchArgs &args, const Launch &ln, const Wa
         ST_HIP_TRY(hipLaunchKernel(k, dim3(ln.grid), dim3(kBT), kargs, ln.lds, stream));
     }
     if (wave && wave->plan.n_tracks > 0 && wave->slab) {
-        slab_sum_kernel<<<(wave->b.hist_lds_words + 63) / 64 + 1, 1024, 0, stream>>>(*wave, w.grid);
+        slab_sum_kernel<<<slab_blocks(wave->b.hist_lds_words), 1024, 0, stream>>>(*wave, w.grid);
         ST_HIP_TRY(hipGetLastError());
     }
     return ST_OK;
@@ -497,27 +498,31 @@ int run_exact(st_batch *b)
     for (int32_t t : L->exact) {
         const TrackDesc &td = L->tracks[t];
         const int64_t n = td.n;
-        if (n > b->scratch.capacity) {
-            st_track_free(&b->scratch);
-            int rc = st_track_alloc(&b->scratch, n);
-            if (rc) return rc;
+        if (n > b->exact_capacity) {
+            (void)dev_free(b->exact_z);
+            b->exact_z = nullptr;
+            b->exact_capacity = 0;
+            ST_ALLOC_TRY(dev_malloc((void **)&b->exact_z, (size_t)n * sizeof(double)));
+            b->exact_capacity = n;
         }
         if (n > b->pairs.capacity) {
             st_pairs_free(&b->pairs);
             int rc = st_pairs_alloc(&b->pairs, n);
             if (rc) return rc;
         }
-        const size_t bytes = (size_t)n * sizeof(double);
-        ST_HIP_TRY(hipMemcpyAsync(b->scratch.x, L->x64 + td.offset, bytes, hipMemcpyDeviceToDevice, b->stream));
-        ST_HIP_TRY(hipMemcpyAsync(b->scratch.y, L->y64 + td.offset, bytes, hipMemcpyDeviceToDevice, b->stream));
-        ST_HIP_TRY(hipMemcpyAsync(b->scratch.z, L->z64 + td.offset, bytes, hipMemcpyDeviceToDevice, b->stream));
-        ST_HIP_TRY(hipMemcpyAsync(b->scratch.edep, L->e64 + td.offset, bytes, hipMemcpyDeviceToDevice, b->stream));
-        b->scratch.n = n;
+        // the library's own arrays, but for the shifted z (copies of all four:
+        // 8 launches and 0.04 ms a pass over two such tracks)
+        st_track track{};
+        track.x = L->x64 + td.offset;
+        track.y = L->y64 + td.offset;
+        track.z = b->exact_z;
+        track.edep = L->e64 + td.offset;
+        track.n = track.capacity = n;
         st_pairs view = b->pairs;
         view.capacity = std::max<int64_t>(n, 1);
         st_vcs *m = b->methods[td.geom];
-        int rc = st_vcs_begin_track(m, &b->scratch, b->opts.seed, b->opts.track_index_base + (uint32_t)t,
-                                    b->opts.n_oversamples);
+        int rc = vcs_begin_track(m, &track, L->z64 + td.offset, b->opts.seed,
+                                 b->opts.track_index_base + (uint32_t)t, b->opts.n_oversamples);
         if (rc) return rc;
         // Tracks that the queued form takes run many oversamples in one launch,
         // a workgroup each (12e3 and 4e3 points x 20 oversamples: 0.60 ms in 80
@@ -525,7 +530,7 @@ int run_exact(st_batch *b)
         const int64_t kExactRows = (int64_t)64 << 20;
         const int group = (int)std::max<int64_t>(1, kExactRows / std::max<int64_t>(n * 16, 1));
         for (int os = 0; os < b->opts.n_oversamples; ++os) {
-            rc = st_vcs_process_oversample(m, &b->scratch, &view);
+            rc = st_vcs_process_oversample(m, &track, &view);
             if (rc) return rc;
             for (st_hist *h : b->hists) {
                 if (m->queue_track) queue_consume(m, h);
@@ -1249,7 +1254,7 @@ void st_batch_destroy(st_batch *b)
     for (hipEvent_t e : b->ev)
         if (e) (void)hipEventDestroy(e);
     report_slot_give(b->report, sizeof(CtlReport));
-    st_track_free(&b->scratch);
+    (void)dev_free(b->exact_z);
     st_pairs_free(&b->pairs);
     void *ptrs[] = {b->ctl, b->rec.seg, b->rec.key, b->rec.box, b->rec.sum, b->rec_dev};
     for (void *p : ptrs) (void)dev_free(p);

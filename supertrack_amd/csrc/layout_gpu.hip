@@ -27,8 +27,10 @@ namespace {
 
 constexpr int kMaxGeoms = 16;
 constexpr int kThreads = 256;
-constexpr int kRows = 8;
-constexpr int kTile = kThreads * kRows;
+// Rows of 256 keys a workgroup sorts: few of them where there are few tiles
+// (125e3 points: 62 tiles of 8 rows, 244 of 2).
+constexpr int kRowsMany = 8, kRowsFew = 2;
+constexpr int64_t kFewPoints = (int64_t)1 << 19;
 constexpr int kDigits = 256;
 
 struct Geoms {
@@ -110,8 +112,10 @@ __device__ __forceinline__ uint32_t digit_of(const SortArgs &a, unsigned long lo
     return a.key ? (uint32_t)(key >> a.shift) & 255u : (a.track[index] >> a.shift) & 255u;
 }
 
+template <int kRows>
 __global__ __launch_bounds__(kThreads) void sort_count_kernel(SortArgs a)
 {
+    constexpr int kTile = kThreads * kRows;
     __shared__ uint32_t s_c[kDigits];
     const int tid = threadIdx.x;
     s_c[tid] = 0;
@@ -155,8 +159,10 @@ __global__ __launch_bounds__(kThreads) void sort_scan_kernel(uint32_t *counts, u
     if (tid == 0) totals[blockIdx.x] = base;
 }
 
+template <int kRows>
 __global__ __launch_bounds__(kThreads) void sort_scatter_kernel(SortArgs a)
 {
+    constexpr int kTile = kThreads * kRows;
     __shared__ uint16_t s_cnt[kRows][kThreads / 64][kDigits];
     __shared__ uint32_t s_off[kDigits];
     __shared__ uint32_t s_w[kThreads / 64];
@@ -537,7 +543,9 @@ int layout_chunk_device(const double *x, const double *y, const double *z, const
         return set_error(ST_ENOMEM, "device layout: run of %lld points", (long long)n_points);
     hipStream_t stream = default_stream();
     const size_t n = (size_t)n_points;
-    const int tiles = (int)((n_points + kTile - 1) / kTile);
+    const bool few = n_points <= kFewPoints;
+    const int tile = kThreads * (few ? kRowsFew : kRowsMany);
+    const int tiles = (int)((n_points + tile - 1) / tile);
     size_t bytes = 0;
     auto add = [&](size_t b) {
         const size_t at = bytes;
@@ -593,9 +601,11 @@ int layout_chunk_device(const double *x, const double *y, const double *z, const
                                                                  (uint32_t *)a.track);
         auto pass = [&](int shift) {
             a.shift = shift;
-            sort_count_kernel<<<tiles, kThreads, 0, stream>>>(a);
+            if (few) sort_count_kernel<kRowsFew><<<tiles, kThreads, 0, stream>>>(a);
+            else sort_count_kernel<kRowsMany><<<tiles, kThreads, 0, stream>>>(a);
             sort_scan_kernel<<<kDigits, kThreads, 0, stream>>>(a.counts, a.totals, tiles);
-            sort_scatter_kernel<<<tiles, kThreads, 0, stream>>>(a);
+            if (few) sort_scatter_kernel<kRowsFew><<<tiles, kThreads, 0, stream>>>(a);
+            else sort_scatter_kernel<kRowsMany><<<tiles, kThreads, 0, stream>>>(a);
             const uint32_t *i = a.index;
             a.index = a.index_out;
             a.index_out = (uint32_t *)i;

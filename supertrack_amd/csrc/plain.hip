@@ -48,6 +48,7 @@ __device__ __forceinline__ double nearest_index(double a, double D, double invD)
 // once per track instead of once per oversample (the same IEEE value), and
 // GenerateRandomXYShift's shift table (:61-83) with Philox.
 struct SetupArgs {
+    const double *z_from;   // (may be z)
     double *z;
     const double *e;
     double *lin;
@@ -65,7 +66,7 @@ __global__ void track_setup_kernel(SetupArgs a)
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     const int64_t first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     for (int64_t i = first; i < a.n; i += stride) {
-        a.z[i] = a.z[i] + a.half_length;
+        a.z[i] = a.z_from[i] + a.half_length;
         a.lin[i] = a.e[i] / a.denominator;
     }
     for (int64_t k = first; k < a.n_os; k += stride) {
@@ -1717,6 +1718,16 @@ int st_vcs_set_queued(st_vcs *m, int32_t on)
 int st_vcs_begin_track(st_vcs *m, st_track *track, uint64_t seed, uint32_t track_index,
                        int32_t n_oversamples)
 {
+    return vcs_begin_track(m, track, nullptr, seed, track_index, n_oversamples);
+}
+
+}  // extern "C"
+
+namespace st {
+
+int vcs_begin_track(st_vcs *m, st_track *track, const double *z_from, uint64_t seed, uint32_t track_index,
+                    int32_t n_oversamples)
+{
     if (!m || !track) return set_error(ST_EINVAL, "st_vcs_begin_track: null argument");
     if (n_oversamples < 0) return set_error(ST_EINVAL, "st_vcs_begin_track: n_oversamples < 0");
     if (track->n < 0 || track->n > ((int64_t)1 << 31) - 1)
@@ -1744,6 +1755,7 @@ int st_vcs_begin_track(st_vcs *m, st_track *track, uint64_t seed, uint32_t track
     // the lineal energies and the shift table
     if (n > 0 || n_oversamples > 0) {
         SetupArgs sa;
+        sa.z_from = z_from ? z_from : track->z;
         sa.z = track->z;
         sa.e = track->edep;
         sa.lin = m->lineal;
@@ -1770,6 +1782,10 @@ int st_vcs_begin_track(st_vcs *m, st_track *track, uint64_t seed, uint32_t track
                      n * (int64_t)std::max(n_oversamples, 1) * 16 <= kQueueScratchBytes;
     return ST_OK;
 }
+
+}  // namespace st
+
+extern "C" {
 
 int st_vcs_process_oversample(st_vcs *m, const st_track *track, st_pairs *out)
 {

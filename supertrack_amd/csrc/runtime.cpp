@@ -55,7 +55,7 @@ namespace {
 // kPoolBlock are kept, kPoolBytes of them at most; a taker waits until the
 // device is done with what used the block before it was given back, as hipFree
 // would have.  An allocation that fails gives them all back and tries again.
-constexpr size_t kPoolBlock = (size_t)8 << 20, kPoolBytes = (size_t)16 << 20;
+constexpr size_t kPoolBlock = (size_t)16 << 20, kPoolBytes = (size_t)32 << 20;
 struct Kept {
     void *p;
     uint64_t given;   // g_pool_clock when it was given back

@@ -124,6 +124,10 @@ struct st_vcs {
 namespace st {
 // Runs the pending queued oversamples of m (no-op if none).
 int queue_flush(st_vcs *m);
+// st_vcs_begin_track with the track's z taken from z_from (null: its own) and,
+// shifted, written to it.
+int vcs_begin_track(st_vcs *m, st_track *track, const double *z_from, uint64_t seed, uint32_t track_index,
+                    int32_t n_oversamples);
 // Makes h a consumer of m's last queued oversample.
 void queue_consume(st_vcs *m, st_hist *h);
 }  // namespace st
