@@ -586,14 +586,18 @@ __global__ __launch_bounds__(kSortThreads) void hist_lds_kernel(HistArgs a)
 // radix sort's reduction read a sphere's run pair by pair from memory (60 ms
 // for 20 oversamples of 2e5 points in 100 nm spheres).
 //
-// A workgroup whose list would exceed kScanList splits its share over 16
-// hash values more, one after the other; a share that still does not fit holds
-// a few spheres with very many pairs each (a 100 nm sphere can take tens of
-// thousands), which are summed one by one in key order.
+// A workgroup whose list would exceed kScanList works through its share list by
+// list, each sphere's sum carried in the table (2e5 points in 100 nm spheres,
+// 78e3 pairs in 71 spheres, ten oversamples with the upload: 1.36 ms; 4.68 ms
+// when such a share was split over 16 more hash values, one after the other,
+// and 3.75 ms with the radix
+// sort).  Only a share of more spheres than the table holds is still split so;
+// one that then does not fit holds a few spheres with very many pairs each,
+// which are summed one by one in key order.
 constexpr int64_t kScanPairs = (int64_t)1 << 18;
 constexpr int kScanThreads = 1024;
 constexpr int kScanWaves = kScanThreads / 64;
-constexpr int kScanList = 1024;
+constexpr int kScanList = 960;
 constexpr int kScanTable = 2048;
 constexpr int kScanAhead = 8;    // rows of 64 pairs per wave read before the count is known
 constexpr int kScanRows = 28;    // rows of 64 keys per wave held in registers
@@ -639,6 +643,9 @@ __global__ __launch_bounds__(kScanThreads) void hist_scan_kernel(ScanArgs a)
     __shared__ uint32_t s_first[kScanTable], s_num[kScanTable];
     __shared__ uint32_t s_cnt[2][kScanWaves];
     __shared__ uint64_t s_min[kScanWaves];
+    // a long share's running sums; the last entry: the key of ~0
+    __shared__ double s_acc[kScanTable + 1];
+    __shared__ uint32_t s_used, s_last_first, s_last_num, s_last_seen;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint64_t lt_mask = (1ull << lane) - 1ull;
     const uint64_t *keys = a.h.keys;
@@ -701,6 +708,27 @@ __global__ __launch_bounds__(kScanThreads) void hist_scan_kernel(ScanArgs a)
         }
         off += (uint32_t)__popcll(mask);
     };
+    // acc and the listed pairs from j on of sphere k, of which there are `more`,
+    // left to right
+    auto add_from = [&](int j, int n, uint64_t k, uint32_t more, double acc) {
+        for (; more != 0u && j < n; j += 8) {
+            uint64_t kj[8];
+            double yj[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int jj = min(j + u, n - 1);
+                kj[u] = s_key[jj];
+                yj[u] = s_y[jj];
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const bool hit = j + u < n && kj[u] == k;
+                acc = acc + (hit ? yj[u] : -0.0);   // (x + -0.0 is x, whatever x is)
+                more -= hit ? 1u : 0u;
+            }
+        }
+        return acc;
+    };
     // Sums and bins the n listed pairs (the table is empty before and after).
     // A key of ~0 takes no table slot: it is told from the others by its list.
     auto reduce_list = [&](int n) {
@@ -734,25 +762,7 @@ __global__ __launch_bounds__(kScanThreads) void hist_scan_kernel(ScanArgs a)
             }
         }
         if (first) {
-            double acc = s_y[tid];
-            for (int j = tid + 1; more != 0u && j < n; j += 4) {
-                uint64_t kj[4];
-                double yj[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int jj = min(j + u, n - 1);
-                    kj[u] = s_key[jj];
-                    yj[u] = s_y[jj];
-                }
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    if (j + u < n && kj[u] == k) {
-                        acc = acc + yj[u];
-                        --more;
-                    }
-                }
-            }
-            scan_bin(a.h, acc);
+            scan_bin(a.h, add_from(tid + 1, n, k, more, s_y[tid]));
         }
     };
     auto clear_table = [&]() {
@@ -792,8 +802,8 @@ __global__ __launch_bounds__(kScanThreads) void hist_scan_kernel(ScanArgs a)
     };
 
     uint32_t total = 0, count = 0;
+    uint32_t sel = 0;   // this lane's selected rows
     if (AHEAD || per_wave <= 64 * kRows) {
-        uint32_t sel = 0;   // this lane's selected rows
         if constexpr (!AHEAD) {
 #pragma unroll
             for (int u = 0; u < kRows; ++u) {
@@ -830,6 +840,107 @@ __global__ __launch_bounds__(kScanThreads) void hist_scan_kernel(ScanArgs a)
         reduce_list((int)total);
         return;
     }
+    // A long share: in steps of some rows per wave, as many waves' pairs at
+    // a time as the list holds, each sphere's sum carried in the table from list
+    // to list (pairs stay in order).  False: the table may not hold its spheres
+    // (nothing has been counted).
+    auto stream = [&]() -> bool {
+        constexpr int kScanStep = AHEAD ? kScanAhead : 14;   // rows of 64 keys per wave and step
+        static_assert(kScanStep * 64 <= kScanList, "a wave's pairs of one step fit the list");
+        if (tid == 0) {
+            s_used = 0;
+            s_last_seen = 0;
+            s_last_first = ~0u;
+            s_last_num = 0;
+        }
+        __syncthreads();
+#pragma unroll 1
+        for (int base = 0; base < m; base += kScanWaves * 64 * kScanStep) {
+            const int lo = base + wave * 64 * kScanStep + lane;
+            uint64_t kq[AHEAD ? 1 : kScanStep];
+            uint32_t cnt = 0, all = 0;
+            if constexpr (AHEAD) {   // one step: the keys read ahead
+                cnt = count;
+            } else {
+                sel = 0;
+#pragma unroll
+                for (int u = 0; u < kScanStep; ++u) kq[u] = lo + u * 64 < m ? keys[lo + u * 64] : 0;
+#pragma unroll
+                for (int u = 0; u < kScanStep; ++u) {
+                    const bool s = lo + u * 64 < m && mine(kq[u]);
+                    sel |= s ? 1u << u : 0u;
+                    cnt += (uint32_t)__popcll(__ballot(s));
+                }
+            }
+            const int counts = half;
+            const uint32_t off = offsets(cnt, all);
+            for (uint32_t r0 = 0; r0 < all;) {
+                uint32_t end = r0, before = 0;
+#pragma unroll
+                for (int w = 0; w < kScanWaves; ++w) {
+                    before += s_cnt[counts][w];
+                    if (before <= r0 + (uint32_t)kScanList) end = max(end, before);
+                }
+                const int n = (int)(end - r0);
+                if (s_used + (uint32_t)n > (uint32_t)kScanTable) return false;
+                if (cnt != 0u && off >= r0 && off + cnt <= end) {
+                    uint32_t pos = off - r0;
+#pragma unroll
+                    for (int u = 0; u < kScanStep; ++u) {
+                        const bool s = (sel >> u) & 1u;
+                        const uint64_t mask = __ballot(s);
+                        if (mask == 0ull) continue;
+                        if constexpr (AHEAD) put(mask, s, pos, q[u], yr[u]);
+                        else put(mask, s, pos, kq[u], s ? y[lo + u * 64] : 0.0);
+                    }
+                }
+                __syncthreads();
+                uint64_t k = 0;
+                uint32_t *first_of = &s_last_first, *num_of = &s_last_num;
+                double *acc_of = &s_acc[kScanTable];
+                if (tid < n) {
+                    k = s_key[tid];
+                    if (k != ~0ull) {
+                        uint32_t slot = (uint32_t)(hash(k) >> 20) & (kScanTable - 1);
+                        while (true) {
+                            const unsigned long long prev = atomicCAS(&s_tkey[slot], ~0ull, (unsigned long long)k);
+                            if (prev == ~0ull) {
+                                s_acc[slot] = -0.0;   // -0.0 + y is y, whatever y is
+                                atomicAdd(&s_used, 1u);
+                            }
+                            if (prev == ~0ull || prev == k) break;
+                            slot = (slot + 1) & (kScanTable - 1);
+                        }
+                        first_of = &s_first[slot];
+                        num_of = &s_num[slot];
+                        acc_of = &s_acc[slot];
+                    } else if (atomicExch(&s_last_seen, 1u) == 0u) {
+                        *acc_of = -0.0;
+                    }
+                    atomicMin(first_of, (uint32_t)tid);
+                    atomicAdd(num_of, 1u);
+                }
+                __syncthreads();
+                const bool first = tid < n && *first_of == (uint32_t)tid;
+                if (first) {
+                    *acc_of = add_from(tid, n, k, *num_of, *acc_of);
+                }
+                __syncthreads();
+                if (first) {
+                    *first_of = ~0u;
+                    *num_of = 0;
+                }
+                __syncthreads();
+                r0 = end;
+            }
+        }
+        for (int s = tid; s < kScanTable; s += kScanThreads)
+            if (s_tkey[s] != ~0ull) scan_bin(a.h, s_acc[s]);
+        if (tid == 0 && s_last_seen) scan_bin(a.h, s_acc[kScanTable]);
+        return true;
+    };
+    if (stream()) return;
+    clear_table();
     for (uint32_t sub = 0; sub < 16; ++sub) {
         const uint32_t want = part * 16 + sub;
         auto match = [&](uint64_t h) { return (uint32_t)(h >> (60 - bits)) == want; };

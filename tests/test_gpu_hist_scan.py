@@ -57,3 +57,18 @@ def test_scan_few_spheres_with_many_pairs(m, capacity):
     keys[rng.random(m) < 0.3] = 123456789
     keys[::50] = np.uint64(0xFFFFFFFFFFFFFFFF)
     _check(keys, ys, capacity)
+
+
+@pytest.mark.parametrize("m,capacity", [(8192, 8192), (14336, 30000), (14337, 30000), (90000, 1 << 18)])
+@pytest.mark.parametrize("spheres", [3, 40, 500])
+def test_scan_sums_carried_from_list_to_list(m, capacity, spheres):
+    """Shares of many lists: spheres that come back in every list and ones that
+    leave, of very uneven sizes."""
+    rng = np.random.default_rng(m + spheres)
+    which = (rng.random(m) ** 4 * spheres).astype(np.int64)
+    which = (which + np.arange(m) * spheres // (2 * m)) % spheres
+    names = rng.integers(0, 1 << 40, spheres).astype(np.uint64)
+    names[0] = np.uint64(0xFFFFFFFFFFFFFFFF)
+    ys = rng.lognormal(-6.0, 3.0, m)
+    ys[::97] = -ys[::97]
+    _check(names[which], ys, capacity)
