@@ -54,7 +54,8 @@ namespace {
 // take 2-5 us each at 80 kB, but 150-220 us at 2-8 MB.  Blocks of up to
 // kPoolBlock are kept, kPoolBytes of them at most; a taker waits until the
 // device is done with what used the block before it was given back, as hipFree
-// would have.  An allocation that fails gives them all back and tries again.
+// would have.  A block given back to a full pool takes the place of those kept
+// longest; an allocation that fails gives all of them back and tries again.
 constexpr size_t kPoolBlock = (size_t)16 << 20, kPoolBytes = (size_t)32 << 20;
 struct Kept {
     void *p;
@@ -156,6 +157,8 @@ hipError_t dev_malloc(void **p, size_t bytes)
 hipError_t dev_free(void *p)
 {
     if (!p) return hipSuccess;
+    std::vector<void *> evicted;   // the blocks kept longest make room
+    bool kept = false;
     {
         std::lock_guard<std::mutex> lock(g_pool_mu);
         auto it = g_pool_live.find(p);
@@ -163,15 +166,28 @@ hipError_t dev_free(void *p)
             const std::pair<int, size_t> where = it->second;
             g_pool_live.erase(it);
             try {
+                while (g_pool_bytes + where.second > kPoolBytes) {
+                    auto oldest = g_pool.end();
+                    for (auto k = g_pool.begin(); k != g_pool.end(); ++k)
+                        if (!k->second.empty() &&
+                            (oldest == g_pool.end() || k->second.front().given < oldest->second.front().given))
+                            oldest = k;
+                    if (oldest == g_pool.end()) break;
+                    evicted.push_back(oldest->second.front().p);
+                    oldest->second.erase(oldest->second.begin());
+                    g_pool_bytes -= oldest->first.second;
+                }
                 if (g_pool_bytes + where.second <= kPoolBytes) {
                     g_pool[where].push_back({p, ++g_pool_clock});
                     g_pool_bytes += where.second;
-                    return hipSuccess;
+                    kept = true;
                 }
             } catch (const std::bad_alloc &) {
             }
         }
     }
+    for (void *old : evicted) (void)hipFree(old);
+    if (kept) return hipSuccess;
     return hipFree(p);
 }
 
