@@ -1,5 +1,5 @@
 // batch.hip -- the batched form of the VoxelConstrainedSphere path: a resident
-// track library and one persistent fused kernel that scores every
+// track library and persistent fused kernels that score every
 // (track, oversample) segment: shift -> voxel -> sphere -> key -> per-sphere
 // sum -> lineal energy -> bin.
 //
@@ -7,15 +7,19 @@
 //   * each track's points sorted by z (a rigid shift keeps that order, so for
 //     any oversample the points inside the voxel in z form one contiguous run
 //     and the sphere layer index iz never decreases along the run);
-//   * FP64 SoA x, y, z, edep in that order (the data in ST_F64 mode, the exact
-//     side copy in ST_F32 mode);
+//   * FP64 SoA x, y, z, edep in that order (the data in ST_F64 mode, where
+//     fast-path tracks hold lineal energies in place of edep; the exact side
+//     copy in ST_F32 mode);
 //   * ST_F32 mode: FP32 (dx, dy, dz, edep) per point, coordinates relative to a
 //     per-256-point block origin (FP64) and a per-block bound on the FP32
 //     rounding error;
 //   * per block: z of its first point (the search index); per track: offsets,
 //     x/y bounds, geometry, eligibility.
 //
-// The fused kernel itself is in batch_kernel.hpp; this file holds the
+// The fused kernels are in wave_kernel.hpp (the default: one wavefront per
+// segment) and batch_kernel.hpp (one workgroup per segment: tracks whose
+// flushes keep too much for a wave's table, and launch shapes that the caller
+// names); the layout runs on the device (layout_gpu.hip).  This file holds the
 // library construction, launch shapes, autotuner, exact path and the C ABI.
 // Tracks whose densest z-window two diameters wide could touch more spheres
 // than a flush may keep (768), with non-finite data, beyond the fixed-point

@@ -590,10 +590,9 @@ __global__ __launch_bounds__(kSortThreads) void hist_lds_kernel(HistArgs a)
 // list, each sphere's sum carried in the table (2e5 points in 100 nm spheres,
 // 78e3 pairs in 71 spheres, ten oversamples with the upload: 1.36 ms; 4.68 ms
 // when such a share was split over 16 more hash values, one after the other,
-// and 3.75 ms with the radix
-// sort).  Only a share of more spheres than the table holds is still split so;
-// one that then does not fit holds a few spheres with very many pairs each,
-// which are summed one by one in key order.
+// and 3.75 ms with the radix sort).  Only a share of more spheres than the
+// table holds is still split so; one that then does not fit holds a few spheres
+// with very many pairs each, which are summed one by one in key order.
 constexpr int64_t kScanPairs = (int64_t)1 << 18;
 constexpr int kScanThreads = 1024;
 constexpr int kScanWaves = kScanThreads / 64;

@@ -2,9 +2,10 @@
 // only): one wavefront scores a (track, oversample) segment, or a part of one,
 // on its own, with its own sphere table in LDS.
 //
-// What bounds it: instruction issue.  A scored point costs about two
-// microseconds of one lane whatever its bytes (points are re-read from L2 by
-// the track's other oversamples), so the layout below is chosen to leave out
+// What bounds it: instruction issue (256 tracks, 2 nm spheres, x 1000: about 85
+// vector and 80 scalar instructions per row of 64 points, vector units busy
+// 0.8 of the time), whatever a point's bytes (points are re-read from L2 by the
+// track's other oversamples), so the layout below is chosen to leave out
 // instructions and waits, not bytes:
 //   * no workgroup barrier between the start and the end of the kernel: the
 //     occupancy check of the table is a scalar compare, a flush runs on 64
@@ -86,7 +87,7 @@ __host__ __device__ inline int64_t track_chunks(int n, int n_os, int chunk_point
 // Builds the queues.  A chunk holds a fixed share of the points still to come
 // in the order (largest tracks first), at least min_points: large chunks while
 // much is left, small ones at the end, so that the last wave to finish is not
-// late.  Fixed chunks, 24 per wave: 6.8 ms on a mixed library of 96 tracks x
+// late.  As first written: fixed chunks, 24 per wave: 6.8 ms on a mixed library of 96 tracks x
 // 1000 oversamples and 1.11 ms on 256 tracks x 100; 48 per wave: 6.2 and 1.28
 // ms; this: 5.9 and 1.06 ms.
 __global__ __launch_bounds__(64 * kQueues) void wave_plan_kernel(const TrackDesc *tracks, const int32_t *order,
@@ -154,8 +155,9 @@ __device__ __forceinline__ int lanes_below(unsigned long long mask)
 
 // Table slots of a wave, flush threshold and list capacity.  A flush at a
 // quarter full keeps the probe chains short, and its entries then mostly fill
-// the two rows of 64 that it handles together (256 tracks, 2 nm spheres: 320
-// slots 14.1 ms, 384 13.8, 416 13.6, 432 13.9); the list holds what a flush
+// the two rows of 64 that it handles together (256 tracks x 1000, 2 nm spheres,
+// as first written: 320 slots 14.1 ms, 384 13.8, 416 13.6, 432 13.9; 416 slots
+// now: a flush at 88 entries 11.3 ms, 104 10.8, 120 11.6); the list holds what a flush
 // keeps (at most kWaveWindow, or fewer than the threshold) and one row of 64
 // points.
 constexpr int kWaveSlots = 416;
