@@ -296,19 +296,21 @@ WaveArgs make_wave_args(const st_library *L, const st_batch_opts &o, st_hist *co
     return wa;
 }
 
-// Queues the kernel that fills a plan: chunks of a tenth of a wave's share of
+// Queues the kernel that fills a plan: chunks of a seventh of a wave's share of
 // the work left, but at least an even share of all of it between 2048 and
 // 12288 points (a chunk's set-up, about five rows of 64 points, then stays
-// small beside the tenth of its points that is scored).  1/8 to 1/12 and 12288
-// to 24576 points measured within 3 % of each other, 1/24 and 6144 points 9 %
-// slower.
+// small beside the tenth of its points that is scored).  Short passes like
+// larger chunks, long ones smaller (ms a pass, ST_F32, 256 tracks: 10 nm x 100,
+// 1 nm x 100, 2 nm x 1000): 1/10 1.005, 0.865, 10.34; 1/7 0.971, 0.820, 10.34;
+// 1/5 0.953, 0.785, 10.59.  At least 6144 points 1.070 and 10.54 (1/10), 16384
+// 0.972 and 10.27 (1/8), but 5 tracks x 200 then take 0.245 instead of 0.201.
 int launch_plan(const st_library *L, int n_os, const WaveLaunch &w, PlanTrack *plan, hipStream_t stream)
 {
     const double waves = (double)w.grid * w.wg_waves;
     const double even = (double)L->wave_points * n_os / waves;
     const int min_points = (int)std::min(std::max(even, 2048.0), 12288.0);
     wave_plan_kernel<<<1, 64 * kQueues, 0, stream>>>(L->tracks_dev, L->wave_order_dev, (int32_t)L->wave_order.size(),
-                                                     n_os, L->wave_points, n_os / (waves * 10.0), min_points,
+                                                     n_os, L->wave_points, n_os / (waves * 7.0), min_points,
                                                      plan_stride(L), plan, plan_totals(L, plan));
     ST_HIP_TRY(hipGetLastError());
     return ST_OK;
