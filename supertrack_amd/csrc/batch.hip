@@ -217,6 +217,10 @@ struct st_batch {
     BatchCtl *ctl = nullptr;   // per-pass control block (device); the plan and slabs follow it
     RecArgs rec{};                // recording buffers (cap 0: off)
     RecArgs *rec_dev = nullptr;   // their descriptor in device memory
+    bool planned = false;      // wave_plan has been queued (before the first pass, on its stream)
+    bool ran = false;          // ctl (and report) hold a pass's outcome
+    bool in_flight = false;    // a pass may still be running,
+    hipEvent_t end = nullptr;  // until this event (one of ev; null: unknown)
     bool graph_ready = false;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -343,9 +347,25 @@ int launch_pass(int precision, const BatchArgs &args, const Launch &ln, const Wa
     return ST_OK;
 }
 
+// Queues what a batch's first pass needs on its stream.  (Not when the batch is
+// made: another pass may be under way on the default stream, and a batch moved
+// to its own stream neither waits for it nor may overtake what it left there.)
+int prepare_passes(st_batch *b)
+{
+    if (!b->wave.on || b->planned) return ST_OK;
+    int rc = launch_plan(b->lib, b->opts.n_oversamples, b->wave, b->wave_plan, b->stream);
+    if (rc) return rc;
+    // (under a capture it was only recorded: the next pass asks again)
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    ST_HIP_TRY(hipStreamIsCapturing(b->stream, &capture));
+    b->planned = capture == hipStreamCaptureStatusNone;
+    return ST_OK;
+}
+
 int launch_fast(st_batch *b)
 {
     const st_library *L = b->lib;
+    b->ran = true;
     BatchArgs a = make_args(L, b->opts, b->hists.data(), (int)b->hists.size(), b->ln, b->ctl, b->wave.on);
     a.rec = b->rec.cap > 0 ? b->rec_dev : nullptr;
     if (!b->wave.on) return launch_pass(L->precision, a, b->ln, nullptr, b->wave, b->stream);
@@ -583,10 +603,12 @@ int autotune(st_batch *b)
     const int cand_copies[] = {1, 2, 4};
     float best = 1e30f;
     const WaveLaunch wave = b->wave;
+    int rc = prepare_passes(b);
+    if (rc) return rc;
     if (wave.on) {
         for (int k = 0; k < 2; ++k) {
             ST_HIP_TRY(hipEventRecord(ev.e[0], b->stream));
-            int rc = launch_fast(b);
+            rc = launch_fast(b);
             if (rc) return rc;
             ST_HIP_TRY(hipEventRecord(ev.e[1], b->stream));
             ST_HIP_TRY(hipEventSynchronize(ev.e[1]));
@@ -606,7 +628,7 @@ int autotune(st_batch *b)
                 if (configure(b, s, bp, pp, cp) != ST_OK) continue;
                 if (b->ln.blocks_per_cu != bp) continue;
                 ST_HIP_TRY(hipEventRecord(ev.e[0], b->stream));
-                int rc = launch_fast(b);
+                rc = launch_fast(b);
                 if (rc) return rc;
                 ST_HIP_TRY(hipEventRecord(ev.e[1], b->stream));
                 ST_HIP_TRY(hipEventSynchronize(ev.e[1]));
@@ -682,11 +704,16 @@ int read_ctl(const BatchCtl *ctl, hipStream_t stream, CtlReport *out)
 }
 
 // The same for a batch: a pass of the one-wave kernel has already reported.
-int read_report(const st_batch *b, CtlReport *out)
+int read_report(st_batch *b, CtlReport *out)
 {
-    if (!b->wave.on || !b->report) return read_ctl(b->ctl, b->stream, out);
-    ST_HIP_TRY(hipStreamSynchronize(b->stream));
-    *out = *b->report;
+    if (b->ran && (!b->wave.on || !b->report)) {
+        int rc = read_ctl(b->ctl, b->stream, out);
+        if (rc) return rc;
+    } else {
+        ST_HIP_TRY(hipStreamSynchronize(b->stream));
+        *out = b->ran ? *b->report : CtlReport{};
+    }
+    b->in_flight = false;
     return ST_OK;
 }
 
@@ -991,10 +1018,6 @@ int st_batch_create(st_library *lib, const st_batch_opts *opts, st_hist *const *
     char *work = nullptr;
     hipError_t e = dev_malloc((void **)&work, c.bytes);
     b->ctl = reinterpret_cast<BatchCtl *>(work);
-    if (e == hipSuccess) {
-        batch_reset_kernel<<<1, 64, 0, b->stream>>>(b->ctl);
-        e = hipGetLastError();
-    }
     if (e != hipSuccess) return fail(set_error(hip_status(e), "st_batch_create: %s", hipGetErrorString(e)));
     if (wave) {
         b->wave_plan = reinterpret_cast<PlanTrack *>(work + at_plan);
@@ -1002,8 +1025,6 @@ int st_batch_create(st_library *lib, const st_batch_opts *opts, st_hist *const *
         b->slab = reinterpret_cast<unsigned int *>(work + at_slab);
         b->report = (CtlReport *)report_slot_take(sizeof(CtlReport));   // (null: the control block is copied)
         if (b->report) *b->report = CtlReport{};
-        rc = launch_plan(lib, opts->n_oversamples, b->wave, b->wave_plan, b->stream);
-        if (rc) return fail(rc);
     }
     for (const st_geometry &g : lib->geoms) {
         st_vcs *m = nullptr;
@@ -1077,7 +1098,19 @@ int st_batch_run_static(st_library *lib, const st_batch_opts *opts, st_hist *con
 int st_batch_set_stream(st_batch *b, void *hip_stream)
 {
     if (!b) return set_error(ST_EINVAL, "st_batch_set_stream: null batch");
-    b->stream = hip_stream ? (hipStream_t)hip_stream : default_stream();
+    const hipStream_t next = hip_stream ? (hipStream_t)hip_stream : default_stream();
+    // A pass under way on the old stream ends first: the next one uses the same
+    // control block, queues, slabs, report and exact-path buffers, and its graph
+    // is given back below.  (Its own event is waited for: what others queued on
+    // the old stream may go on, and the stream itself may be gone.)
+    if (b->in_flight) {
+        if (!b->end || hipEventSynchronize(b->end) != hipSuccess) {   // (an event that a capture recorded)
+            (void)hipGetLastError();
+            ST_HIP_TRY(hipDeviceSynchronize());
+        }
+        b->in_flight = false;
+    }
+    b->stream = next;
     for (st_vcs *m : b->methods) st_vcs_set_stream(m, b->stream);
     if (b->exec) {
         (void)hipGraphExecDestroy(b->exec);
@@ -1097,11 +1130,15 @@ int st_batch_run(st_batch *b)
     if (b->opts.n_oversamples == 0) return ST_OK;
     if (!b->ev[0])
         for (hipEvent_t &e : b->ev) ST_HIP_TRY(hipEventCreate(&e));
+    b->in_flight = true;
+    b->end = nullptr;
+    int rc = prepare_passes(b);
+    if (rc) return rc;
     ST_HIP_TRY(hipEventRecord(b->ev[0], b->stream));
     if (b->opts.use_graph && b->rec.cap == 0) {
         if (!b->graph_ready) {
             ST_HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-            int rc = launch_fast(b);
+            rc = launch_fast(b);
             hipGraph_t g = nullptr;
             hipError_t e = hipStreamEndCapture(b->stream, &g);
             if (rc) return rc;
@@ -1112,14 +1149,16 @@ int st_batch_run(st_batch *b)
         }
         ST_HIP_TRY(hipGraphLaunch(b->exec, b->stream));
     } else {
-        int rc = launch_fast(b);
+        rc = launch_fast(b);
         if (rc) return rc;
     }
     ST_HIP_TRY(hipEventRecord(b->ev[1], b->stream));
-    if (b->lib->exact.empty()) return ST_OK;
-    int rc = run_exact(b);
-    if (rc) return rc;
-    ST_HIP_TRY(hipEventRecord(b->ev[2], b->stream));
+    if (!b->lib->exact.empty()) {
+        rc = run_exact(b);
+        if (rc) return rc;
+        ST_HIP_TRY(hipEventRecord(b->ev[2], b->stream));
+    }
+    b->end = b->ev[b->lib->exact.empty() ? 1 : 2];
     return ST_OK;
 }
 
