@@ -958,11 +958,13 @@ __global__ __launch_bounds__(kScanThreads) void hist_scan_kernel(ScanArgs a)
             uint64_t next = ~0ull;
             bool more = false;
             double acc = -0.0;   // -0.0 + y is y, whatever y is
-            for (int base = 0; base < m; base += kScanThreads) {
+            // (as many pairs a step as the list holds: all may be the key's)
+            static_assert(kScanList <= kScanThreads, "a thread for each pair of a step");
+            for (int base = 0; base < m; base += kScanList) {
                 const int i = base + tid;
                 uint64_t k = 0;
                 bool hit = false;
-                if (i < m) {
+                if (tid < kScanList && i < m) {
                     k = keys[i];
                     const bool sel = match(hash(k));
                     hit = sel && have && k == cur;
