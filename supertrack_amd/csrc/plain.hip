@@ -84,7 +84,6 @@ constexpr int kScoreBlock = 256;
 constexpr int kScoreRows = 4;
 constexpr int kScoreTile = kScoreBlock * kScoreRows;
 constexpr int kWaves = kScoreBlock / 64;
-constexpr int kPlainTiles = 256;
 
 // Geometry of the membership test, in the reference's units.
 struct ScoreGeom {
@@ -155,16 +154,15 @@ __global__ __launch_bounds__(kScoreBlock) void score_kernel(ScoreArgs a)
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
-    // Tiles wait for lower tiles only.  Up to kPlainTiles workgroups are all
-    // resident at once, so theirs need no tickets (a device atomic and a
-    // barrier before the first load: 8.0 -> 7.6 us on a 150e3-point track,
-    // 4.8 us either way on 5e3 points).
-    int tile = blockIdx.x;
-    if (a.num_tiles > kPlainTiles) {
-        if (tid == 0) s_tile = (int)(atomicAdd(a.ticket, 1ull) - a.ticket_base);
-        __syncthreads();
-        tile = s_tile;
-    }
+    // A tile waits for lower tiles, so tiles are numbered in the order in which
+    // workgroups start: the lowest unfinished one is then always running,
+    // whatever else holds the device.  (By blockIdx it might not be: each XCD
+    // starts its own share of a grid, and kernels on several streams or of
+    // several processes may hold one another's places.  The ticket costs 0.4 of
+    // 8.0 us on a 150e3-point track and nothing on 5e3 points.)
+    if (tid == 0) s_tile = (int)(atomicAdd(a.ticket, 1ull) - a.ticket_base);
+    __syncthreads();
+    const int tile = s_tile;
     const int64_t base = (int64_t)tile * kScoreTile;
     const double sx = a.shifts[3 * a.os + 0];
     const double sy = a.shifts[3 * a.os + 1];
@@ -1971,7 +1969,7 @@ int st_vcs_process_oversample(st_vcs *m, const st_track *track, st_pairs *out)
     a.num_tiles = tiles;
     score_kernel<<<tiles, kScoreBlock, 0, m->stream>>>(a);
     ST_HIP_TRY(hipGetLastError());
-    if (tiles > kPlainTiles) m->ticket_base += (uint64_t)tiles;
+    m->ticket_base += (uint64_t)tiles;
     m->oversample++;
     return ST_OK;
 }
