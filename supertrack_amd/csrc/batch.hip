@@ -313,10 +313,9 @@ int launch_plan(const st_library *L, int n_os, const WaveLaunch &w, PlanTrack *p
     const double waves = (double)w.grid * w.wg_waves;
     const double even = (double)L->wave_points * n_os / waves;
     const int min_points = (int)std::min(std::max(even, 2048.0), 12288.0);
-    wave_plan_kernel<<<1, 64 * kQueues, 0, stream>>>(L->tracks_dev, L->wave_order_dev, (int32_t)L->wave_order.size(),
-                                                     n_os, L->wave_points, n_os / (waves * 7.0), min_points,
-                                                     plan_stride(L), plan, plan_totals(L, plan));
-    ST_HIP_TRY(hipGetLastError());
+    ST_HIP_TRY(launch(wave_plan_kernel, 1, 64 * kQueues, 0, stream, L->tracks_dev, L->wave_order_dev,
+                      (int32_t)L->wave_order.size(), n_os, L->wave_points, n_os / (waves * 7.0), min_points,
+                      plan_stride(L), plan, plan_totals(L, plan)));
     return ST_OK;
 }
 
@@ -326,8 +325,7 @@ int launch_plan(const st_library *L, int n_os, const WaveLaunch &w, PlanTrack *p
 int launch_pass(int precision, const BatchArgs &args, const Launch &ln, const WaveArgs *wave, const WaveLaunch &w,
                 hipStream_t stream)
 {
-    batch_reset_kernel<<<1, 64, 0, stream>>>(args.ctl);
-    ST_HIP_TRY(hipGetLastError());
+    ST_HIP_TRY(launch(batch_reset_kernel, 1, 64, 0, stream, args.ctl));
     if (wave && wave->plan.n_tracks > 0) {
         WaveArgs a = *wave;
         void *kargs[] = {&a};
@@ -340,10 +338,8 @@ int launch_pass(int precision, const BatchArgs &args, const Launch &ln, const Wa
         void *kargs[] = {&a};
         ST_HIP_TRY(hipLaunchKernel(k, dim3(ln.grid), dim3(kBT), kargs, ln.lds, stream));
     }
-    if (wave && wave->plan.n_tracks > 0 && wave->slab) {
-        slab_sum_kernel<<<slab_blocks(wave->b.hist_lds_words), 1024, 0, stream>>>(*wave, w.grid);
-        ST_HIP_TRY(hipGetLastError());
-    }
+    if (wave && wave->plan.n_tracks > 0 && wave->slab)
+        ST_HIP_TRY(launch(slab_sum_kernel, slab_blocks(wave->b.hist_lds_words), 1024, 0, stream, *wave, w.grid));
     return ST_OK;
 }
 

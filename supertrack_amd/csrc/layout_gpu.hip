@@ -585,7 +585,7 @@ int layout_chunk_device(const double *x, const double *y, const double *z, const
         const UploadPart first[2] = {column(2), {tds_dev, tds, n_tracks * sizeof(TrackDesc)}};
         ST_HIP_TRY(upload(first, 2));
         const int bt_grid = (int)std::min<int64_t>((n_tracks + 3) / 4, 4096);
-        block_track_kernel<<<bt_grid, kThreads, 0, stream>>>(tds_dev, n_tracks, bbase, bt);
+        ST_HIP_TRY(launch(block_track_kernel, bt_grid, kThreads, 0, stream, tds_dev, n_tracks, bbase, bt));
         SortArgs a{};
         a.key = (unsigned long long *)(s + at_key[0]);
         a.index = (uint32_t *)(s + at_index[0]);
@@ -596,16 +596,15 @@ int layout_chunk_device(const double *x, const double *y, const double *z, const
         a.totals = (uint32_t *)(s + at_totals);
         a.n = n_points;
         a.tiles = tiles;
-        keys_kernel<<<(unsigned)nblocks, kThreads, 0, stream>>>(tds_dev, bt, pbase, bbase, raw + 2 * n,
-                                                                 (unsigned long long *)a.key, (uint32_t *)a.index,
-                                                                 (uint32_t *)a.track);
-        auto pass = [&](int shift) {
+        ST_HIP_TRY(launch(keys_kernel, (unsigned)nblocks, kThreads, 0, stream, tds_dev, bt, pbase, bbase, raw + 2 * n,
+                          (unsigned long long *)a.key, (uint32_t *)a.index, (uint32_t *)a.track));
+        auto count = few ? sort_count_kernel<kRowsFew> : sort_count_kernel<kRowsMany>;
+        auto scatter = few ? sort_scatter_kernel<kRowsFew> : sort_scatter_kernel<kRowsMany>;
+        auto pass = [&](int shift) -> int {
             a.shift = shift;
-            if (few) sort_count_kernel<kRowsFew><<<tiles, kThreads, 0, stream>>>(a);
-            else sort_count_kernel<kRowsMany><<<tiles, kThreads, 0, stream>>>(a);
-            sort_scan_kernel<<<kDigits, kThreads, 0, stream>>>(a.counts, a.totals, tiles);
-            if (few) sort_scatter_kernel<kRowsFew><<<tiles, kThreads, 0, stream>>>(a);
-            else sort_scatter_kernel<kRowsMany><<<tiles, kThreads, 0, stream>>>(a);
+            ST_HIP_TRY(launch(count, tiles, kThreads, 0, stream, a));
+            ST_HIP_TRY(launch(sort_scan_kernel, kDigits, kThreads, 0, stream, a.counts, a.totals, tiles));
+            ST_HIP_TRY(launch(scatter, tiles, kThreads, 0, stream, a));
             const uint32_t *i = a.index;
             a.index = a.index_out;
             a.index_out = (uint32_t *)i;
@@ -614,11 +613,13 @@ int layout_chunk_device(const double *x, const double *y, const double *z, const
                 a.key = a.key_out;
                 a.key_out = (unsigned long long *)k;
             }
+            return ST_OK;
         };
-        for (int shift = 0; shift < 64; shift += 8) pass(shift);
+        int rc = ST_OK;
+        for (int shift = 0; shift < 64 && !rc; shift += 8) rc = pass(shift);
         a.key = nullptr;   // then by track
-        for (int shift = 0; shift < 32 && (n_tracks - 1) >> shift; shift += 8) pass(shift);
-        ST_HIP_TRY(hipGetLastError());
+        for (int shift = 0; shift < 32 && (n_tracks - 1) >> shift && !rc; shift += 8) rc = pass(shift);
+        if (rc) return rc;
         const UploadPart rest[3] = {column(0), column(1), column(3)};
         ST_HIP_TRY(upload(rest, 3));
         BlockArgs ba{};
@@ -634,16 +635,17 @@ int layout_chunk_device(const double *x, const double *y, const double *z, const
         ba.pbase = pbase;
         ba.bbase = bbase;
         ba.geoms = gs;
-        block_kernel<<<(unsigned)nblocks, kThreads, 0, stream>>>(ba);
+        ST_HIP_TRY(launch(block_kernel, (unsigned)nblocks, kThreads, 0, stream, ba));
     }
-    track_kernel<<<(unsigned)n_tracks, 64, 0, stream>>>(tds_dev, (const BlockSum *)(s + at_sums), dst.z, pbase, bbase,
-                                                        precision, gs, tests);
+    ST_HIP_TRY(launch(track_kernel, (unsigned)n_tracks, 64, 0, stream, tds_dev, (const BlockSum *)(s + at_sums), dst.z,
+                      pbase, bbase, precision, gs, tests));
     if (nblocks > 0)
-        window_kernel<<<(unsigned)nblocks, kThreads, 0, stream>>>(tds_dev, bt, dst, pbase, bbase, gs, tests);
-    flags_kernel<<<(unsigned)((n_tracks + kThreads - 1) / kThreads), kThreads, 0, stream>>>(tds_dev, tests, n_tracks);
+        ST_HIP_TRY(launch(window_kernel, (unsigned)nblocks, kThreads, 0, stream, tds_dev, bt, dst, pbase, bbase, gs,
+                          tests));
+    ST_HIP_TRY(launch(flags_kernel, (unsigned)((n_tracks + kThreads - 1) / kThreads), kThreads, 0, stream, tds_dev,
+                      tests, n_tracks));
     if (precision == ST_F64 && nblocks > 0)
-        lineal_kernel<<<(unsigned)nblocks, kThreads, 0, stream>>>(tds_dev, bt, dst.e, pbase, bbase, gs);
-    ST_HIP_TRY(hipGetLastError());
+        ST_HIP_TRY(launch(lineal_kernel, (unsigned)nblocks, kThreads, 0, stream, tds_dev, bt, dst.e, pbase, bbase, gs));
     ST_HIP_TRY(hipMemcpyAsync(tds, tds_dev, n_tracks * sizeof(TrackDesc), hipMemcpyDeviceToHost, stream));
     ST_HIP_TRY(hipStreamSynchronize(stream));
     return ST_OK;

@@ -1458,12 +1458,13 @@ template <typename Use> static int fetch_counts(st_hist *h, bool reset, Use &&us
 {
     const size_t bytes = (size_t)h->nbins * sizeof(uint64_t);
     if (void *slot = report_slot_take(bytes)) {
-        fetch_counts_kernel<<<grid_for(h->nbins, 256, 256), 256, 0, h->stream>>>(
-            (unsigned long long *)h->bins_dev, (unsigned long long *)slot, h->nbins, reset ? 1 : 0);
-        hipError_t e = hipGetLastError();
-        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-        // (after a failed wait the slot may still be written to: it is not used again)
+        const hipError_t e = launch(fetch_counts_kernel, grid_for(h->nbins, 256, 256), 256, 0, h->stream,
+                                    (unsigned long long *)h->bins_dev, (unsigned long long *)slot, h->nbins,
+                                    reset ? 1 : 0);
+        if (e != hipSuccess) report_slot_give(slot, bytes);
         ST_HIP_TRY(e);
+        // (after a failed wait the slot may still be written to: it is not used again)
+        ST_HIP_TRY(hipStreamSynchronize(h->stream));
         use((const uint64_t *)slot);
         report_slot_give(slot, bytes);
         return ST_OK;
@@ -1472,9 +1473,8 @@ template <typename Use> static int fetch_counts(st_hist *h, bool reset, Use &&us
     ST_HIP_TRY(hipStreamSynchronize(h->stream));
     use(h->host_counts.data());
     if (reset) {
-        zero_u64_kernel<<<grid_for(h->nbins, 256, 1024), 256, 0, h->stream>>>((unsigned long long *)h->bins_dev,
-                                                                              h->nbins);
-        ST_HIP_TRY(hipGetLastError());
+        ST_HIP_TRY(launch(zero_u64_kernel, grid_for(h->nbins, 256, 1024), 256, 0, h->stream,
+                          (unsigned long long *)h->bins_dev, h->nbins));
         ST_HIP_TRY(hipStreamSynchronize(h->stream));
     }
     return ST_OK;
@@ -1495,14 +1495,12 @@ int hist_add_pairs(st_hist *h, const st_pairs *pairs, hipStream_t stream)
     h->bins_zero = false;
     if (pairs->capacity <= kScanPairs) {
         const ScanArgs sa{ha, scan_part_bits(pairs->capacity), (int)pairs->capacity};
-        if (pairs->capacity <= kScanSmall) hist_scan_kernel<true><<<1 << sa.part_bits, kScanThreads, 0, stream>>>(sa);
-        else hist_scan_kernel<false><<<1 << sa.part_bits, kScanThreads, 0, stream>>>(sa);
-        ST_HIP_TRY(hipGetLastError());
+        ST_HIP_TRY(launch(pairs->capacity <= kScanSmall ? hist_scan_kernel<true> : hist_scan_kernel<false>,
+                          1 << sa.part_bits, kScanThreads, 0, stream, sa));
         return ST_OK;
     }
     // small inputs (decided on the device) take the one-workgroup LDS sort
-    hist_lds_kernel<<<1, kSortThreads, kLdsBytes, stream>>>(ha);
-    ST_HIP_TRY(hipGetLastError());
+    ST_HIP_TRY(launch(hist_lds_kernel, 1, kSortThreads, kLdsBytes, stream, ha));
     if (pairs->capacity <= kLdsCap) return ST_OK;
     rc = ensure_sort_buffers(h, pairs->capacity);
     if (rc) return rc;
@@ -1512,7 +1510,7 @@ int hist_add_pairs(st_hist *h, const st_pairs *pairs, hipStream_t stream)
     const int passes = (bits + kGBits - 1) / kGBits;
     const int tiles = (int)((pairs->capacity + kOsTile - 1) / kOsTile);
     OsDigitsArgs da{pairs->volume, pairs->count_dev, h->digit_counts, passes};
-    os_digits_kernel<<<tiles, kOsThreads, 0, stream>>>(da);
+    ST_HIP_TRY(launch(os_digits_kernel, tiles, kOsThreads, 0, stream, da));
     const uint64_t *src_k = nullptr;
     const uint32_t *src_v = nullptr;
     uint64_t *bk[2] = {h->keys_a, h->keys_b};
@@ -1532,14 +1530,13 @@ int hist_add_pairs(st_hist *h, const st_pairs *pairs, hipStream_t stream)
         pa.epoch = ++h->os_epoch;
         if ((pa.epoch & 0x3FFFFFFFu) == 0) pa.epoch = ++h->os_epoch;
         pa.shift = p * kGBits;
-        os_pass_kernel<<<tiles, kOsThreads, 0, stream>>>(pa);
+        ST_HIP_TRY(launch(os_pass_kernel, tiles, kOsThreads, 0, stream, pa));
         h->os_ticket_base += (unsigned long long)tiles;
         src_k = bk[p & 1];
         src_v = bv[p & 1];
     }
     OsReduceArgs ra{ha, src_k, src_v, h->digit_counts, passes};
-    os_reduce_kernel<<<grid_for(pairs->capacity, 256, 2048), 256, 0, stream>>>(ra);
-    ST_HIP_TRY(hipGetLastError());
+    ST_HIP_TRY(launch(os_reduce_kernel, grid_for(pairs->capacity, 256, 2048), 256, 0, stream, ra));
     return ST_OK;
 }
 
@@ -1600,8 +1597,9 @@ int queue_flush(st_vcs *m)
                     if (std::find(consumers.begin(), consumers.end(), h) == consumers.end()) consumers.push_back(h);
                     h->bins_zero = false;
                 }
-                queued_track_kernel<<<a.n_os, kSortThreads, kLdsBytes, m->stream>>>(a);
-                if (hipGetLastError() != hipSuccess) rc = set_error(ST_EHIP, "queued_track_kernel launch failed");
+                const hipError_t e = launch(queued_track_kernel, a.n_os, kSortThreads, kLdsBytes, m->stream, a);
+                if (e != hipSuccess)
+                    rc = set_error(ST_EHIP, "queued_track_kernel launch failed: %s", hipGetErrorString(e));
             }
             k0 = k1;
         }
@@ -1734,9 +1732,8 @@ int st_pairs_alloc(st_pairs *p, int64_t capacity)
     }
     const int32_t c = (int32_t)capacity;
     hipStream_t stream = default_stream();
-    empty_pairs_kernel<<<grid_for((int64_t)n, 256, 4096), 256, 0, stream>>>(
-        (unsigned long long *)p->volume, (unsigned long long *)p->edep, (int64_t)n, p->count_dev, c);
-    hipError_t e = hipGetLastError();
+    hipError_t e = launch(empty_pairs_kernel, grid_for((int64_t)n, 256, 4096), 256, 0, stream,
+                          (unsigned long long *)p->volume, (unsigned long long *)p->edep, (int64_t)n, p->count_dev, c);
     if (e == hipSuccess) e = hipStreamSynchronize(stream);
     if (e != hipSuccess) {
         st_pairs_free(p);
@@ -1879,9 +1876,9 @@ int vcs_begin_track(st_vcs *m, st_track *track, const double *z_from, uint64_t s
         sa.track_index = track_index;
         sa.shift_xy = m->shift_xy;
         sa.shift_z = m->shift_z;
-        track_setup_kernel<<<grid_for(std::max<int64_t>(n, n_oversamples), 256, 4096), 256, 0, m->stream>>>(sa);
+        ST_HIP_TRY(launch(track_setup_kernel, grid_for(std::max<int64_t>(n, n_oversamples), 256, 4096), 256, 0,
+                          m->stream, sa));
     }
-    ST_HIP_TRY(hipGetLastError());
     m->n = n;
     m->n_oversamples = n_oversamples;
     m->oversample = 0;
@@ -1967,8 +1964,7 @@ int st_vcs_process_oversample(st_vcs *m, const st_track *track, st_pairs *out)
     a.epoch = ++m->epoch;
     if ((a.epoch & 0x3FFFFFFFu) == 0) a.epoch = ++m->epoch;
     a.num_tiles = tiles;
-    score_kernel<<<tiles, kScoreBlock, 0, m->stream>>>(a);
-    ST_HIP_TRY(hipGetLastError());
+    ST_HIP_TRY(launch(score_kernel, tiles, kScoreBlock, 0, m->stream, a));
     m->ticket_base += (uint64_t)tiles;
     m->oversample++;
     return ST_OK;
@@ -2099,9 +2095,8 @@ int st_hist_begin_track(st_hist *h, const st_pairs *pairs)
     // already are unless something was counted since they were cleared, and
     // they keep the counts carried from tracks ended without a host copy
     if (!h->bins_zero && !h->carry) {
-        zero_u64_kernel<<<grid_for(h->nbins, 256, 1024), 256, 0, h->stream>>>(
-            (unsigned long long *)h->bins_dev, h->nbins);
-        ST_HIP_TRY(hipGetLastError());
+        ST_HIP_TRY(launch(zero_u64_kernel, grid_for(h->nbins, 256, 1024), 256, 0, h->stream,
+                          (unsigned long long *)h->bins_dev, h->nbins));
         h->bins_zero = true;
     }
     h->in_track = true;

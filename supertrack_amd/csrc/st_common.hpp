@@ -38,6 +38,21 @@ hipStream_t default_stream();
 hipError_t dev_malloc(void **p, size_t bytes);
 hipError_t dev_free(void *p);
 
+// Launches a kernel and returns this launch's own status.  (hipGetLastError
+// after a launch may hold an older error of the thread: a failed allocation
+// that was reported long ago, or one of the caller's own calls.)
+template <typename T>
+struct Same {
+    using type = T;
+};
+template <typename... P>
+inline hipError_t launch(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t stream,
+                         typename Same<P>::type... args)
+{
+    void *where[] = {(void *)&args...};
+    return hipLaunchKernel((const void *)kernel, grid, block, where, lds, stream);
+}
+
 // Status for a failed HIP call: ST_ENOMEM for an allocation failure.
 inline int hip_status(hipError_t e)
 {

@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "parallel.hpp"
+#include "st_common.hpp"
 
 namespace st {
 
@@ -209,8 +210,7 @@ hipError_t staged_upload(const UploadPart *parts, int n, size_t total)
                     most = std::max(most, p.bytes);
                 }
                 const dim3 grid((unsigned)((most / 16 + 255) / 256 + 1), (unsigned)pieces.size());
-                gather_kernel<<<grid, 256, 0, nullptr>>>(a);
-                e = hipGetLastError();
+                e = launch(gather_kernel, grid, 256, 0, nullptr, a);
             }
             const hipError_t noted = hipEventRecord(s->ev[k & 1], nullptr);
             if (e == hipSuccess) e = noted;
