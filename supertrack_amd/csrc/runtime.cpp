@@ -8,7 +8,7 @@
 #include <map>
 #include <mutex>
 #include <new>
-#include <unordered_map>
+#include <set>
 #include <vector>
 
 #include "st_common.hpp"
@@ -64,7 +64,11 @@ struct Kept {
 std::mutex g_pool_mu;
 // (the maps are never destroyed: objects may be freed at exit)
 auto &g_pool = *new std::map<std::pair<int, size_t>, std::vector<Kept>>;          // (device, size)
-auto &g_pool_live = *new std::unordered_map<void *, std::pair<int, size_t>>;      // blocks handed out
+struct Live {
+    int dev;
+    size_t size, asked;   // bytes of the block, and those its taker asked for
+};
+auto &g_pool_live = *new std::map<uintptr_t, Live>;   // blocks handed out
 auto &g_pool_synced = *new std::map<int, uint64_t>;   // device: blocks given back before this are free of work
 size_t g_pool_bytes = 0;
 uint64_t g_pool_clock = 0;
@@ -75,6 +79,35 @@ size_t pool_size(size_t bytes)
     size_t step = 256;
     while (bytes > step * 4) step *= 2;
     return (bytes + step - 1) / step * step;
+}
+
+// The handed-out block that holds p (g_pool_mu held).
+std::map<uintptr_t, Live>::iterator live_block(const void *p)
+{
+    auto it = g_pool_live.upper_bound((uintptr_t)p);
+    if (it == g_pool_live.begin()) return g_pool_live.end();
+    --it;
+    return (uintptr_t)p - it->first < it->second.asked ? it : g_pool_live.end();
+}
+
+// Notes that [p, p + bytes) was allocated anew: handed-out blocks noted there
+// were freed by other means (g_pool_mu held).
+void forget_blocks(const void *p, size_t bytes)
+{
+    auto it = g_pool_live.lower_bound((uintptr_t)p);
+    while (it != g_pool_live.end() && it->first - (uintptr_t)p < bytes) it = g_pool_live.erase(it);
+    if (it == g_pool_live.begin()) return;
+    --it;
+    if (it->first + it->second.size > (uintptr_t)p) g_pool_live.erase(it);
+}
+
+// Whether p lies in a kept block, one given back already (g_pool_mu held).
+bool in_kept_block(const void *p)
+{
+    for (const auto &size : g_pool)
+        for (const Kept &k : size.second)
+            if (p >= k.p && (uintptr_t)p - (uintptr_t)k.p < size.first.second) return true;
+    return false;
 }
 
 // All kept blocks back to the device (g_pool_mu held).
@@ -101,6 +134,10 @@ hipError_t dev_malloc(void **p, size_t bytes)
                 pool_trim();
                 e = hipMalloc(p, bytes);
             }
+        }
+        if (e == hipSuccess) {
+            std::lock_guard<std::mutex> lock(g_pool_mu);
+            forget_blocks(*p, bytes);
         }
         return e;
     }
@@ -147,7 +184,8 @@ hipError_t dev_malloc(void **p, size_t bytes)
     }
     try {
         std::lock_guard<std::mutex> lock(g_pool_mu);
-        g_pool_live[got.p] = {dev, size};
+        forget_blocks(got.p, size);
+        g_pool_live[(uintptr_t)got.p] = {dev, size, bytes};
     } catch (const std::bad_alloc &) {   // no host memory to note it in: freed straight away later
     }
     *p = got.p;
@@ -161,9 +199,12 @@ hipError_t dev_free(void *p)
     bool kept = false;
     {
         std::lock_guard<std::mutex> lock(g_pool_mu);
-        auto it = g_pool_live.find(p);
+        auto it = live_block(p);
+        // (a block given back twice would be handed out twice)
+        if (it == g_pool_live.end() && in_kept_block(p)) return hipErrorInvalidValue;
         if (it != g_pool_live.end()) {
-            const std::pair<int, size_t> where = it->second;
+            const std::pair<int, size_t> where{it->second.dev, it->second.size};
+            p = (void *)it->first;   // (as hipFree, which takes any address inside an allocation)
             g_pool_live.erase(it);
             try {
                 while (g_pool_bytes + where.second > kPoolBytes) {
@@ -201,7 +242,9 @@ std::mutex g_slot_mu;
 struct SlotLists {
     std::vector<void *> of[2];
 };
-auto &g_slots = (new SlotLists)->of;   // (never destroyed, as above)
+// (never destroyed, as above)
+auto &g_slots = (new SlotLists)->of;
+auto &g_slots_live = *new std::set<void *>;   // slots handed out
 
 int slot_class(size_t bytes) { return bytes <= kSlotBytes[0] ? 0 : 1; }
 }  // namespace
@@ -214,6 +257,11 @@ void *report_slot_take(size_t bytes, bool counted)
         std::lock_guard<std::mutex> lock(g_slot_mu);
         if (!g_slots[c].empty()) {
             void *p = g_slots[c].back();
+            try {
+                g_slots_live.insert(p);
+            } catch (const std::bad_alloc &) {
+                return nullptr;
+            }
             g_slots[c].pop_back();
             return p;
         }
@@ -225,11 +273,15 @@ void *report_slot_take(size_t bytes, bool counted)
         (void)hipGetLastError();
         return nullptr;
     }
-    if (hipHostGetDevicePointer(&mapped, p, 0) != hipSuccess || mapped != p) {
-        (void)hipHostFree(p);
-        return nullptr;
+    bool ok = hipHostGetDevicePointer(&mapped, p, 0) == hipSuccess && mapped == p;
+    try {
+        std::lock_guard<std::mutex> lock(g_slot_mu);
+        if (ok) g_slots_live.insert(p);
+    } catch (const std::bad_alloc &) {
+        ok = false;
     }
-    return p;
+    if (!ok) (void)hipHostFree(p);
+    return ok ? p : nullptr;
 }
 
 void report_slot_give(void *p, size_t bytes)
@@ -238,12 +290,16 @@ void report_slot_give(void *p, size_t bytes)
     const int c = slot_class(bytes);
     {
         std::lock_guard<std::mutex> lock(g_slot_mu);
-        try {
-            if (g_slots[c].size() < kKeptSlots) {
+        if (g_slots_live.erase(p) == 0) {
+            // given back already, or not one of these slots
+            for (const std::vector<void *> &kept : g_slots)
+                if (std::find(kept.begin(), kept.end(), p) != kept.end()) return;
+        } else if (g_slots[c].size() < kKeptSlots) {
+            try {
                 g_slots[c].push_back(p);
                 return;
+            } catch (const std::bad_alloc &) {
             }
-        } catch (const std::bad_alloc &) {
         }
     }
     (void)hipHostFree(p);
