@@ -87,7 +87,7 @@ std::map<uintptr_t, Live>::iterator live_block(const void *p)
     auto it = g_pool_live.upper_bound((uintptr_t)p);
     if (it == g_pool_live.begin()) return g_pool_live.end();
     --it;
-    return (uintptr_t)p - it->first < it->second.asked ? it : g_pool_live.end();
+    return (uintptr_t)p - it->first < it->second.size ? it : g_pool_live.end();
 }
 
 // Notes that [p, p + bytes) was allocated anew: handed-out blocks noted there
@@ -218,7 +218,8 @@ hipError_t dev_free(void *p)
         std::lock_guard<std::mutex> lock(g_pool_mu);
         auto it = live_block(p);
         // (a block given back twice would be handed out twice)
-        if (it == g_pool_live.end() && in_kept_block(p)) return hipErrorInvalidValue;
+        if (it == g_pool_live.end() ? in_kept_block(p) : (uintptr_t)p - it->first >= it->second.asked)
+            return hipErrorInvalidValue;
         if (it != g_pool_live.end()) {
             const std::pair<int, size_t> where{it->second.dev, it->second.size};
             p = (void *)it->first;   // (as hipFree, which takes any address inside an allocation)
@@ -247,6 +248,47 @@ hipError_t dev_free(void *p)
     for (void *old : evicted) (void)hipFree(old);
     if (kept) return hipSuccess;
     return hipFree(p);
+}
+
+hipError_t dev_check(const void *p, size_t bytes)
+{
+    std::lock_guard<std::mutex> lock(g_pool_mu);
+    auto it = live_block(p);
+    return it != g_pool_live.end() && (uintptr_t)p - it->first + bytes > it->second.asked ? hipErrorInvalidValue
+                                                                                          : hipSuccess;
+}
+
+bool dev_known(const void *p)
+{
+    {
+        std::lock_guard<std::mutex> lock(g_pool_mu);
+        if (live_block(p) != g_pool_live.end()) return true;
+    }
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+    return false;
+}
+
+bool dev_writable(const void *p, size_t bytes)
+{
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    {
+        std::lock_guard<std::mutex> lock(g_pool_mu);
+        auto it = live_block(p);
+        if (it != g_pool_live.end())
+            return it->second.dev == dev && (uintptr_t)p - it->first + bytes <= it->second.asked;
+    }
+    hipPointerAttribute_t a{};
+    hipDeviceptr_t start = nullptr;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess || a.type != hipMemoryTypeDevice || a.device != dev ||
+        hipMemGetAddressRange(&start, &size, const_cast<void *>(p)) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return (uintptr_t)p >= (uintptr_t)start && (uintptr_t)p - (uintptr_t)start + bytes <= size;
 }
 
 namespace {
@@ -454,6 +496,8 @@ int st_memcpy_dtoh(void *dst, const void *src, size_t bytes)
 int st_memcpy_dtod(void *dst, const void *src, size_t bytes)
 {
     if (!bytes) return ST_OK;
+    ST_HIP_TRY(dev_check(dst, bytes));
+    ST_HIP_TRY(dev_check(src, bytes));
     ST_HIP_TRY(hipDeviceSynchronize());
     ST_HIP_TRY(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToDevice));
     ST_HIP_TRY(hipDeviceSynchronize());
@@ -463,6 +507,7 @@ int st_memcpy_dtod(void *dst, const void *src, size_t bytes)
 int st_memset(void *dst, int value, size_t bytes)
 {
     if (!bytes) return ST_OK;
+    ST_HIP_TRY(dev_check(dst, bytes));
     ST_HIP_TRY(hipDeviceSynchronize());
     ST_HIP_TRY(hipMemset(dst, value, bytes));
     ST_HIP_TRY(hipDeviceSynchronize());

@@ -37,6 +37,15 @@ hipStream_t default_stream();
 // work that was queued before they were given back.
 hipError_t dev_malloc(void **p, size_t bytes);
 hipError_t dev_free(void *p);
+// hipErrorInvalidValue if p lies in a block of dev_malloc's and p + bytes
+// passes the size asked for (the block itself is larger, so that HIP's own
+// check of copies and fills would let them pass).
+hipError_t dev_check(const void *p, size_t bytes);
+// Whether HIP knows p as memory of its own.
+bool dev_known(const void *p);
+// Whether a kernel on the current device may write [p, p + bytes): memory of
+// this device, and all of it in one allocation.
+bool dev_writable(const void *p, size_t bytes);
 
 // Launches a kernel and returns this launch's own status.  (hipGetLastError
 // after a launch may hold an older error of the thread: a failed allocation

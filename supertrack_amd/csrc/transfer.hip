@@ -104,15 +104,28 @@ void give(Stage *s)
     destroy(s);
 }
 
-// Whether the copy engine can read p itself (pinned host memory).
-bool is_pinned(const void *p)
+// What [p, p + bytes), which the caller names as host memory, is.  Staging reads
+// and writes it with memcpy: all else (device memory, a range past its pinned
+// allocation) is left to hipMemcpy, which copies or refuses it.
+enum class HostRange { ordinary, pinned, other };
+HostRange host_range(const void *p, size_t bytes)
 {
+    if (!p) return HostRange::other;
     hipPointerAttribute_t a{};
     if (hipPointerGetAttributes(&a, p) != hipSuccess) {
         (void)hipGetLastError();
-        return false;
+        return HostRange::ordinary;
     }
-    return a.type == hipMemoryTypeHost;
+    if (a.type == hipMemoryTypeUnregistered) return HostRange::ordinary;
+    if (a.type != hipMemoryTypeHost && a.type != hipMemoryTypeManaged) return HostRange::other;
+    hipDeviceptr_t start = nullptr;
+    size_t size = 0;
+    if (hipMemGetAddressRange(&start, &size, const_cast<void *>(p)) != hipSuccess) {
+        (void)hipGetLastError();
+        return HostRange::other;
+    }
+    const bool inside = (uintptr_t)p >= (uintptr_t)start && (uintptr_t)p - (uintptr_t)start + bytes <= size;
+    return inside ? HostRange::pinned : HostRange::other;
 }
 
 hipError_t plain_upload(const UploadPart *parts, int n)
@@ -156,7 +169,14 @@ __global__ __launch_bounds__(256) void gather_kernel(GatherArgs a)
 hipError_t staged_upload(const UploadPart *parts, int n, size_t total)
 {
     const int kind = total >= kLargeFrom ? 1 : 0;
-    if (kind && is_pinned(parts[0].src)) return plain_upload(parts, n);
+    for (int i = 0; i < n; ++i) {
+        if (parts[i].bytes == 0) continue;
+        const HostRange range = host_range(parts[i].src, parts[i].bytes);
+        // (the copy engine reads pinned memory itself; host memory in the device's
+        // place is for hipMemcpy to refuse)
+        if (range == HostRange::other || (kind && range == HostRange::pinned) || !dev_known(parts[i].dst))
+            return plain_upload(parts, n);
+    }
     const size_t cap = kSlot[kind];
     std::vector<Piece> pieces;
     std::vector<size_t> fills;   // first piece of each buffer's fill
@@ -175,7 +195,10 @@ hipError_t staged_upload(const UploadPart *parts, int n, size_t total)
     const size_t n_fills = fills.size();
     fills.push_back(pieces.size());
 
-    const bool gather = kind == 0 && n_fills == 1 && pieces.size() <= kGatherParts;
+    // (the kernel's stores are checked by no one else)
+    bool gather = kind == 0 && n_fills == 1 && pieces.size() <= kGatherParts;
+    for (size_t i = 0; gather && i < pieces.size(); ++i)
+        gather = dev_writable(parts[pieces[i].part].dst, parts[pieces[i].part].bytes);
     std::vector<std::thread> pool;
     std::vector<Stage *> stages;
     pool.reserve(kMaxWorkers);
@@ -247,7 +270,11 @@ hipError_t staged_upload(const UploadPart *parts, int n, size_t total)
 hipError_t upload(const UploadPart *parts, int n)
 {
     size_t total = 0;
-    for (int i = 0; i < n; ++i) total += parts[i].bytes;
+    for (int i = 0; i < n; ++i) {
+        total += parts[i].bytes;
+        const hipError_t e = dev_check(parts[i].dst, parts[i].bytes);
+        if (e != hipSuccess) return e;
+    }
     if (total == 0) return hipSuccess;
     try {
         return staged_upload(parts, n, total);
@@ -259,9 +286,11 @@ hipError_t upload(const UploadPart *parts, int n)
 hipError_t download(void *dst, const void *src, size_t bytes)
 {
     if (bytes == 0) return hipSuccess;
-    Stage *s = bytes <= kSlot[0] ? take(0) : nullptr;
+    hipError_t e = dev_check(src, bytes);
+    if (e != hipSuccess) return e;
+    Stage *s = bytes <= kSlot[0] && host_range(dst, bytes) != HostRange::other && dev_known(src) ? take(0) : nullptr;
     if (!s) return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
-    hipError_t e = hipMemcpyAsync(s->slot[0], src, bytes, hipMemcpyDeviceToHost, nullptr);
+    e = hipMemcpyAsync(s->slot[0], src, bytes, hipMemcpyDeviceToHost, nullptr);
     if (e == hipSuccess) e = hipEventRecord(s->ev[0], nullptr);
     const hipError_t waited = e == hipSuccess ? hipEventSynchronize(s->ev[0]) : hipStreamSynchronize(nullptr);
     if (e == hipSuccess) e = waited;
