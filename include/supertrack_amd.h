@@ -239,7 +239,9 @@ typedef struct {
     /* The next four name a launch shape of the block kernel (a workgroup per
      * segment), which then scores every fast track.  All 0: the one-wave
      * kernel (a wavefront per segment or part of one), and the block kernel,
-     * at the shapes below, for tracks that the former does not take. */
+     * at the shapes below, for tracks that the former does not take.  So does
+     * the shape that st_batch_params reports of the one-wave kernel
+     * (table_slots 416; blocks_per_cu then limits its workgroups). */
     int32_t table_slots;          /* LDS hash slots per workgroup: 1280 or 1472
                                      (one point per thread), 1536, 2048 or
                                      4096; 0 (with blocks_per_cu and
@@ -273,7 +275,7 @@ int st_batch_times(st_batch *b, float *ms2);
 /* Launch parameters in use (5 entries): block_threads, table_slots (per
  * workgroup; one-wave kernel: per wave), blocks_per_cu, points_per_thread,
  * hist_copies (0: the histograms count straight into the device counters, too
- * large for LDS). */
+ * large for LDS).  Passed as options they choose the same kernel and shape. */
 int st_batch_params(const st_batch *b, int32_t *params5);
 /* Counts of the last st_batch_run's fused kernel: stats3[0] points scored
  * (points of the in-voxel block ranges of the segments that pass the x/y

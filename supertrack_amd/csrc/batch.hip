@@ -375,8 +375,9 @@ int launch_fast(st_batch *b)
 // Launch shape of the one-wave kernel: the workgroup size (4 to 16 waves share
 // one privatised histogram) that keeps most waves resident on a CU; on a tie
 // the largest (fewest histograms to sum).  Histograms that do not fit beside
-// four waves' tables are counted in the device bins.
-int configure_wave(int precision, int hist_words, WaveLaunch *out)
+// four waves' tables are counted in the device bins.  max_blocks: the caller's
+// limit on workgroups per CU (0: none).
+int configure_wave(int precision, int hist_words, int max_blocks, WaveLaunch *out)
 {
     const void *k = wave_kernel_ptr(precision);
     const size_t per_wave = wave_lds(precision == ST_F64 ? 2 : 1, kWaveSlots);
@@ -405,15 +406,18 @@ int configure_wave(int precision, int hist_words, WaveLaunch *out)
     ST_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, k, 64 * best.wg_waves, best.lds));
     if (fit < 1) return set_error(ST_EHIP, "one-wave kernel cannot be resident with %zu B LDS", best.lds);
     best.blocks_per_cu = std::min(best.blocks_per_cu, fit);
+    if (max_blocks > 0) best.blocks_per_cu = std::min(best.blocks_per_cu, max_blocks);
     best.grid = best.blocks_per_cu * device_cu_count();
     *out = best;
     return ST_OK;
 }
 
-// A launch shape named by the caller is the block kernel's.
+// A launch shape named by the caller is the block kernel's, unless it is the
+// one that st_batch_params reports of the one-wave kernel (its table size).
+bool names_wave_shape(const st_batch_opts &o) { return o.table_slots == kWaveSlots; }
 bool names_block_shape(const st_batch_opts &o)
 {
-    return o.table_slots || o.blocks_per_cu || o.points_per_thread || o.hist_copies;
+    return !names_wave_shape(o) && (o.table_slots || o.blocks_per_cu || o.points_per_thread || o.hist_copies);
 }
 
 // Launch shape for (table slots, workgroups per CU, points per thread, LDS
@@ -458,12 +462,21 @@ int configure(st_batch *b, int slots, int bpc, int ppt, int copies)
 // plus the points of the iterations between occupancy checks, so every
 // fast-path track fits.  Defaults: the fastest shapes measured on MI355X for
 // 2 nm and 10 nm spheres.
-int default_launch(int precision, int hist_words, const st_batch_opts &o, Launch *out)
+int default_launch(int precision, int hist_words, const st_batch_opts &opts, Launch *out)
 {
+    st_batch_opts o = opts;
+    if (names_wave_shape(o)) {
+        if (o.points_per_thread > 1 || o.points_per_thread < 0 || o.hist_copies > 1 || o.hist_copies < 0 ||
+            o.blocks_per_cu < 0)
+            return set_error(ST_EINVAL, "batched run: %d table slots (the one-wave kernel) take one point per thread "
+                                        "and one copy of the histograms", kWaveSlots);
+        o.table_slots = o.blocks_per_cu = o.points_per_thread = o.hist_copies = 0;   // (the tracks left to the other)
+    }
     const bool f32 = precision == ST_F32;
     const int slots = o.table_slots ? o.table_slots : 1536;
     if (slots != 1280 && slots != 1472 && slots != 1536 && slots != 2048 && slots != 4096)
-        return set_error(ST_EINVAL, "batched run: table_slots must be 1280, 1472, 1536, 2048 or 4096");
+        return set_error(ST_EINVAL, "batched run: table_slots must be 1280, 1472, 1536, 2048 or 4096 "
+                                    "(or %d: the one-wave kernel)", kWaveSlots);
     const int bpc = o.blocks_per_cu ? o.blocks_per_cu : (f32 ? 5 : 4);
     const int ppt = o.points_per_thread ? o.points_per_thread : (f32 ? 1 : 2);
     if (ppt != 1 && ppt != 2) return set_error(ST_EINVAL, "batched run: points_per_thread must be 1 or 2");
@@ -1003,7 +1016,7 @@ int st_batch_create(st_library *lib, const st_batch_opts *opts, st_hist *const *
     if (rc) return fail(rc);
     const bool wave = !names_block_shape(*opts) && !lib->wave_order.empty() && opts->n_oversamples > 0;
     if (wave) {
-        rc = configure_wave(lib->precision, b->hist_words, &b->wave);
+        rc = configure_wave(lib->precision, b->hist_words, names_wave_shape(*opts) ? opts->blocks_per_cu : 0, &b->wave);
         if (rc) return fail(rc);
     }
     Carve c;
@@ -1074,7 +1087,7 @@ int st_batch_run_static(st_library *lib, const st_batch_opts *opts, st_hist *con
     WaveLaunch w;
     const bool wave = !names_block_shape(*opts) && !lib->wave_order.empty();
     if (wave) {
-        rc = configure_wave(lib->precision, hist_words, &w);
+        rc = configure_wave(lib->precision, hist_words, names_wave_shape(*opts) ? opts->blocks_per_cu : 0, &w);
         if (!rc) rc = launch_plan(lib, opts->n_oversamples, w, lib->static_plan, stream);
         if (rc) return rc;
     }
