@@ -726,6 +726,55 @@ int read_report(st_batch *b, CtlReport *out)
     return ST_OK;
 }
 
+// Appends a run of tracks (checked by the caller) to the library.
+int append_run(st_library *L, const double *x, const double *y, const double *z, const double *edep,
+               const int64_t *offsets, int64_t n_tracks, const int32_t *geom_of_track)
+{
+    const int n_geoms = (int)L->geoms.size();
+    const int64_t n_points = offsets[n_tracks] - offsets[0];
+    const int precision = L->precision;
+    const int64_t pbase = L->points_done;   // this chunk's first point in the library
+    int64_t bbase = 0;                       // this chunk's first block in the library
+    if (L->tracks_done > 0) {
+        const TrackDesc &last = L->tracks[L->tracks_done - 1];
+        bbase = last.block0 + last.nblocks;
+    }
+    TrackDesc *tds = L->tracks.data() + L->tracks_done;
+    const int64_t nblocks = plan_chunk(offsets, n_tracks, geom_of_track, pbase, bbase, tds);
+    if (bbase + nblocks > L->blocks_cap)
+        return set_error(ST_EINVAL, "st_library_append: block table overflow");
+    const LayoutDst dst{L->x64 + pbase, L->y64 + pbase, L->z64 + pbase, L->e64 + pbase,
+                        precision == ST_F32 ? reinterpret_cast<PointF32 *>(L->p32) + pbase : nullptr,
+                        L->zfirst + bbase, precision == ST_F32 ? L->blocks + bbase : nullptr};
+    int rc = layout_chunk_device(x + offsets[0], y + offsets[0], z + offsets[0], edep + offsets[0], n_points, n_tracks,
+                                 L->geoms.data(), n_geoms, precision, pbase, bbase, nblocks, tds, dst);
+    if (rc == ST_ENOMEM) {
+        // no room for the device's scratch beside the library: on the host
+        clear_error();
+        ChunkLayout lay;
+        fill_chunk(x, y, z, edep, offsets, n_tracks, L->geoms.data(), precision, pbase, bbase, nblocks, tds, lay);
+        if (precision == ST_F64)
+            for (int64_t t = 0; t < n_tracks; ++t) {
+                if (tds[t].flags & kFlagExact) continue;
+                double *e = lay.e.data() + (tds[t].offset - pbase);
+                for (int32_t p = 0; p < tds[t].n; ++p) e[p] = lineal_energy(e[p], L->geoms[tds[t].geom]);
+            }
+        rc = dev_put(dst.x, lay.x.data(), n_points);
+        if (!rc) rc = dev_put(dst.y, lay.y.data(), n_points);
+        if (!rc) rc = dev_put(dst.z, lay.z.data(), n_points);
+        if (!rc) rc = dev_put(dst.e, lay.e.data(), n_points);
+        if (!rc) rc = dev_put(dst.zfirst, lay.zfirst.data(), nblocks);
+        if (!rc && precision == ST_F32) {
+            rc = dev_put(dst.p32, lay.p32.data(), n_points);
+            if (!rc) rc = dev_put(dst.blocks, lay.blocks.data(), nblocks);
+        }
+    }
+    if (rc) return rc;
+    L->tracks_done += n_tracks;
+    L->points_done += n_points;
+    return ST_OK;
+}
+
 // The kernel's error flag and the conservation totals of a finished pass.
 int check_ctl(const CtlReport &c)
 {
@@ -814,46 +863,22 @@ int st_library_append(st_library *L, const double *x, const double *y, const dou
                          "(%lld / %lld left)",
                          (long long)n_tracks, (long long)n_points, (long long)(L->n_tracks - L->tracks_done),
                          (long long)(L->n_points - L->points_done));
-    const int precision = L->precision;
-    const int64_t pbase = L->points_done;   // this chunk's first point in the library
-    int64_t bbase = 0;                       // this chunk's first block in the library
-    if (L->tracks_done > 0) {
-        const TrackDesc &last = L->tracks[L->tracks_done - 1];
-        bbase = last.block0 + last.nblocks;
-    }
-    TrackDesc *tds = L->tracks.data() + L->tracks_done;
-    const int64_t nblocks = plan_chunk(offsets, n_tracks, geom_of_track, pbase, bbase, tds);
-    if (bbase + nblocks > L->blocks_cap)
-        return set_error(ST_EINVAL, "st_library_append: block table overflow");
-    const LayoutDst dst{L->x64 + pbase, L->y64 + pbase, L->z64 + pbase, L->e64 + pbase,
-                        precision == ST_F32 ? reinterpret_cast<PointF32 *>(L->p32) + pbase : nullptr,
-                        L->zfirst + bbase, precision == ST_F32 ? L->blocks + bbase : nullptr};
-    int rc = layout_chunk_device(x + offsets[0], y + offsets[0], z + offsets[0], edep + offsets[0], n_points, n_tracks,
-                                 L->geoms.data(), n_geoms, precision, pbase, bbase, nblocks, tds, dst);
-    if (rc == ST_ENOMEM) {
-        // no room for the device's scratch beside the library: on the host
-        clear_error();
-        ChunkLayout lay;
-        fill_chunk(x, y, z, edep, offsets, n_tracks, L->geoms.data(), precision, pbase, bbase, nblocks, tds, lay);
-        if (precision == ST_F64)
-            for (int64_t t = 0; t < n_tracks; ++t) {
-                if (tds[t].flags & kFlagExact) continue;
-                double *e = lay.e.data() + (tds[t].offset - pbase);
-                for (int32_t p = 0; p < tds[t].n; ++p) e[p] = lineal_energy(e[p], L->geoms[tds[t].geom]);
-            }
-        rc = dev_put(dst.x, lay.x.data(), n_points);
-        if (!rc) rc = dev_put(dst.y, lay.y.data(), n_points);
-        if (!rc) rc = dev_put(dst.z, lay.z.data(), n_points);
-        if (!rc) rc = dev_put(dst.e, lay.e.data(), n_points);
-        if (!rc) rc = dev_put(dst.zfirst, lay.zfirst.data(), nblocks);
-        if (!rc && precision == ST_F32) {
-            rc = dev_put(dst.p32, lay.p32.data(), n_points);
-            if (!rc) rc = dev_put(dst.blocks, lay.blocks.data(), nblocks);
+    // Runs of at most kStagePoints points and kRunTracks tracks (or one larger
+    // track): the layout's scratch and staging stay bounded, and so do its grids
+    // (a workgroup per block of points and per track, 2^32 threads at most).
+    constexpr int64_t kStagePoints = int64_t(1) << 25, kRunTracks = int64_t(1) << 22;
+    const int64_t tracks_before = L->tracks_done, points_before = L->points_done;
+    for (int64_t t0 = 0; t0 < n_tracks;) {
+        int64_t t1 = t0 + 1;
+        while (t1 < n_tracks && t1 - t0 < kRunTracks && offsets[t1 + 1] - offsets[t0] <= kStagePoints) ++t1;
+        const int rc = append_run(L, x, y, z, edep, offsets + t0, t1 - t0, geom_of_track ? geom_of_track + t0 : nullptr);
+        if (rc) {   // all of the call's tracks or none
+            L->tracks_done = tracks_before;
+            L->points_done = points_before;
+            return rc;
         }
+        t0 = t1;
     }
-    if (rc) return rc;
-    L->tracks_done += n_tracks;
-    L->points_done += n_points;
     return ST_OK;
 }
 
@@ -946,16 +971,7 @@ int st_library_create(const double *x, const double *y, const double *z, const d
     st_library *L = nullptr;
     int rc = st_library_begin(n_tracks, n_points, geoms, n_geoms, precision, &L);
     if (rc) return rc;
-    // append runs of tracks of at most kStagePoints points (or one larger
-    // track), so host staging stays bounded
-    constexpr int64_t kStagePoints = int64_t(1) << 25;
-    for (int64_t t0 = 0; t0 < n_tracks && !rc;) {
-        int64_t t1 = t0 + 1;
-        while (t1 < n_tracks && offsets[t1 + 1] - offsets[t0] <= kStagePoints) ++t1;
-        rc = st_library_append(L, x, y, z, edep, offsets + t0, t1 - t0,
-                               geom_of_track ? geom_of_track + t0 : nullptr);
-        t0 = t1;
-    }
+    rc = st_library_append(L, x, y, z, edep, offsets, n_tracks, geom_of_track);
     if (!rc) rc = st_library_finish(L);
     if (rc) {
         st_library_destroy(L);
