@@ -32,7 +32,7 @@ constexpr int kMaxWorkers = 2;
 // each kPerWorker of them.
 constexpr size_t kLargeFrom = (size_t)2 << 20, kPerWorker = (size_t)8 << 20;
 constexpr size_t kSlot[2] = {(size_t)512 << 10, (size_t)8 << 20};   // bytes of a buffer (small, large)
-constexpr size_t kKeep[2] = {16, kMaxWorkers};                      // pairs of buffers kept (16 + 32 MiB)
+constexpr size_t kKeep[2] = {16, kMaxWorkers};   // pairs of buffers kept for a device (16 + 32 MiB)
 
 // A pair of buffers, filled and copied in turn on the null stream, as
 // hipMemcpy copies.
@@ -93,8 +93,10 @@ void give(Stage *s)
     {
         std::lock_guard<std::mutex> lock(g_stage_mu);
         std::vector<Stage *> &kept = g_stages[s->kind];
+        const size_t same =
+            (size_t)std::count_if(kept.begin(), kept.end(), [&](const Stage *k) { return k->dev == s->dev; });
         try {
-            if (kept.size() < kKeep[s->kind]) {
+            if (same < kKeep[s->kind]) {
                 kept.push_back(s);
                 return;
             }
