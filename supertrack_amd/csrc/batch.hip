@@ -374,8 +374,15 @@ int launch_fast(st_batch *b)
 
 // Launch shape of the one-wave kernel: the workgroup size (4 to 16 waves share
 // one privatised histogram) that keeps most waves resident on a CU; on a tie
-// the largest (fewest histograms to sum).  Histograms that do not fit beside
-// four waves' tables are counted in the device bins.  max_blocks: the caller's
+// the largest (fewest histograms to sum).  Histograms so wide that fewer than
+// six waves (ST_F64: five) fit beside them are counted in the device bins, by
+// all the waves that the registers allow.  Which is faster depends on how often
+// spheres share a bin (us a pass, ST_F32, 192 tracks x 60, private / device
+// bins: 31e3 bins, six waves: 10 nm spheres 918 / 663, 100 nm 1640 / 708, 2 nm
+// 1466 / 2863, 1 nm 779 / 1383; 34e3 bins, four waves: 1255 / 676, 2282 / 710,
+// 2038 / 2884, 1048 / 1409); with fewer waves the private bins also lose to the
+// block kernel (34e3 bins: 10 nm 1158, 100 nm 1842; ST_F64, 30e3 bins, four
+// waves: 1321 and 2361 against 1168 and 2109).  max_blocks: the caller's
 // limit on workgroups per CU (0: none).
 int configure_wave(int precision, int hist_words, int max_blocks, WaveLaunch *out)
 {
@@ -384,6 +391,7 @@ int configure_wave(int precision, int hist_words, int max_blocks, WaveLaunch *ou
     hipFuncAttributes attr;
     ST_HIP_TRY(hipFuncGetAttributes(&attr, k));
     const int simd_waves = precision == ST_F64 ? 4 : 6;
+    const int min_private = precision == ST_F64 ? 5 : 6;
     const size_t kCuLds = 160 * 1024;
     WaveLaunch best;
     for (int pass = 0; pass < 2 && !best.on; ++pass) {
@@ -396,6 +404,7 @@ int configure_wave(int precision, int hist_words, int max_blocks, WaveLaunch *ou
             const size_t all = w.lds + attr.sharedSizeBytes + 1024;
             w.blocks_per_cu = std::min<int>((int)(kCuLds / all), 4 * simd_waves / wg);
             if (w.blocks_per_cu < 1) continue;
+            if (w.lds_hist && w.blocks_per_cu * wg < min_private) continue;
             w.on = true;
             if (!best.on || w.blocks_per_cu * wg >= best.blocks_per_cu * best.wg_waves) best = w;
         }
