@@ -1453,8 +1453,9 @@ int ensure_sort_buffers(st_hist *h, int64_t cap)
 }  // namespace
 
 // The device counters, as use(counts of nbins) sees them on the host once
-// everything queued on h's stream is done; reset: cleared.
-template <typename Use> static int fetch_counts(st_hist *h, bool reset, Use &&use)
+// everything queued on h's stream is done; reset: cleared.  Counts beyond a
+// report slot are copied to `wide`, an array of nbins.
+template <typename Use> static int fetch_counts(st_hist *h, bool reset, uint64_t *wide, Use &&use)
 {
     const size_t bytes = (size_t)h->nbins * sizeof(uint64_t);
     if (void *slot = report_slot_take(bytes)) {
@@ -1469,9 +1470,9 @@ template <typename Use> static int fetch_counts(st_hist *h, bool reset, Use &&us
         report_slot_give(slot, bytes);
         return ST_OK;
     }
-    ST_HIP_TRY(hipMemcpyAsync(h->host_counts.data(), h->bins_dev, bytes, hipMemcpyDeviceToHost, h->stream));
+    ST_HIP_TRY(hipMemcpyAsync(wide, h->bins_dev, bytes, hipMemcpyDeviceToHost, h->stream));
     ST_HIP_TRY(hipStreamSynchronize(h->stream));
-    use(h->host_counts.data());
+    use(wide);
     if (reset) {
         ST_HIP_TRY(launch(zero_u64_kernel, grid_for(h->nbins, 256, 1024), 256, 0, h->stream,
                           (unsigned long long *)h->bins_dev, h->nbins));
@@ -2137,7 +2138,7 @@ int st_hist_end_track(st_hist *h, double *host_bins)
         h->in_track = false;
         return ST_OK;
     }
-    rc = fetch_counts(h, true, [&](const uint64_t *counts) {
+    rc = fetch_counts(h, true, h->host_counts.data(), [&](const uint64_t *counts) {
         for (int i = 0; i < h->nbins; ++i) host_bins[i + 1] += (double)counts[i];
     });
     if (rc) return rc;
@@ -2152,8 +2153,8 @@ int st_hist_fetch(st_hist *h, uint64_t *counts, int32_t reset)
     if (!h || !counts) return set_error(ST_EINVAL, "st_hist_fetch: null argument");
     int rc = queue_flush_producers(h);
     if (rc) return rc;
-    rc = fetch_counts(h, reset != 0, [&](const uint64_t *fetched) {
-        std::memcpy(counts, fetched, (size_t)h->nbins * sizeof(uint64_t));
+    rc = fetch_counts(h, reset != 0, counts, [&](const uint64_t *fetched) {
+        if (fetched != counts) std::memcpy(counts, fetched, (size_t)h->nbins * sizeof(uint64_t));
     });
     if (rc) return rc;
     if (reset) {
