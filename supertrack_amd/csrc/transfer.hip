@@ -1,14 +1,22 @@
 // transfer.hip -- staged copies between host and device (transfer.hpp).
 //
-// hipMemcpy from ordinary memory stages or pins pages itself: 18 us for 8 B,
-// 45 us for 80 kB, 136 us for 1 MB and 30 GB/s for 590 MB, where the link
-// carries 57 GB/s.  Here the caller's data go through pinned buffers kept from
-// call to call, copied by up to kMaxWorkers threads while the copy engine
-// empties the buffers filled before (one thread's memcpy runs at 28 GB/s; a
-// copy costs the engine 14 us however small, hence the large buffers): 590 MB
-// 20.7 -> 12 ms.  Up to 512 KiB, four columns of a track say, one kernel reads
-// the buffer over the link and writes them all (the 7000-point tracks of a
-// loop: 69 us with hipMemcpy, 48 us with four queued copies, 25 us so).
+// hipMemcpy from ordinary memory stages or pins pages itself: 22 us for 8 B,
+// 28 us for 16 kB, 14 us for 80 kB, 67 us for 1 MB and 30 GB/s for 590 MB,
+// where the link carries 57 GB/s.  Here the caller's data go through pinned
+// buffers kept from call to call, where that is faster:
+//   * small uploads and several columns of up to 512 KiB in all (a track): one
+//     kernel reads the buffer over the link and writes them where they belong
+//     (8 B 15 us, 32 kB 16 us; tracks of 500, 7000, 16000 points 24, 30 and
+//     42 us, where four hipMemcpy take 64, 52 and 65 us);
+//   * large uploads: up to kMaxWorkers threads fill buffers while the copy
+//     engine empties those filled before (one thread's memcpy runs at 28 GB/s;
+//     a copy costs the engine 14 us however small, hence the large buffers):
+//     590 MB 20.7 -> 12 ms, four columns of 1.2 MB 315 -> 240 us;
+//   * small downloads (8 B 15 us, 32 kB 19 us against 22 and 24; 64 kB 20 us,
+//     where hipMemcpy takes 13 or 36).
+// In between hipMemcpy is the faster one: one column of 80 kB 14 us against 17
+// by the kernel, of 3 MB 147 against 192 by the buffers, of 8 MB 345 against
+// 475; four columns of 480 kB 150 against 175; 80 kB down 14 against 21.
 #include "transfer.hpp"
 
 #include <algorithm>
@@ -28,9 +36,11 @@ namespace st {
 namespace {
 
 constexpr int kMaxWorkers = 2;
-// Uploads from this size on use the large buffers, and one worker more for
-// each kPerWorker of them.
-constexpr size_t kLargeFrom = (size_t)2 << 20, kPerWorker = (size_t)8 << 20;
+// Where the lines above lie: bytes that the kernel takes of one column, that a
+// small download has at most, and from which uploads of one or two columns, or
+// of more, use the large buffers (one worker more for each kPerWorker).
+constexpr size_t kSmall = (size_t)64 << 10, kLargeFrom = (size_t)16 << 20, kLargeColumnsFrom = (size_t)4 << 20;
+constexpr size_t kPerWorker = (size_t)8 << 20;
 constexpr size_t kSlot[2] = {(size_t)512 << 10, (size_t)8 << 20};   // bytes of a buffer (small, large)
 constexpr size_t kKeep[2] = {16, kMaxWorkers};   // pairs of buffers kept for a device (16 + 32 MiB)
 
@@ -140,12 +150,6 @@ hipError_t plain_upload(const UploadPart *parts, int n)
     return hipSuccess;
 }
 
-// The parts cut into pieces of at most a buffer, small neighbours sharing one.
-struct Piece {
-    int part;
-    size_t at, bytes, slot_at;
-};
-
 // A buffer's parts to where they belong, blockIdx.y a part.
 constexpr int kGatherParts = 4;
 struct GatherArgs {
@@ -156,30 +160,56 @@ struct GatherArgs {
     } part[kGatherParts];
 };
 
+template <typename Word>
+__device__ __forceinline__ void copy_words(char *dst, const char *src, size_t bytes)
+{
+    const size_t i0 = (size_t)blockIdx.x * 256 + threadIdx.x, stride = (size_t)gridDim.x * 256;
+    const size_t words = bytes / sizeof(Word);
+    for (size_t i = i0; i < words; i += stride) ((Word *)dst)[i] = ((const Word *)src)[i];
+    for (size_t i = words * sizeof(Word) + i0; i < bytes; i += stride) dst[i] = src[i];
+}
+
 __global__ __launch_bounds__(256) void gather_kernel(GatherArgs a)
 {
     char *const dst = a.part[blockIdx.y].dst;
     const char *const src = a.part[blockIdx.y].src;
     const size_t bytes = a.part[blockIdx.y].bytes;
-    const size_t i0 = (size_t)blockIdx.x * 256 + threadIdx.x, stride = (size_t)gridDim.x * 256;
-    // (a caller's device address may have any alignment)
-    const size_t words = ((uintptr_t)dst & 15) == 0 ? bytes / 16 : 0;
-    for (size_t i = i0; i < words; i += stride) ((uint4 *)dst)[i] = ((const uint4 *)src)[i];
-    for (size_t i = words * 16 + i0; i < bytes; i += stride) dst[i] = src[i];
+    if (((uintptr_t)dst & 15) == 0) copy_words<uint4>(dst, src, bytes);
+    else copy_words<uint2>(dst, src, bytes);
 }
 
-hipError_t staged_upload(const UploadPart *parts, int n, size_t total)
+// Copies up to kGatherParts parts, which fit a small buffer together, with the
+// kernel.
+hipError_t gather_upload(Stage *s, const UploadPart *parts, int n)
 {
-    const int kind = total >= kLargeFrom ? 1 : 0;
+    GatherArgs a{};
+    size_t used = 0, most = 0;
+    int k = 0;
     for (int i = 0; i < n; ++i) {
         if (parts[i].bytes == 0) continue;
-        const HostRange range = host_range(parts[i].src, parts[i].bytes);
-        // (the copy engine reads pinned memory itself; host memory in the device's
-        // place is for hipMemcpy to refuse)
-        if (range == HostRange::other || (kind && range == HostRange::pinned) || !dev_known(parts[i].dst))
-            return plain_upload(parts, n);
+        std::memcpy(s->slot[0] + used, parts[i].src, parts[i].bytes);
+        a.part[k++] = {(char *)parts[i].dst, s->slot[0] + used, parts[i].bytes};
+        used += (parts[i].bytes + 255) / 256 * 256;
+        most = std::max(most, parts[i].bytes);
     }
-    const size_t cap = kSlot[kind];
+    const dim3 grid((unsigned)((most / 16 + 255) / 256 + 1), (unsigned)k);
+    hipError_t e = launch(gather_kernel, grid, 256, 0, nullptr, a);
+    if (e != hipSuccess) return e;
+    e = hipEventRecord(s->ev[0], nullptr);
+    const hipError_t waited = e == hipSuccess ? hipEventSynchronize(s->ev[0]) : hipStreamSynchronize(nullptr);
+    return e == hipSuccess ? waited : e;
+}
+
+// The parts cut into pieces of at most a buffer, small neighbours sharing one.
+struct Piece {
+    int part;
+    size_t at, bytes, slot_at;
+};
+
+// Copies the parts through large buffers, several threads filling them.
+hipError_t large_upload(const UploadPart *parts, int n, size_t total)
+{
+    const size_t cap = kSlot[1];
     std::vector<Piece> pieces;
     std::vector<size_t> fills;   // first piece of each buffer's fill
     size_t used = cap;
@@ -197,15 +227,11 @@ hipError_t staged_upload(const UploadPart *parts, int n, size_t total)
     const size_t n_fills = fills.size();
     fills.push_back(pieces.size());
 
-    // (the kernel's stores are checked by no one else)
-    bool gather = kind == 0 && n_fills == 1 && pieces.size() <= kGatherParts;
-    for (size_t i = 0; gather && i < pieces.size(); ++i)
-        gather = dev_writable(parts[pieces[i].part].dst, parts[pieces[i].part].bytes);
     std::vector<std::thread> pool;
     std::vector<Stage *> stages;
     pool.reserve(kMaxWorkers);
     stages.reserve(kMaxWorkers);
-    Stage *first = take(kind);
+    Stage *first = take(1);
     if (!first) return plain_upload(parts, n);
     stages.push_back(first);
     std::atomic<size_t> next{0};
@@ -222,20 +248,8 @@ hipError_t staged_upload(const UploadPart *parts, int n, size_t total)
             for (size_t i = fills[f]; e == hipSuccess && i < fills[f + 1]; ++i) {
                 const Piece &p = pieces[i];
                 std::memcpy(buf + p.slot_at, (const char *)parts[p.part].src + p.at, p.bytes);
-                if (gather) continue;
                 e = hipMemcpyAsync((char *)parts[p.part].dst + p.at, buf + p.slot_at, p.bytes, hipMemcpyHostToDevice,
                                    nullptr);
-            }
-            if (gather) {
-                GatherArgs a{};
-                size_t most = 0;
-                for (size_t i = 0; i < pieces.size(); ++i) {
-                    const Piece &p = pieces[i];
-                    a.part[i] = {(char *)parts[p.part].dst, buf + p.slot_at, p.bytes};
-                    most = std::max(most, p.bytes);
-                }
-                const dim3 grid((unsigned)((most / 16 + 255) / 256 + 1), (unsigned)pieces.size());
-                e = launch(gather_kernel, grid, 256, 0, nullptr, a);
             }
             const hipError_t noted = hipEventRecord(s->ev[k & 1], nullptr);
             if (e == hipSuccess) e = noted;
@@ -249,7 +263,7 @@ hipError_t staged_upload(const UploadPart *parts, int n, size_t total)
     const size_t helpers = std::min<size_t>({(size_t)std::min(kMaxWorkers, host_threads()) - 1, total / kPerWorker,
                                              n_fills - 1});
     for (size_t w = 0; w < helpers; ++w) {
-        Stage *s = take(kind);
+        Stage *s = take(1);
         if (!s) break;
         try {
             pool.emplace_back([&work, s] {
@@ -265,6 +279,38 @@ hipError_t staged_upload(const UploadPart *parts, int n, size_t total)
     for (std::thread &t : pool) t.join();
     for (Stage *s : stages) give(s);
     return (hipError_t)failed.load();
+}
+
+hipError_t staged_upload(const UploadPart *parts, int n, size_t total)
+{
+    int columns = 0;
+    size_t padded = 0;
+    bool aligned = true;
+    for (int i = 0; i < n; ++i) {
+        if (parts[i].bytes == 0) continue;
+        ++columns;
+        padded += (parts[i].bytes + 255) / 256 * 256;
+        aligned = aligned && ((uintptr_t)parts[i].dst & 7) == 0;
+    }
+    const bool gather = aligned && columns <= kGatherParts && padded <= kSlot[0] && (columns > 1 || total <= kSmall);
+    if (!gather && total < (columns > 2 ? kLargeColumnsFrom : kLargeFrom)) return plain_upload(parts, n);
+    for (int i = 0; i < n; ++i) {
+        if (parts[i].bytes == 0) continue;
+        const HostRange range = host_range(parts[i].src, parts[i].bytes);
+        // (the copy engine reads pinned memory itself; host memory in the device's
+        // place is for hipMemcpy to refuse; the kernel's stores are checked by no
+        // one else)
+        if (range == HostRange::other) return plain_upload(parts, n);
+        if (gather ? !dev_writable(parts[i].dst, parts[i].bytes)
+                   : range == HostRange::pinned || !dev_known(parts[i].dst))
+            return plain_upload(parts, n);
+    }
+    if (!gather) return large_upload(parts, n, total);
+    Stage *s = take(0);
+    if (!s) return plain_upload(parts, n);
+    const hipError_t e = gather_upload(s, parts, n);
+    give(s);
+    return e;
 }
 
 }  // namespace
@@ -290,7 +336,7 @@ hipError_t download(void *dst, const void *src, size_t bytes)
     if (bytes == 0) return hipSuccess;
     hipError_t e = dev_check(src, bytes);
     if (e != hipSuccess) return e;
-    Stage *s = bytes <= kSlot[0] && host_range(dst, bytes) != HostRange::other && dev_known(src) ? take(0) : nullptr;
+    Stage *s = bytes <= kSmall && host_range(dst, bytes) != HostRange::other && dev_known(src) ? take(0) : nullptr;
     if (!s) return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
     e = hipMemcpyAsync(s->slot[0], src, bytes, hipMemcpyDeviceToHost, nullptr);
     if (e == hipSuccess) e = hipEventRecord(s->ev[0], nullptr);
