@@ -194,6 +194,7 @@ struct st_library {
     std::vector<int32_t> wave_order, rest_order;
     int32_t *wave_order_dev = nullptr, *rest_order_dev = nullptr;
     int64_t wave_points = 0;           // points of the wave_order tracks
+    int64_t rest_points = 0;           // and of the rest_order tracks
     // work queues of the allocation-free pass (a batch keeps its own)
     PlanTrack *static_plan = nullptr;
     // streamed construction: begin sizes the device arrays, appends fill them
@@ -427,6 +428,22 @@ bool names_wave_shape(const st_batch_opts &o) { return o.table_slots == kWaveSlo
 bool names_block_shape(const st_batch_opts &o)
 {
     return !names_wave_shape(o) && (o.table_slots || o.blocks_per_cu || o.points_per_thread || o.hist_copies);
+}
+
+// Whether the one-wave kernel takes its tracks of a pass.  Where some tracks are
+// left to the block kernel (rest_order), that kernel still takes as long as the
+// largest of them, so the pass must hold enough work beside it: for each CU at
+// least 24 times that track's points.  (us a pass, all by the block kernel / by
+// both, 4 nm spheres: 192 tracks of 1e3 to 1e6 points, ST_F32 x 60, 8 times the
+// points, 1458 / 1619, x 250, 32 times, 3703 / 2745; 48 tracks of 2e4 to 5e5, 6
+// times 1069 / 1485, 20 times 1754 / 1895, 61 times 4105 / 3282; ST_F64, 20
+// times, 1957 / 1970.  Between 15 and 25 times either may be ahead by a tenth.)
+bool wave_pays(const st_library *L, const st_batch_opts &o)
+{
+    if (L->wave_order.empty() || o.n_oversamples == 0) return false;
+    if (L->rest_order.empty() || names_wave_shape(o)) return true;
+    const double points = (double)L->wave_points + (double)L->rest_points;
+    return points * o.n_oversamples >= 24.0 * device_cu_count() * L->tracks[L->rest_order.front()].n;
 }
 
 // Launch shape for (table slots, workgroups per CU, points per thread, LDS
@@ -911,13 +928,14 @@ int st_library_finish(st_library *L)
 
     L->wave_order.clear();
     L->rest_order.clear();
-    L->wave_points = 0;
+    L->wave_points = L->rest_points = 0;
     for (int32_t t : L->fast_order) {
         if (L->tracks[t].wave & kFlagWave) {
             L->wave_order.push_back(t);
             L->wave_points += L->tracks[t].n;
         } else {
             L->rest_order.push_back(t);
+            L->rest_points += L->tracks[t].n;
         }
     }
 
@@ -1039,7 +1057,9 @@ int st_batch_create(st_library *lib, const st_batch_opts *opts, st_hist *const *
     };
     rc = default_launch(lib->precision, b->hist_words, *opts, &b->ln);
     if (rc) return fail(rc);
-    const bool wave = !names_block_shape(*opts) && !lib->wave_order.empty() && opts->n_oversamples > 0;
+    // (autotune times both ways)
+    const bool wave = !names_block_shape(*opts) && (wave_pays(lib, *opts) || (opts->autotune && opts->n_oversamples > 0 &&
+                                                                              !lib->wave_order.empty()));
     if (wave) {
         rc = configure_wave(lib->precision, b->hist_words, names_wave_shape(*opts) ? opts->blocks_per_cu : 0, &b->wave);
         if (rc) return fail(rc);
@@ -1110,7 +1130,7 @@ int st_batch_run_static(st_library *lib, const st_batch_opts *opts, st_hist *con
     // the histograms of the one-wave kernel's workgroups are merged with
     // atomics here: their slab would have to be allocated
     WaveLaunch w;
-    const bool wave = !names_block_shape(*opts) && !lib->wave_order.empty();
+    const bool wave = !names_block_shape(*opts) && wave_pays(lib, *opts);
     if (wave) {
         rc = configure_wave(lib->precision, hist_words, names_wave_shape(*opts) ? opts->blocks_per_cu : 0, &w);
         if (!rc) rc = launch_plan(lib, opts->n_oversamples, w, lib->static_plan, stream);
