@@ -752,6 +752,9 @@ int read_report(st_batch *b, CtlReport *out)
     return ST_OK;
 }
 
+// Tracks and points up to which a run is laid out on the host.
+constexpr int64_t kHostTracks = 4, kHostPoints = 1024;
+
 // Appends a run of tracks (checked by the caller) to the library.
 int append_run(st_library *L, const double *x, const double *y, const double *z, const double *edep,
                const int64_t *offsets, int64_t n_tracks, const int32_t *geom_of_track)
@@ -772,10 +775,17 @@ int append_run(st_library *L, const double *x, const double *y, const double *z,
     const LayoutDst dst{L->x64 + pbase, L->y64 + pbase, L->z64 + pbase, L->e64 + pbase,
                         precision == ST_F32 ? reinterpret_cast<PointF32 *>(L->p32) + pbase : nullptr,
                         L->zfirst + bbase, precision == ST_F32 ? L->blocks + bbase : nullptr};
-    int rc = layout_chunk_device(x + offsets[0], y + offsets[0], z + offsets[0], edep + offsets[0], n_points, n_tracks,
+    // A few small tracks are laid out on the host: the device's layout is 30
+    // launches, whatever the size (st_library_create of one track, us, host /
+    // device: 300 points 128 / 165 in ST_F32, 87 / 178 in ST_F64, 1000 points 154 /
+    // 165, 98 / 181, 2000 points 201 / 180, 114 / 183; four of 300 points 186 / 184,
+    // 134 / 190; 16 of 50 points 334 / 188).
+    int rc = ST_ENOMEM;
+    if (n_tracks > kHostTracks || n_points > kHostPoints)
+        rc = layout_chunk_device(x + offsets[0], y + offsets[0], z + offsets[0], edep + offsets[0], n_points, n_tracks,
                                  L->geoms.data(), n_geoms, precision, pbase, bbase, nblocks, tds, dst);
     if (rc == ST_ENOMEM) {
-        // no room for the device's scratch beside the library: on the host
+        // (or no room for the device's scratch beside the library)
         clear_error();
         ChunkLayout lay;
         fill_chunk(x, y, z, edep, offsets, n_tracks, L->geoms.data(), precision, pbase, bbase, nblocks, tds, lay);
