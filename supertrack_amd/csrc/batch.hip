@@ -1199,6 +1199,7 @@ int st_batch_run(st_batch *b)
     int rc = prepare_passes(b);
     if (rc) return rc;
     ST_HIP_TRY(hipEventRecord(b->ev[0], b->stream));
+    for (st_hist *h : b->hists) h->bins_zero = false;   // (a replayed graph does not come by make_args)
     if (b->opts.use_graph && b->rec.cap == 0) {
         if (!b->graph_ready) {
             ST_HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
