@@ -3,9 +3,9 @@
 // Laying a library out is the larger part of a job on new tracks (18.5e6
 // points, 100 oversamples: 336 of 340 ms on the host: a stable sort per track,
 // two sliding windows, FP32 records).  Here the points go to the device as
-// they come and everything else is done there; the upload then bounds it: 21 ms,
-// 20 of them the copy at 29 GB/s (24 tracks, 119e3 points: 1.76 -> 0.43 ms, of
-// which 0.2 are the sort's launches).
+// they come and everything else is done there; the upload then bounds it: 14.2 ms
+// for the library, 12 of them the copy (24 tracks, 119e3 points: 1.76 -> 0.34 ms,
+// of which 0.2 are the sort's launches).
 //   * sort: a stable LSD radix sort of (z, index) over the whole run, 8 bits a
 //     pass, then by track number: tile histograms, one scan workgroup per
 //     digit, a ranking scatter (wave ballots), all without spinning;

@@ -8,15 +8,16 @@
 //     kernel reads the buffer over the link and writes them where they belong
 //     (8 B 15 us, 32 kB 16 us; tracks of 500, 7000, 16000 points 24, 30 and
 //     42 us, where four hipMemcpy take 64, 52 and 65 us);
-//   * large uploads: up to kMaxWorkers threads fill buffers while the copy
-//     engine empties those filled before (one thread's memcpy runs at 28 GB/s;
-//     a copy costs the engine 14 us however small, hence the large buffers):
-//     590 MB 20.7 -> 12 ms, four columns of 1.2 MB 315 -> 240 us;
+//   * several columns above that, and uploads from 16 MiB on: up to kMaxWorkers
+//     threads fill large buffers while the copy engine empties those filled
+//     before (one thread's memcpy runs at 28 GB/s; a copy costs the engine 14 us
+//     however small, hence the large buffers): 590 MB 20.7 -> 12 ms, four
+//     columns of 0.16, 0.48 and 1.2 MB 67, 106 and 230 us against 67, 132 and 330;
 //   * small downloads (8 B 15 us, 32 kB 19 us against 22 and 24; 64 kB 20 us,
 //     where hipMemcpy takes 13 or 36).
 // In between hipMemcpy is the faster one: one column of 80 kB 14 us against 17
 // by the kernel, of 3 MB 147 against 192 by the buffers, of 8 MB 345 against
-// 475; four columns of 480 kB 150 against 175; 80 kB down 14 against 21.
+// 475; 80 kB down 14 against 21.
 #include "transfer.hpp"
 
 #include <algorithm>
@@ -36,10 +37,10 @@ namespace st {
 namespace {
 
 constexpr int kMaxWorkers = 2;
-// Where the lines above lie: bytes that the kernel takes of one column, that a
-// small download has at most, and from which uploads of one or two columns, or
-// of more, use the large buffers (one worker more for each kPerWorker).
-constexpr size_t kSmall = (size_t)64 << 10, kLargeFrom = (size_t)16 << 20, kLargeColumnsFrom = (size_t)4 << 20;
+// Where the lines above lie: bytes that the kernel takes of one column and that a
+// small download has at most, and from which one column uses the large buffers
+// (one worker more for each kPerWorker).
+constexpr size_t kSmall = (size_t)64 << 10, kLargeFrom = (size_t)16 << 20;
 constexpr size_t kPerWorker = (size_t)8 << 20;
 constexpr size_t kSlot[2] = {(size_t)512 << 10, (size_t)8 << 20};   // bytes of a buffer (small, large)
 constexpr size_t kKeep[2] = {16, kMaxWorkers};   // pairs of buffers kept for a device (16 + 32 MiB)
@@ -293,7 +294,7 @@ hipError_t staged_upload(const UploadPart *parts, int n, size_t total)
         aligned = aligned && ((uintptr_t)parts[i].dst & 7) == 0;
     }
     const bool gather = aligned && columns <= kGatherParts && padded <= kSlot[0] && (columns > 1 || total <= kSmall);
-    if (!gather && total < (columns > 2 ? kLargeColumnsFrom : kLargeFrom)) return plain_upload(parts, n);
+    if (!gather && (columns > 1 ? total <= kSlot[0] : total < kLargeFrom)) return plain_upload(parts, n);
     for (int i = 0; i < n; ++i) {
         if (parts[i].bytes == 0) continue;
         const HostRange range = host_range(parts[i].src, parts[i].bytes);
