@@ -264,6 +264,9 @@ typedef struct st_batch st_batch;
 
 int st_batch_create(st_library *lib, const st_batch_opts *opts, st_hist *const *hists,
                     int32_t n_hists, st_batch **out);
+/* The stream of the following passes.  A pass under way on the old stream is
+ * waited for (the passes of a batch share its buffers); other work on either
+ * stream is not. */
 int st_batch_set_stream(st_batch *b, void *hip_stream);
 /* One pass: every track x every oversample; counts are added to the device
  * counters of each histogram (read them with st_hist_fetch). */

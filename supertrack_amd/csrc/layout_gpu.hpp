@@ -19,7 +19,8 @@ struct LayoutDst {
 // run's points in their own order, sorts each track by z (stable; NaN last)
 // and fills dst and the records' bounds and flags on the device.  Returns
 // ST_ENOMEM if its scratch (64 B per point) cannot be allocated; the caller
-// then lays the run out on the host.  Waits for the device.
+// then lays the run out on the host.  At most 2^23 blocks and tracks (a
+// workgroup for each).  Waits for the device.
 int layout_chunk_device(const double *x, const double *y, const double *z, const double *edep, int64_t n_points,
                         int64_t n_tracks, const st_geometry *geoms, int n_geoms, int precision, int64_t pbase,
                         int64_t bbase, int64_t nblocks, TrackDesc *tds, const LayoutDst &dst);

@@ -1,5 +1,6 @@
-// transfer.hpp -- copies between ordinary host memory and the device through
-// pinned staging buffers that are kept from call to call.
+// transfer.hpp -- copies between host memory and the device: through pinned
+// staging buffers that are kept from call to call where that is faster than
+// hipMemcpy, and refused where hipMemcpy refuses them.
 #pragma once
 
 #include <hip/hip_runtime.h>

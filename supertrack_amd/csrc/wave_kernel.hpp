@@ -11,7 +11,8 @@
 //     occupancy check of the table is a scalar compare, a flush runs on 64
 //     dense list entries per step, and segment set-up is done once per wave
 //     and segment instead of by every wave of a workgroup;
-//   * table keys are bit fields (x | y << bx | z << by), formed by two shifts;
+//   * table keys are bit fields (x | y << bx | z << by), formed by three
+//     shift-adds (the last may hold a copy number below them);
 //     the hash is a rank-1 lattice over the three indices (24-bit multiply-adds,
 //     constants of the R3 low-discrepancy sequence): neighbouring spheres land
 //     far apart, 2.5 probes for the longest lane of a row where a
