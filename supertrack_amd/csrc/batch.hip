@@ -375,24 +375,28 @@ int launch_fast(st_batch *b)
 
 // Launch shape of the one-wave kernel: the workgroup size (4 to 16 waves share
 // one privatised histogram) that keeps most waves resident on a CU; on a tie
-// the largest (fewest histograms to sum).  Histograms so wide that fewer than
-// six waves (ST_F64: five) fit beside them are counted in the device bins, by
-// all the waves that the registers allow.  Which is faster depends on how often
-// spheres share a bin (us a pass, ST_F32, 192 tracks x 60, private / device
-// bins: 31e3 bins, six waves: 10 nm spheres 918 / 663, 100 nm 1640 / 708, 2 nm
-// 1466 / 2863, 1 nm 779 / 1383; 34e3 bins, four waves: 1255 / 676, 2282 / 710,
-// 2038 / 2884, 1048 / 1409); with fewer waves the private bins also lose to the
-// block kernel (34e3 bins: 10 nm 1158, 100 nm 1842; ST_F64, 30e3 bins, four
-// waves: 1321 and 2361 against 1168 and 2109).  max_blocks: the caller's
-// limit on workgroups per CU (0: none).
-int configure_wave(int precision, int hist_words, int max_blocks, WaveLaunch *out)
+// the largest (fewest histograms to sum).  Histograms so wide that too few waves
+// fit beside them are counted in the device bins, by all the waves that the
+// registers allow: fewer than four waves, and, unless all spheres are small,
+// fewer than six (ST_F64: five).  The device bins cost by the sum, and small
+// spheres have more sums to a point (us a pass, ST_F32, 192 tracks x 60, private
+// / device bins at five waves: 2 nm spheres 1696 / 2874, 3 nm 1567 / 2430, 7 nm
+// 1177 / 1049, 10 nm 1071 / 680, 100 nm 1903 / 751; 5 nm spheres and tracks of up
+// to 2e4 points x 500 1590 / 2215, 10 nm 1323 / 1186).  From 10 nm on, five
+// private waves (ST_F64: four) also lose to the block kernel (100 nm 1878).
+// max_blocks: the caller's limit on workgroups per CU (0: none).
+constexpr double kSmallSphere = 5.0;   // nm
+int configure_wave(const st_library *L, int hist_words, int max_blocks, WaveLaunch *out)
 {
+    const int precision = L->precision;
+    bool small = true;
+    for (const st_geometry &g : L->geoms) small = small && g.diameter <= kSmallSphere;
     const void *k = wave_kernel_ptr(precision);
     const size_t per_wave = wave_lds(precision == ST_F64 ? 2 : 1, kWaveSlots);
     hipFuncAttributes attr;
     ST_HIP_TRY(hipFuncGetAttributes(&attr, k));
     const int simd_waves = precision == ST_F64 ? 4 : 6;
-    const int min_private = precision == ST_F64 ? 5 : 6;
+    const int min_private = small ? 4 : precision == ST_F64 ? 5 : 6;
     const size_t kCuLds = 160 * 1024;
     WaveLaunch best;
     for (int pass = 0; pass < 2 && !best.on; ++pass) {
@@ -1071,7 +1075,7 @@ int st_batch_create(st_library *lib, const st_batch_opts *opts, st_hist *const *
     const bool wave = !names_block_shape(*opts) && (wave_pays(lib, *opts) || (opts->autotune && opts->n_oversamples > 0 &&
                                                                               !lib->wave_order.empty()));
     if (wave) {
-        rc = configure_wave(lib->precision, b->hist_words, names_wave_shape(*opts) ? opts->blocks_per_cu : 0, &b->wave);
+        rc = configure_wave(lib, b->hist_words, names_wave_shape(*opts) ? opts->blocks_per_cu : 0, &b->wave);
         if (rc) return fail(rc);
     }
     Carve c;
@@ -1142,7 +1146,7 @@ int st_batch_run_static(st_library *lib, const st_batch_opts *opts, st_hist *con
     WaveLaunch w;
     const bool wave = !names_block_shape(*opts) && wave_pays(lib, *opts);
     if (wave) {
-        rc = configure_wave(lib->precision, hist_words, names_wave_shape(*opts) ? opts->blocks_per_cu : 0, &w);
+        rc = configure_wave(lib, hist_words, names_wave_shape(*opts) ? opts->blocks_per_cu : 0, &w);
         if (!rc) rc = launch_plan(lib, opts->n_oversamples, w, lib->static_plan, stream);
         if (rc) return rc;
     }
